@@ -204,20 +204,6 @@ constexpr int kCoherent = 1 | 16;
 // open: wait until every vector memory operation of the wave is done.
 constexpr int kWaitVmcnt0 = 0x0F70;
 
-// Inclusive prefix sum over the wave with DPP row shifts and row broadcasts.
-__device__ __forceinline__ int wave_scan_incl(int x)
-{
-    int s = x;
-    s += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);   // row_shr:1
-    s += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);   // row_shr:2
-    s += __builtin_amdgcn_update_dpp(0, x, 0x113, 0xf, 0xf, true);   // row_shr:3
-    s += __builtin_amdgcn_update_dpp(0, s, 0x114, 0xf, 0xe, true);   // row_shr:4, lanes 4-15
-    s += __builtin_amdgcn_update_dpp(0, s, 0x118, 0xf, 0xc, true);   // row_shr:8, lanes 8-15
-    s += __builtin_amdgcn_update_dpp(0, s, 0x142, 0xa, 0xf, true);   // row_bcast:15 -> rows 1, 3
-    s += __builtin_amdgcn_update_dpp(0, s, 0x143, 0xc, 0xf, true);   // row_bcast:31 -> rows 2, 3
-    return s;
-}
-
 // Rows of a tile that attend its column c, from the tile's 16 row masks
 // packed two per word (word k = rows 2k | 2k+1 << 16).
 __device__ __forceinline__ uint32_t column_rows(const uint32_t (&wd)[8], int c)

@@ -6,55 +6,39 @@
 // window_offsets = exclusive prefix of the set sizes (:39).  New output: the
 // 16 row masks of each tile (bit c of row r <=> edge (16w+r, 16b+c)).
 //
-// Design (no sort; an LDS bitmap with one bit per block column):
-//   * convert_light, the main pass: a persistent kernel (as many 256-thread
-//     workgroups as are resident at once) walks the windows of up to
-//     kLightEdges edges on graphs whose block columns fit one bitmap sized
-//     to the graph (up to 4.2 M nodes).  Every edge ORs its block column's
-//     bit into the bitmap; a bit set for the first time is a new tile, so
-//     the count pass needs no scan.  The fill pass marks non-empty bitmap
-//     words in a summary and counts the new tiles under each summary word,
-//     turns those into word bases (a tile's output rank is the base of its
-//     word plus the set bits below it), stages the row masks
-//     and block columns of up to kMaskTiles tiles in LDS and streams them
-//     out in coalesced stores.  Each workgroup keeps the loads of its next
-//     window in flight while it works on the current one, and its barriers
-//     order LDS only, so they do not wait for those loads;
-//   * count_waves: the count pass of graphs whose bitmap is small (W <=
-//     65,536 windows): one window per wave with a bitmap of its own, no
-//     workgroup barrier;
-//   * the windows with more edges (hubs), which the main pass lists: when
-//     counting, count_hubs takes each with a 512-thread workgroup (any
-//     order); when filling, rank_hubs orders them heaviest first and
-//     convert_hubs gives each a 1024-thread workgroup;
-//   * convert_hubs, per window: on graphs too wide for one bitmap it takes
-//     every window with 256 threads, the bitmap swept in column slices of
-//     kSliceCols block columns (only slices holding an edge of the window
-//     are visited).  Each thread owns a contiguous run of the window's edges
-//     and merges consecutive edges that hit the same LDS word before its
-//     atomic; windows with more than NT * kEPT edges re-read them from
-//     memory and OR their masks straight into the zeroed output;
-//   * the main passes clear bitmap words edge by edge after use, so no
-//     window touches all W / 32 words.
-// The per-window work is O(E) plus a few barriers; the output is
-// deterministic and does not depend on the order of columns in a row.
-// Counts become window_offsets through counts_to_offsets (two launches).
-#include <stdio.h>
-
-#include <mutex>
+// Design (no sort; LDS bitmaps with one bit per block column):
+//   * list_hubs, the first launch of either pass, lists the hub windows (more
+//     than kLightEdges edges);
+//   * convert_waves, the main launch: its first workgroups take a hub window
+//     each (hub_window: a bitmap sized to the graph, the edges read in chunks
+//     of kHubChunk), the others a window per wave, with no workgroup barrier:
+//     the edges stay in registers, the bitmap is kept in two levels (a bit
+//     per bitmap word, and the words in use side by side), a tile's output
+//     rank is the tiles before its word plus the set bits below its own, and
+//     row masks and block columns are put together in LDS and leave in
+//     coalesced stores;
+//   * convert_wide: graphs too wide for that (W > kLightMaxW) take a
+//     workgroup per window, the bitmap swept in column slices of kSliceCols
+//     block columns (only slices holding an edge of the window are visited).
+//     Each thread owns a contiguous run of the window's edges and merges
+//     consecutive edges that hit the same LDS word before its atomic; windows
+//     with more than NT * kEPT edges re-read them from memory and OR their
+//     masks straight into the zeroed output.
+// The per-window work is O(E); the output is deterministic and does not
+// depend on the order of columns in a row.  Counts become window_offsets
+// through counts_to_offsets (two launches).
+#include <algorithm>
 
 #include "f3s_common.hpp"
 #include "f3s_device.hpp"
 
 namespace f3s {
 
-constexpr int kConvThreads = 256;                 // persistent kernel; per-window fallback
-constexpr int kHubThreads = 1024;                 // hub windows of the fill pass
+constexpr int kConvThreads = 256;                 // every main launch's workgroup
 constexpr int kBitWords = 2048;                  // bitmap words per column slice
 constexpr int kSumWords = kBitWords / 32;         // summary: one bit per bitmap word
 constexpr int kSliceCols = kBitWords * 32;        // block columns per slice
 constexpr int kMaxSlices = 2048;                  // >= ceil(2^27 / kSliceCols)
-constexpr int kMaskTiles = 256;                   // tile masks staged in LDS at once
 constexpr int kEPT = 8;                           // edges per thread kept in registers
 constexpr int kHubBatch = 4;                      // edge loads in flight per thread, wide windows
 static_assert(kSumWords == kWave, "the summary is scanned by one wave");
@@ -112,8 +96,7 @@ __device__ __forceinline__ int row_of_edge(const int32_t* rp, int nrows, int32_t
     return r;
 }
 
-// One window by one workgroup of NT threads, any edge count (every window of
-// a graph too wide for the persistent kernel's bitmap).  Pass kind: COUNT
+// One window by one workgroup of NT threads, any edge count (convert_wide).  Pass kind: COUNT
 // writes counts[w]; FILL
 // writes block_col / tile_mask at window_offsets[w] and checks the count
 // against the offsets.
@@ -398,790 +381,630 @@ convert_one_window(ConvLds<FILL, NT>& L, int32_t w, const int32_t* __restrict__ 
     }
 }
 
-// The hub windows of the fill pass, heaviest first (hubs != NULL; listed by
-// the main pass, ordered by rank_hubs), or every window (hubs == NULL:
-// graphs too wide for convert_light's bitmap); a workgroup per window.
-template <bool FILL, int NT>
-__global__ void __launch_bounds__(NT)
-convert_hubs(const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ col_idx,
+// Every window of a graph too wide for convert_waves, a workgroup per window.
+template <bool FILL>
+__global__ void __launch_bounds__(kConvThreads)
+convert_wide(const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ col_idx,
              int32_t n, int64_t nnz, int32_t W, int32_t* __restrict__ counts,
              const int32_t* __restrict__ window_offsets, int32_t* __restrict__ block_col,
-             uint16_t* __restrict__ tile_mask, const int32_t* __restrict__ hubs,
-             const int32_t* __restrict__ num_hubs, int32_t* __restrict__ err)
+             uint16_t* __restrict__ tile_mask, int32_t* __restrict__ err)
 {
-    __shared__ ConvLds<FILL, NT> L;
-    // the main pass lists each window at most once (num_hubs <= W); the clamp
-    // keeps the list read inside its W + 1 entries whatever the count holds
-    const int32_t nh = hubs ? min(*num_hubs, W) : W;
-    for (int32_t i = blockIdx.x; i < nh; i += gridDim.x) {
-        const int32_t w = hubs ? hubs[i] : i;
-        if (w < 0 || w >= W) continue;   // uniform
-        convert_one_window<FILL, NT>(L, w, row_ptr, col_idx, n, nnz, W, counts, window_offsets,
-                                     block_col, tile_mask, err);
+    __shared__ ConvLds<FILL, kConvThreads> L;
+    for (int32_t w = blockIdx.x; w < W; w += gridDim.x)
+        convert_one_window<FILL, kConvThreads>(L, w, row_ptr, col_idx, n, nnz, W, counts,
+                                               window_offsets, block_col, tile_mask, err);
+}
+
+// ---------------------------------------------------------------------------
+// Hub windows (more than kLightEdges edges).  list_hubs, the first launch of
+// either pass, lists them per block of kListBlock windows: the heavy ones
+// (more than kHeavyEdges edges) from the front of the block's part of
+// `hubs`, the others from its back, and both counts in seg[block] -- no
+// counter to clear first.  It also clears the pass's error bits.  The first
+// workgroups of the main launch take one listed window each, heavy ones
+// first, so that the longest chains start first and the light windows fill
+// in behind them (hub workgroups dealt out between the light ones: 8 to 36 us
+// slower on 1 M nodes with 1,310 hubs).
+// ---------------------------------------------------------------------------
+constexpr int kLightEdges = 1024;
+constexpr int kHeavyEdges = 4096;
+constexpr int kListBlock = 1024;
+constexpr int kHubLaunch = 2048;   // hub workgroups of a launch at most (they loop over the list)
+constexpr int kLightMaxW = 262144; // windows of the widest graph convert_waves takes
+static_assert(kLightMaxW / kListBlock <= kConvThreads, "one thread per block of the list");
+
+// The window's edges as the main launch counts them too.
+__device__ __forceinline__ int32_t window_edges(int32_t first, int32_t end)
+{
+    return (int32_t)((uint32_t)end - (uint32_t)first);
+}
+
+__global__ void __launch_bounds__(kListBlock)
+list_hubs(const int32_t* __restrict__ row_ptr, int32_t n, int32_t W, int2* __restrict__ seg,
+          int32_t* __restrict__ hubs, int32_t* __restrict__ err)
+{
+    __shared__ int2 part[kListBlock / kWave];
+    const int t = threadIdx.x, lane = t & (kWave - 1), wid = t / kWave;
+    const int32_t w = blockIdx.x * kListBlock + t;
+    int32_t E = 0;
+    if (w < W) E = window_edges(row_ptr[(int64_t)w * 16], row_ptr[min((int64_t)w * 16 + 16, (int64_t)n)]);
+    const bool heavy = E > kHeavyEdges, other = E > kLightEdges && !heavy;
+    const uint64_t mh = __ballot(heavy), mo = __ballot(other);
+    if (lane == 0) part[wid] = make_int2(__popcll(mh), __popcll(mo));
+    __syncthreads();
+    int2 before = make_int2(0, 0), all = make_int2(0, 0);
+#pragma unroll
+    for (int i = 0; i < kListBlock / kWave; ++i) {
+        const int2 p = part[i];
+        if (i < wid) before = make_int2(before.x + p.x, before.y + p.y);
+        all = make_int2(all.x + p.x, all.y + p.y);
+    }
+    const uint64_t below = (1ull << lane) - 1ull;
+    int32_t* dst = hubs + (int64_t)blockIdx.x * kListBlock;
+    if (heavy) dst[before.x + __popcll(mh & below)] = w;
+    if (other) dst[kListBlock - 1 - (before.y + __popcll(mo & below))] = w;
+    if (t == 0) {
+        seg[blockIdx.x] = all;
+        if (blockIdx.x == 0) *err = 0;
     }
 }
 
-// ---------------------------------------------------------------------------
-// Persistent kernel for the windows with at most kLightEdges edges, on graphs
-// whose block columns fit one LDS bitmap (W <= 32 kLightMaxWords).
-//
-// Each workgroup walks windows w_i = blockIdx.x + i G (G = grid size) and
-// keeps its memory traffic one window ahead of its work: while it works on
-// w_i, the edges of w_{i+1} are in flight into a second register set, and
-// the row pointers (and, when filling, output offsets) of w_{i+3} into a
-// register; those of w_{i+2}, fetched one window earlier, go into a
-// three-slot LDS ring.  The bitmap (one bit per block column, sized to the
-// graph) stays clear between windows: each edge clears its own word after
-// use.  Per window:
-//   mark   every edge ORs its block column's bit into the bitmap; a bit set
-//          for the first time is a new tile (count; filling, it adds one to
-//          its summary word's tile count); the first setter of a word also
-//          marks the word in the summary (fill);
-//   base   (fill) wave 0 scans the summary words' tile counts and turns the
-//          summary into word bases: a tile's output rank is the base of its
-//          word plus the set bits below it;
-//   stage  (fill) every edge ORs its bit into its tile's staged row masks and
-//          records the tile's block column, kMaskTiles tiles per round; each
-//          thread then streams out (and re-zeroes) the tiles it owns, so
-//          block columns and masks leave in coalesced stores;
-//   clear  every edge clears its bitmap word.
-// The per-edge work is a handful of VALU operations and one or two LDS
-// atomics: the passes are bound by instruction issue, and the fill pass also
-// by the occupancy its LDS allows, so they keep no per-edge state beyond the
-// column (and, filling, the row) and stage no more than kMaskTiles tiles.
-// Windows with more edges are listed for the hub launches, so that one heavy
-// window never holds up the windows queued behind it in this workgroup.
-// ---------------------------------------------------------------------------
-constexpr int kLightEPT = 4;                      // edges per thread, light windows
-constexpr int kLightEdges = kConvThreads * kLightEPT;
-constexpr int kLightMaxWords = 8192;              // bitmap words: W <= 262,144 (n <= 4,194,304)
-constexpr int kHubCountThreads = 512;             // count_hubs workgroup
-
-// The hub windows (more than kLightEdges edges), listed by the main passes:
-// entry {window, first edge, edges, 0}, from the window description the
-// main pass has already validated.
-struct HubList {
-    int32_t* count;   // entries listed (atomic; zeroed before the main pass)
-    int4* hubs;       // [cap]
-    int32_t cap;      // entries `hubs` holds (each window is listed at most once)
-};
-
-// Lists window w (edges [e0, e0 + E)).  One thread lists a window: a listing
-// spread over a wave (a broadcast of the atomic's result) measured 40 %
-// slower in convert_light's fill pass, whose other waves wait for it at a
-// barrier.
-__device__ __forceinline__ void list_hub(const HubList& hl, int32_t w, int32_t e0, int32_t E)
+// Window of list entry i (heavy windows first), or -1 past the list's end.
+// Every thread of the workgroup calls it; `lds` needs kConvThreads / 64 + 1
+// int64.
+__device__ __forceinline__ int32_t hub_entry(int32_t i, int32_t W, const int2* __restrict__ seg,
+                                             const int32_t* __restrict__ hubs, int64_t* lds)
 {
-    const int32_t i = atomicAdd(hl.count, 1);
-    if (i < hl.cap) hl.hubs[i] = make_int4(w, e0, E, 0);
-}
-
-constexpr int kMetaInts = 20;                     // rp[0..16], out_base, expect, flags
-constexpr int kMetaSlots = 3;                     // windows w_i, w_{i+1}, w_{i+2}
-constexpr int kMiscInts = 8;                      // cnt[2], total[2], bad
-constexpr int kFlagLive = 1, kFlagRowsOk = 2, kFlagOutOk = 4;
-
-// Dynamic LDS layout of convert_light (bytes; 16-byte aligned sections).
-struct LightLayout {
-    int32_t words;   // bitmap words, ceil(W / 32)
-    int32_t sums;    // summary words, ceil(words / 32) (fill)
-    uint32_t off_base, off_sum, off_masks, off_tcol, off_meta, bytes;
-};
-
-__host__ __device__ inline uint32_t align16(uint32_t x) { return (x + 15u) & ~15u; }
-
-__host__ __device__ inline LightLayout light_layout(int32_t W, bool fill)
-{
-    LightLayout l;
-    l.words = (W + 31) / 32;
-    l.sums = (l.words + 31) / 32;
-    uint32_t o = align16(4u * (uint32_t)l.words);
-    l.off_base = o;
-    if (fill) o = align16(o + 2u * (uint32_t)l.words);
-    l.off_sum = o;
-    if (fill) o = align16(o + 8u * (uint32_t)l.sums);   // summary, then tiles per summary word
-    l.off_masks = o;
-    if (fill) o = align16(o + 4u * kMaskTiles * 8);
-    l.off_tcol = o;
-    if (fill) o = align16(o + 4u * kMaskTiles);
-    l.off_meta = o;
-    o = align16(o + 4u * (kMetaSlots * kMetaInts + kMiscInts));
-    l.bytes = o;
-    return l;
+    const int32_t nb = (W + kListBlock - 1) / kListBlock;
+    const int t = threadIdx.x;
+    int32_t* found = reinterpret_cast<int32_t*>(lds + kConvThreads / kWave);
+    const int2 s = t < nb ? seg[t] : make_int2(0, 0);
+    if (t == 0) *found = -1;
+    int64_t all;
+    const int64_t ex = block_exclusive_scan<kConvThreads>(
+        (int64_t)s.x | ((int64_t)s.y << 32), lds, all);   // barriers inside
+    const int32_t h = i - (int32_t)(ex & 0xffffffff);
+    const int32_t o = i - (int32_t)(all & 0xffffffff) - (int32_t)(ex >> 32);
+    if (h >= 0 && h < s.x) *found = t * kListBlock + h;
+    if (i >= (int32_t)(all & 0xffffffff) && o >= 0 && o < s.y)
+        *found = t * kListBlock + kListBlock - 1 - o;
+    __syncthreads();
+    const int32_t at = *found;
+    __syncthreads();
+    return at < 0 ? -1 : hubs[at];
 }
 
 extern __shared__ __align__(16) unsigned char conv_lds[];
 
-struct LightLds {
-    uint32_t* bits;     // [words] block columns of the window
-    uint16_t* base;     // [words] tiles before each word (fill)
-    uint32_t* summary;  // [sums] non-empty bitmap words (fill)
-    int32_t* scnt;      // [sums] tiles under each summary word (fill)
-    uint32_t* masks;    // [kMaskTiles * 8] staged row masks, two rows per word (fill)
-    int32_t* tcol;      // [kMaskTiles] staged block columns (fill)
-    int32_t* meta;      // [kMetaSlots][kMetaInts] window descriptions (ring)
-    int32_t* cnt;       // [2] count: tiles of a window, by parity
-    int32_t* total;     // [2] fill: tiles of a window, by parity
-    int32_t* bad;       // a column outside [0, n) was seen
-    int32_t words, sums;
+__host__ __device__ inline uint32_t align16(uint32_t x) { return (x + 15u) & ~15u; }
+
+// Hub window w by a workgroup of kConvThreads.  Every edge ORs its block
+// column's bit into an LDS bitmap sized to the graph; edges are read in
+// coalesced chunks of kHubChunk, all loads of a chunk in flight at once.
+// Counting, the bits set for the first time are the tiles.  Filling, each
+// thread scans a run of bitmap words, and a tile's rank is `chunk` (tiles
+// before its run) plus `base` (in the run, before its word) plus the bits
+// below its own.  A window of one chunk keeps its edges in registers and
+// stages its tiles in LDS, over the bitmap, once their ranks are known; a
+// heavier one ORs its edges' bits into its zeroed output.
+constexpr int kHubEPT = 16;
+constexpr int kHubChunk = kConvThreads * kHubEPT;
+static_assert(kHubChunk == kHeavyEdges, "heavy windows are those of more than one chunk");
+
+struct HubHead {
+    int64_t scan[kConvThreads / kWave + 1];
+    int32_t rp[17];
+    uint32_t chunk[kConvThreads];
 };
 
-__device__ __forceinline__ LightLds light_lds(const LightLayout& lay)
+// log2 of the bitmap words per thread
+__host__ __device__ inline int hub_shift(int32_t W)
 {
-    LightLds L;
-    L.bits = reinterpret_cast<uint32_t*>(conv_lds);
-    L.base = reinterpret_cast<uint16_t*>(conv_lds + lay.off_base);
-    L.summary = reinterpret_cast<uint32_t*>(conv_lds + lay.off_sum);
-    L.scnt = reinterpret_cast<int32_t*>(L.summary + lay.sums);
-    L.masks = reinterpret_cast<uint32_t*>(conv_lds + lay.off_masks);
-    L.tcol = reinterpret_cast<int32_t*>(conv_lds + lay.off_tcol);
-    L.meta = reinterpret_cast<int32_t*>(conv_lds + lay.off_meta);
-    L.cnt = L.meta + kMetaSlots * kMetaInts;
-    L.total = L.cnt + 2;
-    L.bad = L.cnt + 4;
-    L.words = lay.words;
-    L.sums = lay.sums;
-    return L;
+    int s = 0;
+    while (((W + 31) / 32) > (kConvThreads << s)) ++s;
+    return s;
+}
+// bytes at least: the bitmap (a multiple of 16 bytes) and, filling, a u16 per word
+__host__ __device__ inline uint32_t hub_bits_bytes(int32_t W) { return (uint32_t)((W + 127) / 128 * 16); }
+__host__ __device__ inline uint32_t hub_work_bytes(int32_t W, bool fill)
+{
+    const uint32_t b = hub_bits_bytes(W);
+    return align16(fill ? b + b / 2 : b);
 }
 
-// What lane t (< 19) fetches for window wn: row_ptr[16 wn + t] for t <=
-// nrows, window_offsets[wn] (t = 17) and [wn + 1] (t = 18) when filling.
-// One vector load with a per-lane address (a uniform window_offsets load
-// would become a scalar load into the same register, and that register
-// write would have to wait for every load in flight).
-template <bool FILL>
-__device__ __forceinline__ int32_t fetch_meta(int32_t wn, int32_t W, int32_t n,
-                                              const int32_t* __restrict__ row_ptr,
-                                              const int32_t* __restrict__ window_offsets)
+// Staged row masks to the output, coalesced.  `stream` (the output may be
+// larger than the Infinity Cache, kStreamTiles, so nobody finds it there
+// afterwards): non-temporal stores, which leave the L2 to the edges and to the
+// lines the heavy hubs' atomics work on (the fill of 17 M edges with hubs
+// 174 -> 130 us; 122 M edges without hubs 512 -> 517 us).
+constexpr int64_t kStreamTiles = ((int64_t)256 << 20) / 32;
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void store_masks(uint4* __restrict__ dst, const uint4* src, int count,
+                                            int first, int step, bool stream)
 {
-    const int t = threadIdx.x & (kWave - 1);
-    const int32_t* p = nullptr;
-    if (wn < W) {
-        const int nrows = min(16, n - wn * 16);
-        if (t <= nrows) p = row_ptr + (int64_t)wn * 16 + t;
-        if (FILL && (t == 17 || t == 18)) p = window_offsets + wn + (t - 17);
-    }
-    int32_t v = 0;
-    if (p) v = *p;
-    return v;
-}
-
-// Wave 0 stores a fetched window description into ring slot `slot`, with
-// flags: live (wn < W), row pointers usable (0 <= rp[0] <= ... <= rp[nrows]
-// <= nnz) and output range usable ([out_base, out_base + expect) inside
-// [0, total_tiles)).
-template <bool FILL>
-__device__ __forceinline__ void publish_meta(const LightLds& L, int slot, int32_t v, int32_t wn,
-                                             int32_t W, int32_t n, int64_t nnz,
-                                             int32_t total_tiles, int32_t* __restrict__ err)
-{
-    const int lane = threadIdx.x;   // wave 0 only
-    const bool live = wn < W;
-    const int nrows = live ? min(16, n - wn * 16) : 0;
-    const int32_t rp0 = __shfl(v, 0, kWave), rpn = __shfl(v, nrows, kWave);
-    const int32_t nxt = __shfl_down(v, 1, kWave);
-    const bool back = lane < nrows && nxt < v;
-    const bool rows_ok = live && !__any(back) && rp0 >= 0 && rpn >= rp0 && (int64_t)rpn <= nnz;
-    bool out_ok = true;
-    int32_t val = v;
-    if (FILL) {
-        // lanes 17 and 18 hold window_offsets[wn] and [wn + 1]
-        const int32_t ob = __shfl(v, 17, kWave), end = __shfl(v, 18, kWave);
-        out_ok = ob >= 0 && end >= ob && end <= total_tiles;
-        if (lane == 18) val = out_ok ? end - ob : 0;   // expect
-    }
-    int32_t* dst = L.meta + slot * kMetaInts;
-    if (lane < 19) dst[lane] = val;
-    if (lane == 19)
-        dst[19] = (live ? kFlagLive : 0) | (rows_ok ? kFlagRowsOk : 0) |
-                  (out_ok ? kFlagOutOk : 0) | (nrows << 8);
-    if (lane == 0 && live) {
-        if (!rows_ok) atomicOr(err, kErrRowPtr);
-        else if (!out_ok) atomicOr(err, kErrCount);
+    if (stream) {
+        for (int k = first; k < count; k += step)
+            __builtin_nontemporal_store(__builtin_bit_cast(u32x4, src[k]),
+                                        reinterpret_cast<u32x4*>(dst) + k);
+    } else {
+        for (int k = first; k < count; k += step) dst[k] = src[k];
     }
 }
 
-struct LightWin {
-    int32_t e0, E, nrows, out_base, expect, flags;
-};
-
-__device__ __forceinline__ LightWin read_meta(const LightLds& L, int slot)
-{
-    const int32_t* m0 = L.meta + slot * kMetaInts;
-    LightWin m;
-    m.flags = m0[19];
-    m.nrows = m.flags >> 8;
-    m.e0 = m0[0];
-    m.E = (m.flags & kFlagRowsOk) ? m0[m.nrows] - m.e0 : 0;
-    m.out_base = m0[17];
-    m.expect = m0[18];
-    return m;
-}
-
-// Issues the loads of this thread's run of edges of the window in ring slot
-// `slot` (nothing for hub windows): col[j] for j < cnt, and (filling) the
-// rows, packed 4 bits per edge.  The loaded values are not used here, so the
-// loads stay in flight.
 template <bool FILL>
-__device__ __forceinline__ void issue_edges(const LightLds& L, int slot,
-                                            const int32_t* __restrict__ col_idx,
-                                            int32_t (&col)[kLightEPT], uint32_t& rows, int& cnt)
+__device__ __forceinline__ void
+hub_window(int32_t w, const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ col_idx,
+           int32_t n, int64_t nnz, int32_t W, int32_t* __restrict__ counts,
+           const int32_t* __restrict__ window_offsets, int32_t* __restrict__ block_col,
+           uint16_t* __restrict__ tile_mask, bool stream, HubHead& head, unsigned char* work,
+           uint32_t work_bytes, int32_t* __restrict__ err)
 {
-    const LightWin m = read_meta(L, slot);
-    cnt = 0;
-    rows = 0;
-    if (m.E <= 0 || m.E > kLightEdges) return;
-    const int per = (m.E + kConvThreads - 1) / kConvThreads;
-    const int i0 = min(m.E, (int)threadIdx.x * per), i1 = min(m.E, i0 + per);
-    cnt = i1 - i0;
-#pragma unroll
-    for (int j = 0; j < kLightEPT; ++j)
-        if (j < cnt) col[j] = col_idx[m.e0 + i0 + j];
-    if (FILL && cnt > 0) {
-        const int32_t* rp = L.meta + slot * kMetaInts;
-        int r = row_of_edge(rp, m.nrows, m.e0 + i0);
-#pragma unroll
-        for (int j = 0; j < kLightEPT; ++j) {
-            const int32_t e = m.e0 + i0 + j;
-            while (r + 1 < m.nrows && e >= rp[r + 1]) ++r;
-            rows |= (uint32_t)r << (4 * j);
+    constexpr int NT = kConvThreads;
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));   // nothing derived from it is kept across windows
+    const int words = (W + 31) / 32;
+    uint32_t* bits = reinterpret_cast<uint32_t*>(work);
+    uint16_t* base = reinterpret_cast<uint16_t*>(work + hub_bits_bytes(W));
+    for (uint32_t g = tid; g < hub_bits_bytes(W) / 16; g += NT)
+        reinterpret_cast<uint4*>(bits)[g] = make_uint4(0u, 0u, 0u, 0u);
+    const WindowRows wr = load_window_rows(row_ptr, n, nnz, w, head.rp, err);   // a barrier inside
+    if (wr.E < 0 || wr.e0 < 0 || wr.e0 + wr.E > nnz) {   // uniform
+        if (tid == 0) {
+            atomicOr(err, kErrRowPtr);
+            if (!FILL) counts[w] = 0;
         }
-    }
-}
-
-// One window (at most kLightEdges edges, in col / rows) described by ring
-// slot `slot`.  Every thread runs the same sequence of barriers.  Nothing
-// here waits for a load: the only loads in flight are the next window's.
-template <bool FILL>
-__device__ __forceinline__ void light_window(const LightLds& L, int slot, int32_t w,
-                                             int32_t (&col)[kLightEPT], uint32_t rows, int cnt,
-                                             int& round, int32_t n,
-                                             int32_t* __restrict__ counts,
-                                             int32_t* __restrict__ block_col,
-                                             uint16_t* __restrict__ tile_mask,
-                                             const HubList& hl,
-                                             int32_t* __restrict__ err)
-{
-    const int tid = threadIdx.x;
-    const int lane = tid & (kWave - 1);
-    const int wid = tid / kWave;
-    const LightWin m = read_meta(L, slot);
-    const bool usable = (m.flags & kFlagLive) && (m.flags & kFlagRowsOk) &&
-                        (!FILL || (m.flags & kFlagOutOk));
-
-    if (!usable || m.E > kLightEdges || m.E == 0) {
-        // hub (listed for count_hubs / convert_hubs, which also write its
-        // count or tiles), empty or rejected window: no tiles here
-        if (usable && m.E > 0) {
-            if (tid == 0) list_hub(hl, w, m.e0, m.E);
-        } else if (tid == 0) {
-            if (FILL) {
-                if (usable && m.expect != 0) atomicOr(err, kErrCount);
-            } else {
-                counts[w] = 0;
-            }
-        }
-        lds_barrier();   // the description published for window w + 2G is visible
         return;
     }
-
-    // absent (j >= cnt) and invalid columns become -1; an invalid column
-    // (outside [0, n)) is reported and left out
-#pragma unroll
-    for (int j = 0; j < kLightEPT; ++j) {
-        const int32_t c = col[j];
-        const bool present = j < cnt;
-        const bool ok = present && c >= 0 && c < n;
-        if (present && !ok) *L.bad = 1;
-        col[j] = ok ? c : -1;
-    }
-    const int k = round & 1;
-    ++round;
+    const uint32_t E = (uint32_t)wr.E;
+    const int32_t* cols = col_idx + wr.e0;
 
     // ---- mark ----
+    int32_t col[kHubEPT];
     int32_t fresh = 0;
+    bool bad = false;
+    for (uint32_t c0 = 0; c0 < E; c0 += kHubChunk) {
 #pragma unroll
-    for (int j = 0; j < kLightEPT; ++j) {
-        const int32_t c = col[j];
-        if (c < 0) continue;
-        const int32_t wi = c >> 9;
-        const uint32_t bit = 1u << ((c >> 4) & 31);
-        const uint32_t old = atomicOr(&L.bits[wi], bit);
-        if (FILL) {
-            if (old == 0u) atomicOr(&L.summary[wi >> 5], 1u << (wi & 31));
-            if ((old & bit) == 0u) atomicAdd(&L.scnt[wi >> 5], 1);   // a new tile
-        } else {
-            fresh += (old & bit) == 0u;
+        for (int j = 0; j < kHubEPT; ++j) {
+            const uint32_t e = c0 + tid + NT * j;
+            col[j] = e < E ? cols[e] : 0;
+        }
+#pragma unroll
+        for (int j = 0; j < kHubEPT; ++j) {
+            const bool in = c0 + tid + NT * j < E;
+            const int32_t c = col[j];
+            const bool ok = in && (uint32_t)c < (uint32_t)n;
+            bad |= in && !ok;
+            col[j] = ok ? c : -1;
+            if (ok) {
+                const uint32_t bit = 1u << ((c >> 4) & 31);
+                if constexpr (FILL)
+                    atomicOr(&bits[c >> 9], bit);
+                else
+                    fresh += (atomicOr(&bits[c >> 9], bit) & bit) == 0u;
+            }
         }
     }
-    if (!FILL) {
-        fresh = wave_sum(fresh);
-        if (lane == 0 && fresh) atomicAdd(&L.cnt[k], fresh);
-    }
-    lds_barrier();   // B1: bitmap (+ summary) complete
-    if (tid == 0) L.cnt[k ^ 1] = 0;   // read before B1 by the previous window
-
-    int32_t total;
+    if (__any(bad) && (tid & (kWave - 1)) == 0) atomicOr(err, kErrCol);
     if constexpr (!FILL) {
-        total = L.cnt[k];
+        int64_t T;
+        (void)block_exclusive_scan<NT>((int64_t)fresh, head.scan, T);   // barriers inside
+        if (tid == 0) counts[w] = (int32_t)T;
+        return;
     } else {
-        // ---- base (wave 0): lane l owns summary words [l spl, (l + 1) spl) ----
-        if (wid == 0) {
-            const int spl = (L.sums + kWave - 1) / kWave;
-            const int s0 = min(L.sums, lane * spl), s1 = min(L.sums, s0 + spl);
-            // the tiles under each summary word were counted while marking
-            int32_t own = 0;
-            for (int sw = s0; sw < s1; ++sw) own += L.scnt[sw];
-            const int32_t incl = wave_inclusive_scan(own);
-            int32_t t0 = incl - own;
-            for (int sw = s0; sw < s1; ++sw) {
-                uint32_t t = L.summary[sw];
-                if (!t) continue;
-                L.summary[sw] = 0u;
-                L.scnt[sw] = 0;
-                for (; t; t &= t - 1u) {
-                    const int wi = sw * 32 + __builtin_ctz(t);
-                    L.base[wi] = (uint16_t)t0;
-                    t0 += __popc(L.bits[wi]);
-                }
-            }
-            if (lane == kWave - 1) L.total[k] = incl;
+        const int32_t out_base = window_offsets[w];
+        const int32_t expect = window_offsets[w + 1] - out_base;
+        // ---- scan ----
+        __syncthreads();   // every mark is done
+        const int sh = hub_shift(W);
+        const int a0 = min(words, tid << sh), a1 = min(words, (tid + 1) << sh);
+        int32_t own = 0;
+        for (int a = a0; a < a1; ++a) {
+            base[a] = (uint16_t)own;
+            own += __popc(bits[a]);
         }
-        lds_barrier();   // B2: bases and the window's tile count
-        total = L.total[k];
-        if (total <= m.expect) {
-            // ---- stage, kMaskTiles tiles per round ----
-            for (int32_t ms = 0; ms < total; ms += kMaskTiles) {
-                if (ms > 0) lds_barrier();   // the previous round's tiles are re-zeroed
+        int64_t all;
+        const int64_t before = block_exclusive_scan<NT>((int64_t)own, head.scan, all);
+        head.chunk[tid] = (uint32_t)before;
+        __syncthreads();
+        const int32_t total = (int32_t)all;
+        // the caller's offsets have to describe this CSR, and stay inside
+        // [0, window_offsets[W]], the size of block_col / tile_mask
+        const bool fits = out_base >= 0 && expect >= 0 &&
+                          out_base <= window_offsets[W] - expect && total <= expect;
+        if ((!fits || total != expect) && tid == 0) atomicOr(err, kErrCount);
+        if (!fits) return;   // uniform
+        auto rank = [&](int32_t c) __attribute__((always_inline)) -> uint32_t {
+            const int32_t wi = c >> 9;
+            return head.chunk[wi >> sh] + base[wi] +
+                   __popc(bits[wi] & ((1u << ((c >> 4) & 31)) - 1u));
+        };
+        auto load_chunk = [&](uint32_t c0) __attribute__((always_inline)) {
 #pragma unroll
-                for (int j = 0; j < kLightEPT; ++j) {
-                    const int32_t c = col[j];
-                    if (c < 0) continue;
-                    const int32_t wi = c >> 9;
-                    const uint32_t below = (1u << ((c >> 4) & 31)) - 1u;
-                    const int32_t t2 = (int32_t)L.base[wi] + __popc(L.bits[wi] & below) - ms;
-                    if (t2 < 0 || t2 >= kMaskTiles) continue;
-                    const int r = (int)((rows >> (4 * j)) & 15u);
-                    atomicOr(&L.masks[t2 * 8 + (r >> 1)], (1u << (c & 15)) << (16 * (r & 1)));
-                    L.tcol[t2] = c >> 4;   // every edge of the tile writes the same value
-                }
-                lds_barrier();   // B3: the round's staged tiles are complete
-                const int32_t nt = min(kMaskTiles, total - ms);
-                for (int t3 = tid; t3 < nt; t3 += kConvThreads) {
-                    const int64_t o = (int64_t)m.out_base + ms + t3;
-                    block_col[o] = L.tcol[t3];
-                    uint4* src = reinterpret_cast<uint4*>(&L.masks[t3 * 8]);
-                    if (tile_mask) {
-                        uint4* dst = reinterpret_cast<uint4*>(tile_mask + o * 16);
-                        dst[0] = src[0];
-                        dst[1] = src[1];
-                    }
-                    src[0] = make_uint4(0u, 0u, 0u, 0u);
-                    src[1] = make_uint4(0u, 0u, 0u, 0u);
-                }
+            for (int j = 0; j < kHubEPT; ++j) {
+                const uint32_t e = c0 + tid + NT * j;
+                col[j] = e < E ? cols[e] : -1;
             }
-        }
-    }
-    // ---- clear (every reader of the bitmap is past B1, B2 or B3) ----
+        };
+        auto row_at = [&](uint32_t c0, int j) __attribute__((always_inline)) -> int {
+            return row_of_edge(head.rp, wr.nrows, (int32_t)((uint32_t)wr.e0 + c0 + tid + NT * j));
+        };
+        auto put = [&](uint32_t t, int r, int32_t c, uint32_t* masks, int32_t* tcol)
+                       __attribute__((always_inline)) {
+            atomicOr(&masks[t * 8 + (r >> 1)], 1u << ((c & 15) + 16 * (r & 1)));
+            tcol[t] = c >> 4;   // every edge of the tile writes the same
+        };
+        // The window's tiles, st at a time: put together at `at`, then stored.
+        auto stage_tiles = [&](int32_t tiles, int32_t out, unsigned char* at, int32_t st,
+                               auto&& fill) __attribute__((always_inline)) {
+            uint32_t* masks = reinterpret_cast<uint32_t*>(at);
+            int32_t* tcol = reinterpret_cast<int32_t*>(masks + 8 * st);
+            for (int32_t ms = 0; ms < tiles; ms += st) {
+                const int32_t nt = min(st, tiles - ms);
+                __syncthreads();   // ranks taken, or the last round's tiles read
+                for (int k = tid; k < 2 * nt; k += NT)
+                    reinterpret_cast<uint4*>(masks)[k] = make_uint4(0u, 0u, 0u, 0u);
+                __syncthreads();
+                fill((uint32_t)ms, (uint32_t)nt, masks, tcol);
+                __syncthreads();
+                const int64_t o = (int64_t)out + ms;
+                for (int k = tid; k < nt; k += NT) block_col[o + k] = tcol[k];
+                if (tile_mask)
+                    store_masks(reinterpret_cast<uint4*>(tile_mask + o * 16),
+                                reinterpret_cast<const uint4*>(masks), 2 * nt, tid, NT, stream);
+            }
+        };
+        const uint32_t both = align16(hub_bits_bytes(W) * 3 / 2);
+        const int32_t beside = (int32_t)((work_bytes - both) / 36) & ~3;   // tiles
+        if (E <= kHubChunk) {
+            uint32_t aux[kHubEPT];   // rank, row << 16
 #pragma unroll
-    for (int j = 0; j < kLightEPT; ++j)
-        if (col[j] >= 0) L.bits[col[j] >> 9] = 0u;
-    lds_barrier();   // B4: bitmap and staged masks clear for the next window
-    if (tid == 0) {
-        if (FILL) {
-            if (total != m.expect) atomicOr(err, kErrCount);
+            for (int j = 0; j < kHubEPT; ++j) {
+                asm volatile("" : "+v"(col[j]));   // recompute, do not keep from the marking
+                aux[j] = 0xffffu;
+                if (col[j] >= 0)
+                    aux[j] = rank(col[j]) | ((uint32_t)row_at(0u, j) << 16);
+            }
+            stage_tiles(total, out_base, work, (int32_t)(work_bytes / 36) & ~3,
+                        [&](uint32_t ms, uint32_t nt, uint32_t* masks, int32_t* tcol)
+                            __attribute__((always_inline)) {
+#pragma unroll
+                            for (int j = 0; j < kHubEPT; ++j) {
+                                asm volatile("" : "+v"(col[j]), "+v"(aux[j]));
+                                const uint32_t t = (aux[j] & 0xffffu) - ms;
+                                if (t < nt) put(t, (int)(aux[j] >> 16), col[j], masks, tcol);
+                            }
+                        });
+        } else if (total <= 4 * beside) {
+            // few tiles for its edges: a stage beside the bitmap, the edges
+            // read again for each of at most four rounds
+            stage_tiles(total, out_base, work + both, beside,
+                        [&](uint32_t ms, uint32_t nt, uint32_t* masks, int32_t* tcol)
+                            __attribute__((always_inline)) {
+                            for (uint32_t c0 = 0; c0 < E; c0 += kHubChunk) {
+                                load_chunk(c0);
+#pragma unroll
+                                for (int j = 0; j < kHubEPT; ++j) {
+                                    if ((uint32_t)col[j] >= (uint32_t)n) continue;
+                                    const uint32_t t = rank(col[j]) - ms;
+                                    if (t < nt) put(t, row_at(c0, j), col[j], masks, tcol);
+                                }
+                            }
+                        });
         } else {
-            counts[w] = total;
+            uint32_t* gm = reinterpret_cast<uint32_t*>(tile_mask + (int64_t)out_base * 16);
+            if (tile_mask) {
+                for (int64_t k = tid; k < 2 * (int64_t)total; k += NT)
+                    reinterpret_cast<uint4*>(gm)[k] = make_uint4(0u, 0u, 0u, 0u);
+                // the zeros reach the L2, where the atomics act, before any OR
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                __syncthreads();
+            }
+            for (uint32_t c0 = 0; c0 < E; c0 += kHubChunk) {
+                load_chunk(c0);
+#pragma unroll
+                for (int j = 0; j < kHubEPT; ++j) {
+                    const int32_t c = col[j];
+                    if ((uint32_t)c >= (uint32_t)n) continue;
+                    const uint32_t t = rank(c);
+                    block_col[(int64_t)out_base + t] = c >> 4;   // every edge of the tile: the same
+                    if (tile_mask) {
+                        const int r = row_at(c0, j);
+                        atomicOr(&gm[(int64_t)t * 8 + (r >> 1)], 1u << ((c & 15) + 16 * (r & 1)));
+                    }
+                }
+            }
         }
+        __syncthreads();   // the next window's bitmap goes over this one's
     }
+}
+
+// ---------------------------------------------------------------------------
+// convert_waves, the main pass of graphs of up to kLightMaxW windows: after
+// the hub workgroups (above), one window of up to kLightEdges edges per wave,
+// no workgroup barrier, the edges in registers (lane + 64 j).  A window's
+// block columns are a sparse set, so its bitmap is kept in two levels: `sp`
+// has one bit per bitmap word of the graph (32 block columns) and the words
+// that hold an edge sit side by side in `bits`.  Per window:
+//   mark   every edge ORs its word's bit into sp (a run of edges in one word
+//          once); a scan over sp gives each word's place;
+//   words  every edge ORs its block column's bit into its word;
+//          counting, the set bits are the tiles;
+//   ranks  (fill) a scan over the words gives the tiles before each, and an
+//          edge's tile is that plus the set bits below its own;
+//   stage  (fill) kStageTiles tiles at a time, row masks and block columns
+//          are put together in LDS, over the words, and leave in coalesced
+//          stores.
+// What bounds it (MI355X): on sparse windows the stores, on full ones the
+// VALU and LDS instructions (about 65 and 12 per 64 edges when filling).  The
+// fill's launch takes 130 us for 1 M nodes and 17 M edges on random ids (hub
+// windows included; 0.68 GB, 5.2 TB/s) and 515 us for 2.4 M nodes in
+// communities with 122 M edges (2.7 GB, 5.2 TB/s); the former pass of one
+// window per 256-thread workgroup, whose barriers and wave 0's walk over the
+// summary set the pace, took 207 + 106 us (hubs in launches of their own) and
+// 1,000 us.  Counting takes 35 us (39 + 13) and 217 us (209).
+// Several windows per wave, the next one's edges in flight, measured slower
+// the more there were (both calls of the second graph: 745 us with one, 806
+// with two, 945 with sixteen): a prefetch's wait is also a wait for the
+// stores of the window before.
+// ---------------------------------------------------------------------------
+constexpr int kWaveSlots = kLightEdges / kWave;   // edge slots per lane
+constexpr int kWaveGroup = 2;                     // slots per uniform branch
+constexpr int kWavesPerWg = kConvThreads / kWave;
+constexpr int kStageTiles = 160;                  // tiles staged at once (256: 10 % slower, fewer waves)
+// a wave's words (u32 bits, and filling u16 tiles before), or its stage
+constexpr uint32_t kFillWork = 6 * kLightEdges, kCountWork = 4 * kLightEdges;
+static_assert(kStageTiles * 36 <= (int)kFillWork, "the stage fits over the words");
+
+// Orders this wave's LDS accesses between its lanes.  The LDS unit runs a
+// wave's operations in their order, so only the compiler has to be held.
+__device__ __forceinline__ void wave_lds_order()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+}
+
+__host__ __device__ inline uint32_t wave_lds_bytes(int32_t sums, bool fill)
+{
+    return align16(8u * (uint32_t)sums) + 4 * kWave + (fill ? 4 * 32 + 4 * 16 + kFillWork : kCountWork);
+}
+
+constexpr uint32_t kHubHead = (sizeof(HubHead) + 15) / 16 * 16;
+
+__host__ __device__ inline uint32_t convert_lds_bytes(int32_t W, bool fill)
+{
+    const uint32_t light = kWavesPerWg * wave_lds_bytes((W + 1023) / 1024, fill);
+    const uint32_t hub = kHubHead + hub_work_bytes(W, fill);
+    return light > hub ? light : hub;
+}
+
+template <int V>
+struct IntC {
+    static constexpr int value = V;
+};
+
+template <int G, typename Fn>
+__device__ __forceinline__ void for_groups_from(int32_t E, Fn& fn)
+{
+    if constexpr (G * kWaveGroup < kWaveSlots) {
+        if (E <= kWave * kWaveGroup * G) return;
+        fn(IntC<G>());
+        for_groups_from<G + 1>(E, fn);
+    }
+}
+
+// Calls fn(slot) for the slots that hold one of E edges, kWaveGroup slots per
+// uniform branch; fn masks the lanes past the window's last edge.
+template <typename Fn>
+__device__ __forceinline__ void for_slots(int32_t E, Fn&& fn)
+{
+    auto group = [&](auto G) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = kWaveGroup * G.value; j < kWaveGroup * (G.value + 1); ++j) fn(j);
+    };
+    for_groups_from<0>(E, group);
 }
 
 template <bool FILL>
-__global__ void __launch_bounds__(kConvThreads) __attribute__((amdgpu_waves_per_eu(4, 8)))
-convert_light(const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ col_idx,
+__global__ void __launch_bounds__(kConvThreads) __attribute__((amdgpu_waves_per_eu(FILL ? 5 : 8)))
+convert_waves(const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ col_idx,
               int32_t n, int64_t nnz, int32_t W, int32_t* __restrict__ counts,
               const int32_t* __restrict__ window_offsets, int32_t* __restrict__ block_col,
-              uint16_t* __restrict__ tile_mask, HubList hl, int32_t* __restrict__ err)
+              uint16_t* __restrict__ tile_mask, bool stream, int32_t hub_wgs,
+              const int2* __restrict__ seg,
+              const int32_t* __restrict__ hubs, int32_t* __restrict__ err)
 {
-    const LightLayout lay = light_layout(W, FILL);
-    const LightLds L = light_lds(lay);
-    const int tid = threadIdx.x;
-    const int wid = tid / kWave;
-    const int32_t G = gridDim.x;
-    int32_t w = blockIdx.x;
-    if (w >= W) return;   // uniform
-    for (int g = tid; g < (L.words + 3) / 4; g += kConvThreads)
-        *reinterpret_cast<uint4*>(&L.bits[4 * g]) = make_uint4(0u, 0u, 0u, 0u);
-    if constexpr (FILL) {
-        for (int g = tid; g < kMaskTiles * 2; g += kConvThreads)
-            *reinterpret_cast<uint4*>(&L.masks[4 * g]) = make_uint4(0u, 0u, 0u, 0u);
-        for (int g = tid; g < 2 * L.sums; g += kConvThreads) L.summary[g] = 0u;   // + scnt
-    }
-    if (tid < kMiscInts) L.cnt[tid] = 0;
-    const int32_t total_tiles = FILL ? window_offsets[W] : 0;
-    // descriptions in flight (every wave fetches them; wave 0 publishes)
-    int32_t aheadX = 0, aheadY = 0;
-    {
-        const int32_t v0 = fetch_meta<FILL>(w, W, n, row_ptr, window_offsets);
-        const int32_t v1 = fetch_meta<FILL>(w + G, W, n, row_ptr, window_offsets);
-        aheadX = fetch_meta<FILL>(w + 2 * G, W, n, row_ptr, window_offsets);
-        if (wid == 0) {
-            publish_meta<FILL>(L, 0, v0, w, W, n, nnz, total_tiles, err);
-            publish_meta<FILL>(L, 1, v1, w + G, W, n, nnz, total_tiles, err);
+    if ((int32_t)blockIdx.x < hub_wgs) {
+        HubHead& head = *reinterpret_cast<HubHead*>(conv_lds);
+        for (int32_t i = blockIdx.x;; i += hub_wgs) {
+            const int32_t w = hub_entry(i, W, seg, hubs, head.scan);
+            if (w < 0 || w >= W) return;   // uniform: past the list's end
+            hub_window<FILL>(w, row_ptr, col_idx, n, nnz, W, counts, window_offsets, block_col,
+                             tile_mask, stream, head, conv_lds + kHubHead,
+                             convert_lds_bytes(W, FILL) - kHubHead, err);
         }
     }
-    lds_barrier();
-
-    static_assert(kLightEPT == 4, "the register uses in the loop name every edge register");
-    int32_t colA[kLightEPT], colB[kLightEPT];
-    uint32_t rowsA = 0, rowsB = 0;
-    int cntA = 0, cntB = 0;
-    int round = 0;
-    int slot = 0;   // ring slot of the current window
-    issue_edges<FILL>(L, 0, col_idx, colA, rowsA, cntA);
-    // Two windows per trip so that the register sets alternate without copies
-    // (a copy would wait for the loads in flight).  Each half first uses the
-    // registers loaded one window ago -- gfx950 counts loads and stores with
-    // one counter, so once a store is pending any wait is a wait for
-    // everything, and it must come before the next window's loads issue --
-    // then publishes the description of w + 2G into the ring slot whose last
-    // readers (window w - G) are past a barrier, issues the loads of w + G
-    // and w + 3G, and works on w.
-    while (true) {
-        {
-            const int s1 = slot == 2 ? 0 : slot + 1, s2 = s1 == 2 ? 0 : s1 + 1;
-            asm volatile("" ::"v"(colA[0]), "v"(colA[1]), "v"(colA[2]), "v"(colA[3]), "v"(aheadX));
-            if (wid == 0) publish_meta<FILL>(L, s2, aheadX, w + 2 * G, W, n, nnz, total_tiles, err);
-            aheadY = fetch_meta<FILL>(w + 3 * G, W, n, row_ptr, window_offsets);
-            issue_edges<FILL>(L, s1, col_idx, colB, rowsB, cntB);
-            light_window<FILL>(L, slot, w, colA, rowsA, cntA, round, n, counts, block_col,
-                               tile_mask, hl, err);
-            w += G;
-            slot = s1;
-            if (w >= W) break;
-        }
-        {
-            const int s1 = slot == 2 ? 0 : slot + 1, s2 = s1 == 2 ? 0 : s1 + 1;
-            asm volatile("" ::"v"(colB[0]), "v"(colB[1]), "v"(colB[2]), "v"(colB[3]), "v"(aheadY));
-            if (wid == 0) publish_meta<FILL>(L, s2, aheadY, w + 2 * G, W, n, nnz, total_tiles, err);
-            aheadX = fetch_meta<FILL>(w + 3 * G, W, n, row_ptr, window_offsets);
-            issue_edges<FILL>(L, s1, col_idx, colA, rowsA, cntA);
-            light_window<FILL>(L, slot, w, colB, rowsB, cntB, round, n, counts, block_col,
-                               tile_mask, hl, err);
-            w += G;
-            slot = s1;
-            if (w >= W) break;
-        }
-    }
-    if (tid == 0 && *L.bad) atomicOr(err, kErrCol);
-}
-
-// ---------------------------------------------------------------------------
-// count_waves: the count pass of graphs whose bitmap is small (W <=
-// 32 * kWaveCountMaxWords windows): one window per wave, each wave with a
-// bitmap of its own in LDS, so a window costs no workgroup barrier.  A wave
-// takes windows w, w + GW, w + 2 GW, ... (GW waves in the grid); while it
-// marks one window, the columns of its next window and the row pointers of
-// the one after are in flight.  Its counts leave 64 windows at a time (lane
-// k keeps the count of the batch's k-th window): gfx950 counts loads and
-// stores with one counter, so a store pending at every window would make
-// each wait a wait for the prefetched loads too.  Windows of more than
-// kLightEdges edges are listed for count_hubs, which writes their counts
-// (the zero this pass leaves there is overwritten).  Same counts, same hub
-// list and same error bits as convert_light<false>; on graphs of many block
-// columns the bitmap per wave leaves fewer windows in flight per CU than
-// convert_light's shared one, which is used there.
-// ---------------------------------------------------------------------------
-constexpr int kWaveCountWaves = 4;                   // waves per workgroup
-constexpr int kWaveCountEPL = kLightEdges / kWave;   // edge slots per lane
-constexpr int32_t kWaveCountMaxWords = 2048;         // 8 KB of bitmap per wave
-
-struct WaveWin {
-    int32_t e0, E;
-    bool ok;   // row pointers usable
-};
-
-// Row pointers of window wn: lane t <= nrows holds row_ptr[16 wn + t]; the
-// other lanes (and every lane past the last window) load past the end of
-// the descriptor `rp` over row_ptr[0..n], which reads 0 -- one unconditional
-// load, so nothing waits for it before its value is used.
-__device__ __forceinline__ int32_t wave_fetch_rp(__amdgpu_buffer_rsrc_t rp, int32_t n, int32_t W,
-                                                 int64_t wn, int lane)
-{
-    uint32_t off = 4u * ((uint32_t)n + 1u);   // out of range
-    if (wn < W) {
-        const int nrows = min(16, n - (int32_t)wn * 16);
-        if (lane <= nrows) off = 4u * (uint32_t)(wn * 16 + lane);
-    }
-    return (int32_t)__builtin_amdgcn_raw_buffer_load_b32(rp, off, 0, 0);
-}
-
-// The window's edge range, and whether its row pointers are usable (0 <=
-// rp[0] <= ... <= rp[nrows] <= nnz), from the fetched row pointers; all
-// wave-uniform (scalar).
-__device__ __forceinline__ WaveWin wave_describe(int32_t v, int32_t n, int64_t nnz, int64_t wn,
-                                                 int32_t W, int lane)
-{
-    WaveWin d{0, 0, false};
-    if (wn >= W) return d;
-    const int nrows = min(16, n - (int32_t)wn * 16);
-    const int32_t rp0 = __builtin_amdgcn_readfirstlane(__shfl(v, 0, kWave));
-    const int32_t rpn = __builtin_amdgcn_readfirstlane(__shfl(v, nrows, kWave));
-    const int32_t nxt = __shfl_down(v, 1, kWave);
-    const bool back = lane < nrows && nxt < v;
-    d.ok = !__any(back) && rp0 >= 0 && rpn >= rp0 && (int64_t)rpn <= nnz;
-    d.e0 = rp0;
-    d.E = d.ok ? rpn - rp0 : 0;
-    return d;
-}
-
-// Issues the loads of a light window's columns: edge lane + 64 j in col[j],
-// through a buffer descriptor over the window's edges (32-bit offsets; a
-// load past them reads 0 and touches no memory).  The values are not used
-// here, so the loads stay in flight.
-__device__ __forceinline__ void wave_issue_cols(const WaveWin& d,
-                                                const int32_t* __restrict__ col_idx, int lane,
-                                                int32_t (&col)[kWaveCountEPL])
-{
-    const int32_t E = d.E <= kLightEdges ? d.E : 0;   // hubs and unusable windows: none
-    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<int32_t*>(col_idx) + (E > 0 ? d.e0 : 0), (short)0, 4 * E, 0x00020000);
-#pragma unroll
-    for (int j = 0; j < kWaveCountEPL; ++j) {
-        if (kWave * j >= E) break;   // wave-uniform: the window has no edge here
-        col[j] = (int32_t)__builtin_amdgcn_raw_buffer_load_b32(r, 4 * (lane + kWave * j), 0, 0);
-    }
-}
-
-__global__ void __launch_bounds__(kWaveCountWaves * kWave)
-count_waves(const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ col_idx, int32_t n,
-            int64_t nnz, int32_t W, int32_t* __restrict__ counts, HubList hl,
-            int32_t* __restrict__ err)
-{
-    const int words = (W + 31) / 32;
     const int lane = threadIdx.x & (kWave - 1);
-    const int wave = threadIdx.x / kWave;
-    uint32_t* bits = reinterpret_cast<uint32_t*>(conv_lds) + (size_t)wave * words;
-    for (int i = lane; i < words; i += kWave) bits[i] = 0u;
-    F3S_WAVE_LDS_SYNC();
-    const int64_t GW = (int64_t)gridDim.x * kWaveCountWaves;
-    int64_t w = (int64_t)blockIdx.x * kWaveCountWaves + wave;
-    if (w >= W) return;   // wave-uniform; the kernel has no workgroup barrier
-
-    bool bad = false;           // a column outside [0, n) was seen
-    int32_t mycount = 0;        // count of the batch's lane-th window
-    int nb = 0;                 // windows in the batch
-    int64_t wfirst = w;         // the batch's first window
-    // Marks window wn's columns, leaves the bitmap clear again and returns
-    // its tile count (0 for an unusable, empty or hub window).
-    auto process = [&](const WaveWin& d, int64_t wn, const int32_t (&col)[kWaveCountEPL]) {
-        int32_t cnt = 0;
-        if (!d.ok) {
-            if (lane == 0) atomicOr(err, kErrRowPtr);
-        } else if (d.E > kLightEdges) {
-            if (lane == 0) list_hub(hl, (int32_t)wn, d.e0, d.E);
-        } else if (d.E > 0) {
-            int fresh = 0;
-#pragma unroll
-            for (int j = 0; j < kWaveCountEPL; ++j) {
-                if (kWave * j >= d.E) break;   // wave-uniform: no edge in this slot
-                const int32_t c = col[j];
-                if (lane + kWave * j < d.E) {
-                    if (c < 0 || c >= n) {
-                        bad = true;
-                    } else {
-                        const uint32_t bit = 1u << ((c >> 4) & 31);
-                        fresh += (atomicOr(&bits[c >> 9], bit) & bit) == 0u;
-                    }
-                }
-            }
-            cnt = wave_sum(fresh);
-            F3S_WAVE_LDS_SYNC();   // every mark is done before the clears
-#pragma unroll
-            for (int j = 0; j < kWaveCountEPL; ++j) {
-                if (kWave * j >= d.E) break;
-                const int32_t c = col[j];
-                if (lane + kWave * j < d.E && c >= 0 && c < n) bits[c >> 9] = 0u;
-            }
-            F3S_WAVE_LDS_SYNC();
-        }
-        if (lane == nb) mycount = cnt;
-        if (++nb == kWave) {
-            counts[wfirst + lane * GW] = mycount;
-            nb = 0;
-            wfirst = wn + GW;
-        }
-    };
-
-    const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<int32_t*>(row_ptr), (short)0, (int32_t)(4 * ((int64_t)n + 1)), 0x00020000);
-    int32_t colA[kWaveCountEPL], colB[kWaveCountEPL];
-    WaveWin dA = wave_describe(wave_fetch_rp(rp, n, W, w, lane), n, nnz, w, W, lane);
-    int32_t rpN = wave_fetch_rp(rp, n, W, w + GW, lane);   // next window, in flight
-    wave_issue_cols(dA, col_idx, lane, colA);
-    WaveWin dB;
-    // Two windows per trip so that the two column register sets alternate
-    // without copies (a copy would wait for the loads in flight).
-    while (true) {
-        dB = wave_describe(rpN, n, nnz, w + GW, W, lane);
-        wave_issue_cols(dB, col_idx, lane, colB);
-        rpN = wave_fetch_rp(rp, n, W, w + 2 * GW, lane);
-        process(dA, w, colA);
-        w += GW;
-        if (w >= W) break;
-        dA = wave_describe(rpN, n, nnz, w + GW, W, lane);
-        wave_issue_cols(dA, col_idx, lane, colA);
-        rpN = wave_fetch_rp(rp, n, W, w + 2 * GW, lane);
-        process(dB, w, colB);
-        w += GW;
-        if (w >= W) break;
+    // (read into a scalar register: the compiler then knows that everything
+    // about the window is the same for the whole wave)
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int32_t w = ((int32_t)blockIdx.x - hub_wgs) * kWavesPerWg + wave;
+    if (w >= W) return;
+    // lane t <= nrows: row_ptr[16 w + t]; filling, lanes 17 and 18 the
+    // window's output offsets, lane 19 the tiles in all
+    const int nrows = min(16, n - w * 16);
+    int32_t v = 0;
+    {
+        const int32_t* p = nullptr;
+        if (lane <= nrows) p = row_ptr + (int64_t)w * 16 + lane;
+        if (FILL && (lane == 17 || lane == 18)) p = window_offsets + w + (lane - 17);
+        if (FILL && lane == 19) p = window_offsets + W;
+        if (p) v = *p;
     }
-    if (lane < nb) counts[wfirst + lane * GW] = mycount;
-    if (__any(bad) && lane == 0) atomicOr(err, kErrCol);
-}
+    const int32_t sums = (W + 1023) / 1024;
+    unsigned char* lds = conv_lds + wave * wave_lds_bytes(sums, FILL);
+    uint2* sp = reinterpret_cast<uint2*>(lds);   // .x words that hold an edge, .y words before
+    // lanes with nothing to OR do so here, each in its own word
+    uint32_t* dummy = reinterpret_cast<uint32_t*>(lds + align16(8u * (uint32_t)sums));
+    uint32_t* start = dummy + kWave;   // (fill) a bit for the first edge of each non-empty row
+    uint32_t* rowtab = start + 32;     // (fill) the i-th non-empty row
+    uint32_t* bits = dummy + kWave + (FILL ? 32 + 16 : 0);
+    uint16_t* base = reinterpret_cast<uint16_t*>(bits + kLightEdges);   // (fill) tiles before a word
+    uint32_t* masks = bits;   // (fill) the stage, once the ranks are known
+    int32_t* tcol = reinterpret_cast<int32_t*>(bits + kStageTiles * 8);
+    for (int i = lane; i < sums; i += kWave) sp[i].x = 0u;
+    if (FILL && lane < 32) start[lane] = 0u;
 
-// ---------------------------------------------------------------------------
-// count_hubs: the count pass of the hub windows the main pass listed, one
-// kHubCountThreads workgroup per window (any order, a grid-stride loop over
-// the list): every edge ORs its block column's bit into an LDS bitmap, and
-// the bits set for the first time add up to the window's tile count.  The
-// edges are read in coalesced chunks of kHubCountThreads * kHubCountEPT, all
-// loads of a chunk in flight at once.  Measured on config 4's 1,310 hubs:
-// 13 us, against 29 us with the fill pass's 1024-thread kernel plus 10 us to
-// order the list first.
-// ---------------------------------------------------------------------------
-constexpr int kHubCountEPT = 8;
-
-__global__ void __launch_bounds__(kHubCountThreads)
-count_hubs(const int32_t* __restrict__ col_idx, int32_t n, int64_t nnz, int32_t W,
-           int32_t* __restrict__ counts, HubList hl, int32_t* __restrict__ err)
-{
-    constexpr int NT = kHubCountThreads;
-    constexpr int32_t kChunk = NT * kHubCountEPT;
-    uint32_t* bits = reinterpret_cast<uint32_t*>(conv_lds);
-    const int words4 = ((W + 31) / 32 + 3) & ~3;
-    int32_t* scan = reinterpret_cast<int32_t*>(conv_lds) + words4;   // [NT / 64]
-    int32_t* bad = scan + NT / kWave;
-    const int tid = threadIdx.x;
-    const int32_t nh = min(*hl.count, hl.cap);
-    if ((int32_t)blockIdx.x >= nh) return;   // uniform
-    for (int g = tid; g < words4 / 4; g += NT)
-        reinterpret_cast<uint4*>(bits)[g] = make_uint4(0u, 0u, 0u, 0u);
-    if (tid == 0) *bad = 0;
-    for (int32_t i = blockIdx.x; i < nh; i += gridDim.x) {
-        const int4 h = hl.hubs[i];
-        const int32_t w = h.x, e0 = h.y, E = h.z;
-        // (the main pass listed the window with usable row pointers; the
-        // check keeps every access in bounds whatever the list holds)
-        if ((uint32_t)w >= (uint32_t)W || e0 < 0 || E <= 0 || (int64_t)e0 + E > nnz)
-            continue;   // uniform
-        __syncthreads();   // the previous window's bitmap is clear
-        int32_t fresh = 0;
-        for (int64_t c0 = 0; c0 < E; c0 += kChunk) {
-            int32_t col[kHubCountEPT];
-#pragma unroll
-            for (int j = 0; j < kHubCountEPT; ++j) {
-                const int64_t e = c0 + tid + NT * j;
-                col[j] = e < E ? col_idx[e0 + e] : 0;
-            }
-#pragma unroll
-            for (int j = 0; j < kHubCountEPT; ++j) {
-                const int64_t e = c0 + tid + NT * j;
-                if (e >= E) continue;
-                const int32_t c = col[j];
-                if (c < 0 || c >= n) {
-                    *bad = 1;
-                    continue;
-                }
-                const uint32_t bit = 1u << ((c >> 4) & 31);
-                fresh += (atomicOr(&bits[c >> 9], bit) & bit) == 0u;
-            }
-        }
-        int32_t T;
-        (void)block_exclusive_scan<NT>(fresh, scan, T);   // barriers inside: the marks are done
-        if (tid == 0) counts[w] = T;
-        for (int g = tid; g < words4 / 4; g += NT)
-            reinterpret_cast<uint4*>(bits)[g] = make_uint4(0u, 0u, 0u, 0u);
+    const int32_t e0 = __builtin_amdgcn_readlane(v, 0);
+    const int32_t end = __builtin_amdgcn_readlane(v, nrows);
+    const int32_t nxt = __builtin_amdgcn_update_dpp(0, v, 0x130, 0xf, 0xf, false);   // lane + 1's
+    const bool in_rows = lane < nrows;
+    const uint64_t back = __ballot(in_rows && nxt < v);
+    const uint64_t nonempty = __ballot(in_rows && nxt > v);
+    const int32_t E = window_edges(e0, end);
+    const bool rows_ok = back == 0 && e0 >= 0 && end >= e0 && (int64_t)end <= nnz;
+    int32_t out_base = 0, expect = 0;
+    bool out_ok = true;
+    if constexpr (FILL) {
+        const int32_t oe = __builtin_amdgcn_readlane(v, 18);
+        out_base = __builtin_amdgcn_readlane(v, 17);
+        expect = oe - out_base;
+        out_ok = out_base >= 0 && oe >= out_base && oe <= __builtin_amdgcn_readlane(v, 19);
     }
-    __syncthreads();
-    if (tid == 0 && *bad) atomicOr(err, kErrCol);
-}
-
-// Hub windows heaviest first, for the fill pass.  The main pass lists them
-// in the order its workgroups find them; rank_hubs writes their windows again,
-// ordered by descending edge count (ties: ascending window index, so the
-// order is deterministic), and the hub launch that follows gives each listed
-// window a workgroup of its own, dispatched in list order, so the longest
-// windows start first.  Every workgroup of rank_hubs loads the keys of the
-// whole list (up to kHubSortCap) into LDS and places 64 of them at their
-// ranks, four lanes per entry each counting the smaller keys in a quarter of
-// the list; keys are unique, so the ranks are a permutation.  A longer list
-// is copied as listed.
-constexpr int kHubSortCap = 4096;
-constexpr int kHubLaunch = 2048;   // hub-launch workgroups (one per listed window up to this)
-
-__global__ void __launch_bounds__(256)
-rank_hubs(int32_t W, HubList hl, int32_t* __restrict__ sorted)
-{
-    __shared__ __align__(16) uint64_t key[kHubSortCap];
-    const int32_t nh = min(*hl.count, hl.cap);
-    const int tid = threadIdx.x;
-    if (nh > kHubSortCap) {   // uniform: copy in listing order
-        for (int64_t i = (int64_t)blockIdx.x * 256 + tid; i < nh; i += (int64_t)gridDim.x * 256)
-            sorted[i] = hl.hubs[i].x;
+    if (rows_ok && E > kLightEdges) return;   // a hub window: list_hubs has it
+    if (!rows_ok || !out_ok || E == 0) {
+        if (lane == 0) {
+            if (!FILL) counts[w] = 0;
+            if (!rows_ok)
+                atomicOr(err, kErrRowPtr);
+            else if (FILL && (!out_ok || expect != 0))
+                atomicOr(err, kErrCount);
+        }
         return;
     }
-    const int32_t base = blockIdx.x * 64;
-    if (base >= nh) return;   // uniform
-    constexpr int kPer = kHubSortCap / 256;
-    int4 h[kPer];
-#pragma unroll
-    for (int k = 0; k < kPer; ++k) {
-        const int i = tid + 256 * k;
-        h[k] = i < nh ? hl.hubs[i] : make_int4(-1, 0, 0, 0);
+
+    int32_t col[kWaveSlots];
+    const __amdgpu_buffer_rsrc_t er = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<int32_t*>(col_idx) + e0, (short)0, 4 * E, 0x00020000);
+    for_slots(E, [&](int j) __attribute__((always_inline)) {
+        col[j] = (int32_t)__builtin_amdgcn_raw_buffer_load_b32(er, 4 * lane + 4 * kWave * j, 0, 0);
+    });
+    if (FILL && ((nonempty >> lane) & 1ull)) {
+        const int32_t pos = v - e0;
+        atomicOr(&start[pos >> 5], 1u << (pos & 31));
+        rowtab[__builtin_amdgcn_mbcnt_lo((uint32_t)nonempty, 0u)] = (uint32_t)lane;
     }
-#pragma unroll
-    for (int k = 0; k < kPer; ++k) {
-        // (~edges, window) ascending = edges descending, window ascending; an
-        // entry naming no window sorts last, keyed by its position
-        const int i = tid + 256 * k;
-        if (i >= nh) break;
-        uint64_t key_i = (0xffffffffull << 32) | (uint32_t)i;
-        if ((uint32_t)h[k].x < (uint32_t)W) {
-            const uint32_t edges = (uint32_t)max(1, h[k].z);
-            key_i = ((uint64_t)(~edges) << 32) | (uint32_t)h[k].x;
+
+    // ---- mark ----
+    bool bad = false;
+    for_slots(E, [&](int j) __attribute__((always_inline)) {
+        const bool in = lane < E - kWave * j;   // (a scalar subtraction)
+        const int32_t c = col[j];
+        const bool ok = in && (uint32_t)c < (uint32_t)n;
+        bad |= in && !ok;
+        const int32_t wi = ok ? c >> 9 : -1;
+        col[j] = ok ? c : -1;
+        const int32_t pw = __builtin_amdgcn_update_dpp(-1, wi, 0x111, 0xf, 0xf, false);   // lane - 1's
+        uint32_t* p = wi != pw ? &sp[wi >> 5].x : &dummy[lane];
+        if (!ok) p = &dummy[lane];
+        atomicOr(p, 1u << (wi & 31));
+    });
+    if (__any(bad) && lane == 0) atomicOr(err, kErrCol);
+    wave_lds_order();
+    int32_t nw = 0;
+    for (int s0 = 0; s0 < sums; s0 += kWave) {
+        const int sw = s0 + lane;
+        const int cnt = sw < sums ? __popc(sp[sw].x) : 0;
+        const int incl = wave_scan_incl(cnt);
+        if (sw < sums) sp[sw].y = (uint32_t)(nw + incl - cnt);
+        nw += __builtin_amdgcn_readlane(incl, kWave - 1);
+    }
+    // ---- words (nw <= E <= kLightEdges) ----
+    for (int k = 0; k < nw; k += kWave) bits[k + lane] = 0u;
+    wave_lds_order();
+    uint32_t aux[kWaveSlots];   // the edge's word; then its place in the masks
+    for_slots(E, [&](int j) __attribute__((always_inline)) {
+        asm volatile("" : "+v"(col[j]));   // recompute, do not keep across phases
+        const int32_t c = col[j];
+        const int32_t wi = max(c, 0) >> 9;
+        const uint2 s = sp[wi >> 5];
+        const uint32_t ci = s.y + __popc(s.x & ((1u << (wi & 31)) - 1u));
+        aux[j] = ci;
+        atomicOr(c >= 0 ? &bits[ci] : &dummy[lane], 1u << ((c >> 4) & 31));
+    });
+    wave_lds_order();
+    if constexpr (!FILL) {
+        int32_t t = 0;
+        for (int k = lane; k < nw; k += kWave) t += __popc(bits[k]);
+        t = wave_scan_incl(t);
+        if (lane == kWave - 1) counts[w] = t;
+    } else {
+        // ---- ranks ----
+        int32_t total = 0;
+        for (int k0 = 0; k0 < nw; k0 += kWave) {
+            const int k = k0 + lane;
+            const int cnt = k < nw ? __popc(bits[k]) : 0;
+            const int incl = wave_scan_incl(cnt);
+            base[k] = (uint16_t)(total + incl - cnt);
+            total += __builtin_amdgcn_readlane(incl, kWave - 1);
         }
-        key[i] = key_i;
+        wave_lds_order();
+        if (total != expect) {
+            if (lane == 0) atomicOr(err, kErrCount);
+            if (total > expect) return;
+        }
+        // an edge's row: the first edges of the non-empty rows up to its own
+        const uint32_t starts = start[lane & 31];
+        const bool full = nonempty == 0xffffull;   // uniform: every row has an edge
+        int32_t rowrun = -1;
+        for_slots(E, [&](int j) __attribute__((always_inline)) {
+            const uint32_t lo = __builtin_amdgcn_readlane(starts, 2 * j);
+            const uint32_t hi = __builtin_amdgcn_readlane(starts, 2 * j + 1);
+            const uint64_t m = ((uint64_t)hi << 32) | lo;
+            const uint64_t m1 = m >> 1;
+            const int32_t idx = (int32_t)__builtin_amdgcn_mbcnt_hi(
+                (uint32_t)(m1 >> 32),
+                __builtin_amdgcn_mbcnt_lo((uint32_t)m1, (uint32_t)(rowrun + (int32_t)(lo & 1u))));
+            rowrun += __popcll(m);
+            asm volatile("" : "+v"(col[j]));
+            const int32_t c = col[j];
+            const uint32_t r = full ? (uint32_t)idx : rowtab[idx];
+            const uint32_t ci = aux[j];
+            const uint32_t below = (1u << ((c >> 4) & 31)) - 1u;
+            const uint32_t t = base[ci] + __popc(bits[ci] & below);
+            // byte offset of the (tile, row pair) word, its bit's position above
+            aux[j] = c >= 0 ? t * 32 + (r >> 1) * 4 + (((c & 15) + 16 * (r & 1)) << 16) : 0xffffu;
+        });
+        // ---- stage ----
+        for (int32_t ms = 0; ms < total; ms += kStageTiles) {
+            wave_lds_order();
+            const int32_t nt = min(kStageTiles, total - ms);
+            for (int k = lane; k < 2 * nt; k += kWave)
+                reinterpret_cast<uint4*>(masks)[k] = make_uint4(0u, 0u, 0u, 0u);
+            wave_lds_order();
+            for_slots(E, [&](int j) __attribute__((always_inline)) {
+                asm volatile("" : "+v"(col[j]), "+v"(aux[j]));
+                const uint32_t o = (aux[j] & 0xffffu) - (uint32_t)ms * 32;
+                if (o < (uint32_t)nt * 32) {
+                    atomicOr(&masks[o >> 2], 1u << (aux[j] >> 16));
+                    tcol[o >> 5] = col[j] >> 4;   // every edge of the tile writes the same
+                }
+            });
+            wave_lds_order();
+            const int64_t o = (int64_t)out_base + ms;
+            for (int k = lane; k < nt; k += kWave) block_col[o + k] = tcol[k];
+            if (tile_mask) {
+                store_masks(reinterpret_cast<uint4*>(tile_mask + o * 16),
+                            reinterpret_cast<const uint4*>(masks), 2 * nt, lane, kWave, stream);
+            }
+        }
     }
-    __syncthreads();
-    // lanes 4e..4e+3 of a wave rank entry base + tid / 4, each over a quarter
-    // of the list in steps of eight keys (four 16-byte LDS reads, from a
-    // multiple of 8); their counts add up with two lane swaps
-    const int32_t i = base + tid / 4;
-    const uint64_t ki = key[i < nh ? i : 0];
-    const int32_t quarter = ((nh + 31) / 32) * 8;   // a multiple of 8
-    const int32_t j0 = min(nh, (tid & 3) * quarter), j1 = min(nh, j0 + quarter);
-    int32_t rank = 0;
-    int32_t j = j0;
-    for (; j + 8 <= j1; j += 8) {
-        const ulonglong2* k2 = reinterpret_cast<const ulonglong2*>(&key[j]);
-        const ulonglong2 a = k2[0], b = k2[1], c = k2[2], d = k2[3];
-        rank += (a.x < ki) + (a.y < ki) + (b.x < ki) + (b.y < ki) + (c.x < ki) + (c.y < ki) +
-                (d.x < ki) + (d.y < ki);
-    }
-    for (; j < j1; ++j) rank += key[j] < ki ? 1 : 0;
-    rank += __shfl_xor(rank, 1, kWave);
-    rank += __shfl_xor(rank, 2, kWave);
-    if (i < nh && (tid & 3) == 0)
-        sorted[rank] = (ki >> 32) == 0xffffffffull ? -1 : (int32_t)(uint32_t)ki;
 }
 
-// int64 window offsets -> the caller's int32 offsets; thread 0 also reports
-// the error bits and the tile count for the host (status[0], status[1]).
 // ---------------------------------------------------------------------------
 // Counts -> window_offsets in two launches: block sums, then each workgroup
 // adds up the sums of the blocks before its own (at most kOffsFusedBlocks of
-// them; wider graphs scan the sums in one workgroup first), scans its block
+// them; wider graphs scan the sums in one workgroup first; a single block
+// needs none), scans its block
 // straight into the int32 offsets -- T <= nnz <= INT32_MAX, since a tile
 // holds at least one edge -- and its last workgroup writes offsets[W] and the
 // host's status words (error bits, T).
@@ -1265,8 +1088,9 @@ static f3s_status counts_to_offsets(const int32_t* counts, int32_t* offsets, int
                                     hipStream_t stream)
 {
     const int64_t nb = offsets_sum_elems(W);
-    hipLaunchKernelGGL(offsets_block_sums, dim3((unsigned)nb), dim3(kOffsThreads), 0, stream,
-                       counts, W, sums);
+    if (nb > 1)
+        hipLaunchKernelGGL(offsets_block_sums, dim3((unsigned)nb), dim3(kOffsThreads), 0, stream,
+                           counts, W, sums);
     const bool scanned = nb > kOffsFusedBlocks;
     if (scanned)
         hipLaunchKernelGGL(offsets_scan_sums, dim3(1), dim3(kOffsThreads), 0, stream, sums, nb);
@@ -1286,149 +1110,79 @@ __global__ void fill_status(const int32_t* __restrict__ window_offsets, int32_t 
     }
 }
 
-// Per-call workspace of the converter, one allocation: status words (error
-// bits, the hub count, two int64 results), the hub list as found and (fill)
-// ordered heaviest first and, for the count pass, the counts, their int64
-// scan and its temporaries.
+// Per-call workspace of the converter, one allocation: the error bits, the
+// two status words where the host cannot be written to, the hub list and, for
+// the count pass, the counts and their scan's block sums.
 struct ConvertScratch {
     int32_t* err;
-    HubList hl;
-    int32_t* hubs_sorted;
     int64_t* status;
+    int2* seg;
+    int32_t* hubs;
     int32_t* counts;
     int64_t* tmp;
 };
 
 static f3s_status convert_scratch(StreamBuffer& buf, int32_t W, bool count, ConvertScratch& s)
 {
-    const size_t head = 32;   // err, hub count, pad, status[2]
-    const size_t hubs = sizeof(int4) * ((size_t)W + 1);
-    const size_t sorted = count ? 0 : sizeof(int32_t) * ((size_t)W + 1);
+    const size_t blocks = W <= kLightMaxW ? (size_t)ceil_div(W, kListBlock) : 0;
+    const size_t head = 32;   // err, pad, status[2]
+    const size_t seg = sizeof(int2) * blocks;
+    const size_t hubs = sizeof(int32_t) * blocks * kListBlock;
     const size_t counts = count ? sizeof(int32_t) * (size_t)W : 0;
     const size_t tmp = count ? sizeof(int64_t) * (size_t)offsets_sum_elems(W) : 0;
     auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
-    F3S_TRY(buf.reserve(al(head) + al(hubs) + al(sorted) + al(counts) + al(tmp)));
+    F3S_TRY(buf.reserve(al(head) + al(seg) + al(hubs) + al(counts) + al(tmp)));
     char* p = static_cast<char*>(buf.ptr);
     s.err = reinterpret_cast<int32_t*>(p);
-    s.hl.count = s.err + 1;
     s.status = reinterpret_cast<int64_t*>(p + 16);
     p += al(head);
-    s.hl.hubs = reinterpret_cast<int4*>(p);
-    s.hl.cap = W + 1;
+    s.seg = reinterpret_cast<int2*>(p);
+    p += al(seg);
+    s.hubs = reinterpret_cast<int32_t*>(p);
     p += al(hubs);
-    s.hubs_sorted = reinterpret_cast<int32_t*>(p);
-    p += al(sorted);
     s.counts = reinterpret_cast<int32_t*>(p);
     p += al(counts);
     s.tmp = reinterpret_cast<int64_t*>(p);
     return F3S_OK;
 }
 
-// Workgroups of `fn` (`threads` wide, `lds` bytes of dynamic LDS) resident
-// on the current device at once: the grid of a persistent pass.  Cached per
-// device, kernel and LDS size -- a conversion asks for three of them, and
-// the runtime's occupancy query is host time on every call.
-static f3s_status resident_workgroups(const void* fn, int threads, uint32_t lds, int64_t* out)
-{
-    struct Entry {
-        int dev;
-        const void* fn;
-        int threads;
-        uint32_t lds;
-        int64_t resident;
-    };
-    constexpr int kEntries = 32;
-    static std::mutex mu;
-    static Entry cache[kEntries];
-    static int used = 0, next = 0;
-    int dev = 0;
-    F3S_HIP(hipGetDevice(&dev));
-    {
-        std::lock_guard<std::mutex> lock(mu);
-        for (int i = 0; i < used; ++i) {
-            const Entry& e = cache[i];
-            if (e.dev == dev && e.fn == fn && e.threads == threads && e.lds == lds) {
-                *out = e.resident;
-                return F3S_OK;
-            }
-        }
-    }
-    int cus = 0, per_cu = 0;
-    F3S_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    F3S_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, threads, lds));
-    const int64_t r = (int64_t)(per_cu > 0 ? per_cu : 1) * (cus > 0 ? cus : 1);
-    {
-        std::lock_guard<std::mutex> lock(mu);
-        cache[next] = Entry{dev, fn, threads, lds, r};
-        next = (next + 1) % kEntries;
-        if (used < kEntries) ++used;
-    }
-    *out = r;
-    return F3S_OK;
-}
-
-// One pass (count or fill) over all windows: the persistent kernel with as
-// many workgroups as fit on the device at once, then the hub windows it
-// listed (the hub count is known only on the device, so the hub launches
-// have a fixed grid that walks the list).  Graphs too wide for one LDS
-// bitmap run every window through the per-window kernel.
+// One pass (count or fill) over all windows: the hub list, then one launch of
+// a workgroup per hub window and a wave per other window.  A valid CSR of nnz
+// edges has at most nnz / (kLightEdges + 1) hub windows; how many it has is
+// known on the device only, so that many hub workgroups (at most kHubLaunch)
+// look for their entry and leave if there is none.  Graphs too wide for a
+// wave's bitmap run every window through the per-window kernel.
 template <bool FILL>
 static f3s_status launch_pass(const int32_t* row_ptr, const int32_t* col_idx, int32_t n,
-                              int64_t nnz, int32_t W, int32_t* counts,
-                              const int32_t* window_offsets, int32_t* block_col,
-                              uint16_t* tile_mask, const HubList& hl, int32_t* hubs_sorted,
-                              int32_t* err, hipStream_t stream)
+                              int64_t nnz, int32_t W, const int32_t* window_offsets,
+                              int32_t* block_col, uint16_t* tile_mask, const ConvertScratch& s,
+                              hipStream_t stream)
 {
-    if (W <= 0) return F3S_OK;
-    if ((int64_t)W > 32LL * kLightMaxWords) {
-        hipLaunchKernelGGL((convert_hubs<FILL, kConvThreads>), dim3((unsigned)W), dim3(kConvThreads), 0,
-                           stream, row_ptr, col_idx, n, nnz, W, counts, window_offsets,
-                           block_col, tile_mask, nullptr, nullptr, err);
+    if (W <= 0 || W > kLightMaxW) {
+        F3S_HIP(hipMemsetAsync(s.err, 0, sizeof(int32_t), stream));
+        if (W > 0)
+            hipLaunchKernelGGL(convert_wide<FILL>, dim3((unsigned)W), dim3(kConvThreads), 0,
+                               stream, row_ptr, col_idx, n, nnz, W, s.counts, window_offsets,
+                               block_col, tile_mask, s.err);
         F3S_HIP(hipGetLastError());
         return F3S_OK;
     }
-    int64_t resident = 0;
-    if (!FILL && (int64_t)W <= 32LL * kWaveCountMaxWords) {
-        // small bitmap: the count pass with one window per wave
-        const uint32_t lds = (uint32_t)(sizeof(uint32_t) * kWaveCountWaves * ((W + 31) / 32));
-        F3S_TRY(resident_workgroups(reinterpret_cast<const void*>(count_waves),
-                                    kWaveCountWaves * kWave, lds, &resident));
-        const int64_t need = ceil_div(W, kWaveCountWaves);
-        hipLaunchKernelGGL(count_waves, dim3((unsigned)(need < resident ? need : resident)),
-                           dim3(kWaveCountWaves * kWave), lds, stream, row_ptr, col_idx, n, nnz,
-                           W, counts, hl, err);
-    } else {
-        const LightLayout lay = light_layout(W, FILL);
-        F3S_TRY(resident_workgroups(reinterpret_cast<const void*>(convert_light<FILL>),
-                                    kConvThreads, lay.bytes, &resident));
-        const unsigned grid = (unsigned)(W < resident ? W : resident);
-        hipLaunchKernelGGL((convert_light<FILL>), dim3(grid), dim3(kConvThreads), lay.bytes,
-                           stream, row_ptr, col_idx, n, nnz, W, counts, window_offsets, block_col,
-                           tile_mask, hl, err);
-    }
-    F3S_HIP(hipGetLastError());
-    if (!FILL) {
-        const uint32_t lds = (uint32_t)(4 * ((((W + 31) / 32 + 3) & ~3) + kHubCountThreads / kWave + 4));
-        F3S_TRY(resident_workgroups(reinterpret_cast<const void*>(count_hubs), kHubCountThreads,
-                                    lds, &resident));
-        hipLaunchKernelGGL(count_hubs, dim3((unsigned)(W < resident ? W : resident)),
-                           dim3(kHubCountThreads), lds, stream, col_idx, n, nnz, W, counts, hl, err);
-    } else {
-        const int32_t rank_wgs = (int32_t)ceil_div(W < kHubSortCap ? W : kHubSortCap, 64);
-        hipLaunchKernelGGL(rank_hubs, dim3((unsigned)rank_wgs), dim3(256), 0, stream, W, hl,
-                           hubs_sorted);
-        hipLaunchKernelGGL((convert_hubs<true, kHubThreads>),
-                           dim3((unsigned)(W < kHubLaunch ? W : kHubLaunch)), dim3(kHubThreads), 0,
-                           stream, row_ptr, col_idx, n, nnz, W, counts, window_offsets, block_col,
-                           tile_mask, hubs_sorted, hl.count, err);
-    }
+    hipLaunchKernelGGL(list_hubs, dim3((unsigned)ceil_div(W, kListBlock)), dim3(kListBlock), 0,
+                       stream, row_ptr, n, W, s.seg, s.hubs, s.err);
+    const int64_t most = std::min<int64_t>(nnz / (kLightEdges + 1), W);
+    const int32_t hub_wgs = (int32_t)std::min<int64_t>(most, kHubLaunch);
+    hipLaunchKernelGGL(convert_waves<FILL>, dim3((unsigned)(hub_wgs + ceil_div(W, kWavesPerWg))),
+                       dim3(kConvThreads), convert_lds_bytes(W, FILL), stream, row_ptr, col_idx,
+                       n, nnz, W, s.counts, window_offsets, block_col, tile_mask, nnz > kStreamTiles,
+                       hub_wgs, s.seg, s.hubs, s.err);
     F3S_HIP(hipGetLastError());
     return F3S_OK;
 }
 
 // Count call: tile counts, their scan into the caller's offsets, and one
 // host round trip for the error bits and T.  Fill call: the lists, and one
-// round trip for the error bits.
+// round trip for the error bits.  The last kernel of either writes the two
+// words to pinned host memory itself (a copy is one more launch).
 static f3s_status convert_impl(const int32_t* row_ptr, const int32_t* col_idx, int32_t n,
                                int64_t nnz, int32_t* window_offsets, int32_t* block_col,
                                uint16_t* tile_mask, int64_t* T_out, hipStream_t stream)
@@ -1438,20 +1192,22 @@ static f3s_status convert_impl(const int32_t* row_ptr, const int32_t* col_idx, i
     StreamBuffer buf(stream);
     ConvertScratch s;
     F3S_TRY(convert_scratch(buf, W, count, s));
-    F3S_HIP(hipMemsetAsync(s.err, 0, 2 * sizeof(int32_t), stream));   // err, hub count
+    bool pinned = false;
+    int64_t* h = host_staging(&pinned);
+    int64_t* status = pinned ? h : s.status;
     if (count) {
-        F3S_TRY(launch_pass<false>(row_ptr, col_idx, n, nnz, W, s.counts, nullptr, nullptr,
-                                   nullptr, s.hl, nullptr, s.err, stream));
-        F3S_TRY(counts_to_offsets(s.counts, window_offsets, W, s.tmp, s.err, s.status, stream));
+        F3S_TRY(launch_pass<false>(row_ptr, col_idx, n, nnz, W, nullptr, nullptr, nullptr, s,
+                                   stream));
+        F3S_TRY(counts_to_offsets(s.counts, window_offsets, W, s.tmp, s.err, status, stream));
     } else {
-        F3S_TRY(launch_pass<true>(row_ptr, col_idx, n, nnz, W, nullptr, window_offsets,
-                                  block_col, tile_mask, s.hl, s.hubs_sorted, s.err, stream));
+        F3S_TRY(launch_pass<true>(row_ptr, col_idx, n, nnz, W, window_offsets, block_col,
+                                  tile_mask, s, stream));
         hipLaunchKernelGGL(fill_status, dim3(1), dim3(64), 0, stream, window_offsets, W, s.err,
-                           s.status);
+                           status);
     }
     F3S_HIP(hipGetLastError());
-    int64_t* h = host_staging();
-    F3S_HIP(hipMemcpyAsync(h, s.status, 2 * sizeof(int64_t), hipMemcpyDeviceToHost, stream));
+    if (!pinned)
+        F3S_HIP(hipMemcpyAsync(h, s.status, 2 * sizeof(int64_t), hipMemcpyDeviceToHost, stream));
     F3S_HIP(hipStreamSynchronize(stream));
     const int32_t h_err = (int32_t)h[0];
     const int64_t total = h[1];

@@ -60,7 +60,9 @@ void dev_free_idle(void* ptr, int device);
 void dev_free_synced(void* ptr, int device);
 // Host-pinned staging words of the calling thread (16 x int64), for the small
 // device-to-host reads of counts and status that size outputs.
-int64_t* host_staging();
+// Kernels may write them too (then wait for the stream), unless *pinned comes
+// back false: no pinned memory was to be had.
+int64_t* host_staging(bool* pinned = nullptr);
 
 // Grow-only device buffer owned by a long-lived object (a plan): allocated on
 // the owner's stream, which the owner synchronises before handing the buffer

@@ -35,6 +35,20 @@ __device__ __forceinline__ T wave_inclusive_scan(T v)
     return v;
 }
 
+// Inclusive prefix sum over the wave with DPP row shifts and row broadcasts.
+__device__ __forceinline__ int wave_scan_incl(int x)
+{
+    int s = x;
+    s += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);   // row_shr:1
+    s += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);   // row_shr:2
+    s += __builtin_amdgcn_update_dpp(0, x, 0x113, 0xf, 0xf, true);   // row_shr:3
+    s += __builtin_amdgcn_update_dpp(0, s, 0x114, 0xf, 0xe, true);   // row_shr:4, lanes 4-15
+    s += __builtin_amdgcn_update_dpp(0, s, 0x118, 0xf, 0xc, true);   // row_shr:8, lanes 8-15
+    s += __builtin_amdgcn_update_dpp(0, s, 0x142, 0xa, 0xf, true);   // row_bcast:15 -> rows 1, 3
+    s += __builtin_amdgcn_update_dpp(0, s, 0x143, 0xc, 0xf, true);   // row_bcast:31 -> rows 2, 3
+    return s;
+}
+
 template <typename T>
 __device__ __forceinline__ T wave_sum(T v)
 {

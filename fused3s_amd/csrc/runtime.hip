@@ -260,18 +260,22 @@ void dev_free_synced(void* ptr, int device)
     if (switch_dev) (void)hipSetDevice(cur);
 }
 
-int64_t* host_staging()
+int64_t* host_staging(bool* pinned)
 {
     thread_local int64_t* words = nullptr;   // one small pinned block per host thread
     if (!words) {
         void* p = nullptr;
-        if (hipHostMalloc(&p, 16 * sizeof(int64_t), hipHostMallocDefault) != hipSuccess) {
+        // portable and mapped: kernels on any device may write it
+        if (hipHostMalloc(&p, 16 * sizeof(int64_t), hipHostMallocPortable | hipHostMallocMapped) !=
+            hipSuccess) {
             (void)hipGetLastError();
             thread_local int64_t fallback[16];
+            if (pinned) *pinned = false;
             return fallback;   // pageable: correct, only slower to copy into
         }
         words = static_cast<int64_t*>(p);
     }
+    if (pinned) *pinned = true;
     return words;
 }
 

@@ -1,0 +1,85 @@
+"""The converter's main launch at the sizes where its branches meet, bit for
+bit against the oracle: windows around one wave's 1,024 edges, a hub
+workgroup's one chunk of 4,096 edges and the heavier hubs' two ways out (few
+tiles for their edges: staged beside the bitmap; many: atomics on the zeroed
+output), windows around a stage of 160 tiles, rows in any order, empty rows,
+and the lists without masks."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import _oracle as orc
+from conftest import rng
+
+pytestmark = pytest.mark.gpu
+
+
+def window_graph(windows: dict[int, np.ndarray], n: int, sort: bool, seed: int):
+    """CSR of n nodes; windows[w] = columns dealt at random to the 16 rows of
+    window w (some rows get none)."""
+    r = rng(seed)
+    rows, cols = [], []
+    for w, c in windows.items():
+        used = r.choice(16, size=int(r.integers(1, 17)), replace=False)
+        rows.append(16 * w + r.choice(used, len(c)))
+        cols.append(c)
+    rr = np.concatenate(rows).astype(np.int64)
+    cc = np.concatenate(cols).astype(np.int64)
+    order = np.lexsort((cc, rr)) if sort else np.argsort(rr, kind="stable")
+    rr, cc = rr[order], cc[order]
+    rp = np.zeros(n + 1, np.int64)
+    np.add.at(rp, rr + 1, 1)
+    return np.cumsum(rp).astype(np.int32), cc.astype(np.int32)
+
+
+def check(gpu, rp, ci, masks=True):
+    n = len(rp) - 1
+    offs, bcol, mask = orc.convert(n, rp, ci)
+    bsf = gpu.convert_device(gpu.DeviceCSR(rp, ci), masks=masks)
+    assert np.array_equal(bsf.window_offsets.numpy(), offs)
+    assert np.array_equal(bsf.block_col.numpy(), bcol)
+    if masks:
+        assert np.array_equal(bsf.tile_mask.numpy().reshape(-1, 16), mask)
+
+
+@pytest.mark.parametrize("n", [16 * 1023 + 5, 16 * 1024, 16 * 2050, 70_001])
+@pytest.mark.parametrize("sort", [True, False])
+def test_window_sizes(gpu, n, sort):
+    r = rng(n + sort)
+    W = (n + 15) // 16
+    edges = (1, 63, 64, 65, 127, 128, 129, 1023, 1024, 1025, 4095, 4096, 4097, 8200)
+    windows = {}
+    for k, E in enumerate(edges):
+        windows[3 + 5 * k] = r.integers(0, n, E)               # columns anywhere
+        windows[5 + 5 * k] = 16 * 7 + r.integers(0, 16 * 40, E)   # within 40 block columns
+    windows[W - 1] = r.integers(0, n, 300)
+    last = n - 16 * (W - 1)   # rows of the last window
+    rp, ci = window_graph(windows, 16 * W, sort, 5)
+    if last < 16:             # its edges move to the rows it has
+        e0 = rp[16 * (W - 1)]
+        rp = np.concatenate([rp[:16 * (W - 1) + 1], np.full(last, rp[-1], np.int32)])
+        ci[e0:] = np.sort(ci[e0:]) if sort else ci[e0:]
+    check(gpu, rp, ci)
+
+
+@pytest.mark.parametrize("tiles", [159, 160, 161, 320, 321, 1000])
+def test_stage_rounds(gpu, tiles):
+    # every block column once, in one wave's window and in a hub window
+    n = 16 * 1100
+    r = rng(tiles)
+    c = 16 * np.arange(tiles) + r.integers(0, 16, tiles)
+    windows = {0: c, 9: np.concatenate([c, r.choice(c, 1100), r.choice(c, 100)])}
+    rp, ci = window_graph(windows, n, True, 6)
+    check(gpu, rp, ci)
+
+
+def test_many_hubs_and_lists_without_masks(gpu):
+    # more hub windows than one list block's share, light ones between them
+    n = 16 * 2100
+    r = rng(3)
+    windows = {w: r.integers(0, n, int(r.integers(1000, 1200)) if w % 3 else 5000)
+               for w in range(0, 2100, 2)}
+    rp, ci = window_graph(windows, n, True, 7)
+    check(gpu, rp, ci)
+    check(gpu, rp, ci, masks=False)
