@@ -73,7 +73,7 @@ enum Mode : int {
 // (m, l, O) of a batch are rescaled to the batch's running max, so one pass
 // suffices.  The partials were written through to memory by segments that
 // may have run on other XCDs, and are read the same way (kCoherent).
-template <int KB>
+template <int KB, bool HALF_OUT>
 __device__ __forceinline__ void merge_split(const AttnParams& p, const SplitInfo si, int h,
                                             int lane)
 {
@@ -135,11 +135,16 @@ __device__ __forceinline__ void merge_split(const AttnParams& p, const SplitInfo
     const float inv = Ls > 0.f ? 1.0f / Ls : 0.f;
     const int32_t row = si.w * 16 + r;
     if (row < p.n) {
-        float* dst = p.O + ((int64_t)row * H + h) * kD + 16 * g;
+        const int64_t at = ((int64_t)row * H + h) * kD + 16 * g;
 #pragma unroll
-        for (int v = 0; v < 4; ++v)
-            *reinterpret_cast<float4*>(dst + 4 * v) =
-                make_float4(o[v].x * inv, o[v].y * inv, o[v].z * inv, o[v].w * inv);
+        for (int v = 0; v < 4; ++v) {
+            const f4 x = {o[v].x * inv, o[v].y * inv, o[v].z * inv, o[v].w * inv};
+            if (HALF_OUT && p.out_half)
+                *reinterpret_cast<h4*>(reinterpret_cast<_Float16*>(p.O) + at + 4 * v) =
+                    __builtin_convertvector(x, h4);
+            else
+                *reinterpret_cast<f4*>(p.O + at + 4 * v) = x;
+        }
     }
 }
 
@@ -147,11 +152,18 @@ __device__ __forceinline__ void merge_split(const AttnParams& p, const SplitInfo
 // chunk's gathers in flight per wave (double-buffered registers, 3 waves per
 // SIMD) measured no faster than one chunk per wave at 4-5 waves per SIMD, so
 // the simpler single-buffered loop is kept.
-template <int MODE, int WPG, bool WIDE, int TEAM>
+// PACKED: Q, K and V are the thirds of one [n][3][H][64] tensor, as one
+// projection writes it (rows 3 H heads apart), and O may be asked for in
+// binary16; on compiled lists only, whose references are tripled.  It takes
+// the three copies and the cast around a layer's pass away: 500,000 nodes, 2
+// heads, layer 984 -> 742 us (copies 166 us, cast 57 us; the pass itself 491
+// -> 475 us, half the bytes of O).
+template <int MODE, int WPG, bool WIDE, int TEAM, bool PACKED>
 __global__ void __launch_bounds__(kWave * WPG) __attribute__((amdgpu_waves_per_eu(4)))
 fused_attention_kernel(const AttnParams p)
 {
     static_assert(TEAM == 1 || TEAM == WPG, "a team fills its workgroup");
+    static_assert(!PACKED || (MODE == kModeList && !WIDE), "packed tensors: compiled lists");
     const int H = p.H;
     __shared__ WaveLds lds_all[WPG];
     const int wave = threadIdx.x / kWave;
@@ -226,7 +238,7 @@ fused_attention_kernel(const AttnParams p)
     const __amdgpu_buffer_rsrc_t kres = make_rsrc(p.K, p.feat_bytes);
     const __amdgpu_buffer_rsrc_t vres = make_rsrc(p.V, p.feat_bytes);
     const uint32_t head_off = (uint32_t)h * kRowBytes;
-    const uint32_t row_stride = H * kRowBytes;
+    const uint32_t row_stride = (PACKED ? 3 : 1) * H * kRowBytes;
     const uint32_t ref_stride = WIDE ? 1u : row_stride;   // node -> row reference
     const uint32_t no_ref = WIDE ? kNoIdx : kNoRow;
 
@@ -268,7 +280,8 @@ fused_attention_kernel(const AttnParams p)
                 h8 krow[4], vrow[4];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    const uint32_t ref = m[(lane >> 3) + 8 * i];
+                    uint32_t ref = m[(lane >> 3) + 8 * i];
+                    if constexpr (PACKED) ref *= 3;   // kNoRow stays past the tensor: kNoRow3
                     krow[i] = load_ref<WIDE>(kres, p.K, ref, row_stride, piece_off);
                     vrow[i] = load_ref<WIDE>(vres, p.V, ref, row_stride, piece_off);
                 }
@@ -496,6 +509,31 @@ fused_attention_kernel(const AttnParams p)
         // instruction writes four complete 256-byte rows instead of 16-byte
         // pieces of all sixteen.
         F3S_WAVE_LDS_SYNC();   // this wave's last reads of its stage are done
+        if constexpr (PACKED) {
+            if (p.out_half) {
+                // binary16 rows of 128 bytes, rounded once: two stores of
+                // eight whole rows each
+                _Float16* hst = L.stage;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const f4 x = {st.acc[0][v] * inv, st.acc[1][v] * inv, st.acc[2][v] * inv,
+                                  st.acc[3][v] * inv};
+                    *reinterpret_cast<h4*>(&hst[r * kStageRow + 16 * g + 4 * v]) =
+                        __builtin_convertvector(x, h4);
+                }
+                F3S_WAVE_LDS_SYNC();
+#pragma unroll
+                for (int v = 0; v < 2; ++v) {
+                    const int rr = 8 * v + (lane >> 3);
+                    const h8 x = *reinterpret_cast<const h8*>(&hst[rr * kStageRow + 8 * (lane & 7)]);
+                    const int32_t row = w * 16 + rr;
+                    if (row < n)
+                        *reinterpret_cast<h8*>(reinterpret_cast<_Float16*>(p.O) +
+                                               ((int64_t)row * H + h) * kD + 8 * (lane & 7)) = x;
+                }
+                return;
+            }
+        }
         float* ost = reinterpret_cast<float*>(L.stage);
 #pragma unroll
         for (int v = 0; v < 4; ++v)
@@ -545,7 +583,7 @@ fused_attention_kernel(const AttnParams p)
         if (last) atomicExch(cnt, 0);
     }
     if (!__shfl(last, 0, kWave)) return;
-    merge_split<2>(p, si, h, lane);
+    merge_split<2, PACKED>(p, si, h, lane);
 }
 
 __global__ void warm_attention_kernel() {}
@@ -1159,19 +1197,21 @@ static f3s_status check_attention_args(const void* Q, const void* K, const void*
     return F3S_OK;
 }
 
-template <int MODE, bool WIDE>
+template <int MODE, bool WIDE, bool PACKED>
 static void launch_mw(const AttnParams& p, int64_t waves, hipStream_t st)
 {
     if constexpr (!WIDE) {
         // teams (small graphs; never wide): one workgroup per (window, head)
-        if (p.team == kTeamLarge) {
-            hipLaunchKernelGGL((fused_attention_kernel<MODE, kTeamLarge, false, kTeamLarge>),
-                               dim3((unsigned)(waves / kTeamLarge)), dim3(kTeamLarge * kWave), 0,
-                               st, p);
-            return;
+        if constexpr (!PACKED) {   // (compiled lists have teams of kTeamSmall only)
+            if (p.team == kTeamLarge) {
+                hipLaunchKernelGGL((fused_attention_kernel<MODE, kTeamLarge, false, kTeamLarge, false>),
+                                   dim3((unsigned)(waves / kTeamLarge)), dim3(kTeamLarge * kWave),
+                                   0, st, p);
+                return;
+            }
         }
         if (p.team == kTeamSmall) {
-            hipLaunchKernelGGL((fused_attention_kernel<MODE, kTeamSmall, false, kTeamSmall>),
+            hipLaunchKernelGGL((fused_attention_kernel<MODE, kTeamSmall, false, kTeamSmall, PACKED>),
                                dim3((unsigned)(waves / kTeamSmall)), dim3(kTeamSmall * kWave), 0,
                                st, p);
             return;
@@ -1179,10 +1219,10 @@ static void launch_mw(const AttnParams& p, int64_t waves, hipStream_t st)
     }
     // Small launches use one-wave workgroups so they spread over all CUs.
     if (waves < 4 * 256 * 2) {
-        hipLaunchKernelGGL((fused_attention_kernel<MODE, 1, WIDE, 1>), dim3((unsigned)waves),
-                           dim3(kWave), 0, st, p);
+        hipLaunchKernelGGL((fused_attention_kernel<MODE, 1, WIDE, 1, PACKED>),
+                           dim3((unsigned)waves), dim3(kWave), 0, st, p);
     } else {
-        hipLaunchKernelGGL((fused_attention_kernel<MODE, 4, WIDE, 1>),
+        hipLaunchKernelGGL((fused_attention_kernel<MODE, 4, WIDE, 1, PACKED>),
                            dim3((unsigned)ceil_div(waves, 4)), dim3(4 * kWave), 0, st, p);
     }
 }
@@ -1191,9 +1231,9 @@ template <int MODE>
 static void launch_m(const AttnParams& p, int64_t waves, hipStream_t st)
 {
     if (wide_features(p.n, p.H))
-        launch_mw<MODE, true>(p, waves, st);
+        launch_mw<MODE, true, false>(p, waves, st);
     else
-        launch_mw<MODE, false>(p, waves, st);
+        launch_mw<MODE, false, false>(p, waves, st);
 }
 
 static f3s_status launch(AttnParams p, int32_t H, float scale, hipStream_t st)
@@ -1205,7 +1245,8 @@ static f3s_status launch(AttnParams p, int32_t H, float scale, hipStream_t st)
     p.H = H;
     // narrow launches range-check buffer loads against the tensor size;
     // wide ones never use the buffer descriptors
-    p.feat_bytes = wide_features(p.n, H) ? 0u : (uint32_t)((int64_t)p.n * H * kRowBytes);
+    if (!p.packed)
+        p.feat_bytes = wide_features(p.n, H) ? 0u : (uint32_t)((int64_t)p.n * H * kRowBytes);
     if (p.team > 1) {
         F3S_REQUIRE((p.team == kTeamSmall || p.team == kTeamLarge) && p.num_items % p.team == 0 &&
                         p.num_split == 0 && !wide_features(p.n, H),
@@ -1213,7 +1254,9 @@ static f3s_status launch(AttnParams p, int32_t H, float scale, hipStream_t st)
     }
     F3S_REQUIRE(p.num_split == 0 || (p.items && p.splits && p.slot_split && p.counters && p.partials),
                 "attention: split windows need the plan's merge state");
-    if (!p.tile_mask)
+    if (p.packed)
+        launch_mw<kModeList, false, true>(p, waves, st);
+    else if (!p.tile_mask)
         launch_m<kModeDense>(p, waves, st);
     else if (p.chunk_base)
         launch_m<kModeList>(p, waves, st);
@@ -1221,6 +1264,26 @@ static f3s_status launch(AttnParams p, int32_t H, float scale, hipStream_t st)
         launch_m<kModeRing>(p, waves, st);
     F3S_HIP(hipGetLastError());
     return F3S_OK;
+}
+
+// A planned pass's launch: the plan's items (tile-dense passes run the finer
+// set when the plan has one) and merge state.
+static AttnParams plan_params(const f3s_plan* plan, bool masked, int32_t n)
+{
+    AttnParams p{};
+    const f3s_item_set& set = (!masked && plan->has_dense) ? plan->dense : plan->masked;
+    p.items = reinterpret_cast<const Item*>(set.items.ptr);
+    p.num_items = set.num_items;
+    p.W = plan->W;
+    p.n = n;
+    p.xcd_contiguous = plan->xcd_contiguous;
+    p.partials = reinterpret_cast<float*>(plan->partials.ptr);
+    p.splits = reinterpret_cast<const SplitInfo*>(set.splits.ptr);
+    p.slot_split = reinterpret_cast<const int32_t*>(set.slot_split.ptr);
+    p.counters = reinterpret_cast<int32_t*>(plan->counters.ptr);
+    p.num_split = set.num_split;
+    p.team = set.team;
+    return p;
 }
 
 // f3s_attention_fwd; the scheduled launch takes its scratch from
@@ -1585,31 +1648,49 @@ f3s_status f3s_attention_fwd_planned(const f3s_plan* plan, const uint16_t* Q, co
                 "f3s_attention_fwd_planned: tile_mask alignment");
     F3S_TRY(require_device());
     clear_error();
-    AttnParams p{};
+    AttnParams p = plan_params(plan, d_tile_mask != nullptr, n);
     p.Q = reinterpret_cast<const _Float16*>(Q);
     p.K = reinterpret_cast<const _Float16*>(K);
     p.V = reinterpret_cast<const _Float16*>(V);
     p.O = O;
     p.block_col = d_block_col;
     p.tile_mask = d_tile_mask;
-    // tile-dense passes run the finer item set when the plan has one
-    const f3s_item_set& set = (!d_tile_mask && plan->has_dense) ? plan->dense : plan->masked;
-    p.items = reinterpret_cast<const Item*>(set.items.ptr);
-    p.num_items = set.num_items;
-    p.W = plan->W;
-    p.n = n;
-    p.xcd_contiguous = plan->xcd_contiguous;
-    p.partials = reinterpret_cast<float*>(plan->partials.ptr);
-    p.splits = reinterpret_cast<const SplitInfo*>(set.splits.ptr);
-    p.slot_split = reinterpret_cast<const int32_t*>(set.slot_split.ptr);
-    p.counters = reinterpret_cast<int32_t*>(plan->counters.ptr);
-    p.num_split = set.num_split;
-    p.team = set.team;
     if (d_tile_mask && d_tile_mask == plan->compiled_tile_mask &&
         d_block_col == plan->compiled_block_col && n == plan->compiled_n) {
         p.chunk_base = reinterpret_cast<const int32_t*>(plan->chunk_base.ptr);
         p.columns = reinterpret_cast<const uint32_t*>(plan->columns.ptr);
     }
+    return launch(p, H, scale, as_stream(stream));
+}
+
+f3s_status f3s_attention_fwd_packed(const f3s_plan* plan, const uint16_t* QKV, void* O,
+                                    int32_t out_half, int32_t n, int32_t d, int32_t H, float scale,
+                                    void* stream)
+{
+    F3S_REQUIRE(plan != nullptr, "f3s_attention_fwd_packed: NULL plan");
+    F3S_TRY(check_attention_args(QKV, QKV, QKV, O, n, d, H));
+    F3S_REQUIRE(H == plan->H, "f3s_attention_fwd_packed: H differs from the plan's");
+    F3S_REQUIRE(plan->compiled_n >= 0, "f3s_attention_fwd_packed: the plan is not compiled");
+    F3S_REQUIRE(n == plan->compiled_n, "f3s_attention_fwd_packed: n differs from the compiled lists'");
+    const int64_t bytes = 3 * (int64_t)n * H * kRowBytes;
+    if (bytes > (int64_t)kNoRow3) {
+        set_error("f3s_attention_fwd_packed: tensors of n * H * 384 bytes past 4 GiB");
+        return F3S_EUNSUPPORTED;
+    }
+    F3S_TRY(require_device());
+    clear_error();
+    AttnParams p = plan_params(plan, true, n);
+    const uint32_t third = (uint32_t)H * kD;
+    p.Q = reinterpret_cast<const _Float16*>(QKV);
+    p.K = p.Q + third;
+    p.V = p.K + third;
+    p.O = static_cast<float*>(O);
+    p.packed = 1;
+    p.out_half = out_half != 0;
+    // (one size for the three descriptors: the last rows of V end it)
+    p.feat_bytes = n > 0 ? (uint32_t)(bytes - 2 * (int64_t)H * kRowBytes) : 0u;
+    p.chunk_base = reinterpret_cast<const int32_t*>(plan->chunk_base.ptr);
+    p.columns = reinterpret_cast<const uint32_t*>(plan->columns.ptr);
     return launch(p, H, scale, as_stream(stream));
 }
 

@@ -88,6 +88,8 @@ struct AttnParams {
     const int32_t* slot_split;       // planned launch: the split window of each partial slot
     int32_t* counters;               // planned launch: segments arrived per (split window,
                                      // head); zero between passes
+    int32_t packed;                  // Q, K, V are thirds of one [n][3][H][64] tensor
+    int32_t out_half;                // (packed) O in binary16
 };
 
 // A window is heavy for the unplanned launch's teams when its tiles exceed
@@ -233,6 +235,10 @@ __device__ __forceinline__ int slot_of(int g, int j) { return (j < 4) ? 4 * g + 
 // under 8,256 bytes at 64 heads) cannot wrap past 2^32, and the feature
 // tensors are required to end at or below it.
 constexpr uint32_t kNoRow = 0xffffc000u;
+// What a packed launch makes of it (references tripled, modulo 2^32): past a
+// packed tensor of at most that many bytes, offsets added as above.
+constexpr uint32_t kNoRow3 = kNoRow * 3u;
+static_assert(kNoRow3 == 0xffff4000u, "still near the top");
 // Wide launches (feature tensors beyond kNoRow bytes) address rows by node
 // index with 64-bit loads; kNoIdx marks a slot with no row.
 constexpr uint32_t kNoIdx = 0xffffffffu;

@@ -129,6 +129,34 @@ class TorchGraph:
         return out
 
 
+    def takes_packed(self) -> bool:
+        """Whether attention_packed takes this graph: masked semantics, and
+        the packed tensor within the 32-bit offsets of its launch."""
+        return self.masked and 3 * self.n * self.heads * 2 * HEAD_DIM <= 0xffff4000
+
+    def attention_packed(self, qkv: torch.Tensor, scale: float = 1.0,
+                         dtype: torch.dtype = torch.float32) -> torch.Tensor:
+        """attention() on the [n, 3 * H * 64] fp16 output of one projection
+        (q, k and v side by side in each row, no copies made), O [n, H, 64]
+        in float32 or float16 (f3s_attention_fwd_packed)."""
+        if qkv.requires_grad:
+            raise RuntimeError("the fused pass is forward-only (no autograd)")
+        if qkv.dtype != torch.float16 or not qkv.is_cuda or not qkv.is_contiguous():
+            raise ValueError("qkv must be a contiguous float16 CUDA tensor")
+        if tuple(qkv.shape) != (self.n, 3 * self.heads * HEAD_DIM):
+            raise ValueError(f"qkv must have shape {(self.n, 3 * self.heads * HEAD_DIM)}, "
+                             f"got {tuple(qkv.shape)}")
+        if dtype not in (torch.float32, torch.float16):
+            raise ValueError("dtype must be float32 or float16")
+        out = torch.empty((self.n, self.heads, HEAD_DIM), dtype=dtype, device=qkv.device)
+        if self.n:
+            check(_lib.hip().f3s_attention_fwd_packed(
+                self.plan.handle, qkv.data_ptr(), out.data_ptr(), int(dtype == torch.float16),
+                self.n, HEAD_DIM, self.heads, float(scale),
+                torch.cuda.current_stream().cuda_stream), "f3s_attention_fwd_packed")
+        return out
+
+
 class GraphTransformerLayer(torch.nn.Module):
     """x -> [Q K V] = x W_qkv -> fused edge attention per head -> concat ->
     W_o, forward only.  Compute dtype of the projections is the module's
@@ -148,10 +176,18 @@ class GraphTransformerLayer(torch.nn.Module):
         if graph.heads != self.heads:
             raise ValueError("graph was planned for a different head count")
         n = x.shape[0]
-        qkv = self.qkv(x).to(torch.float16).view(n, 3, self.heads, HEAD_DIM)
-        q, k, v = (qkv[:, i].contiguous() for i in range(3))
-        o = graph.attention(q, k, v, scale=self.scale)
-        return self.proj(o.view(n, self.heads * HEAD_DIM).to(self.proj.weight.dtype))
+        qkv = self.qkv(x).to(torch.float16)
+        dtype = self.proj.weight.dtype
+        if graph.takes_packed() and qkv.dim() == 2 and qkv.is_contiguous():
+            # the pass reads q, k and v where the projection wrote them, and
+            # writes O in the dtype the output projection takes
+            o = graph.attention_packed(qkv, self.scale,
+                                       dtype if dtype == torch.float16 else torch.float32)
+        else:
+            qkv = qkv.view(n, 3, self.heads, HEAD_DIM)
+            q, k, v = (qkv[:, i].contiguous() for i in range(3))
+            o = graph.attention(q, k, v, scale=self.scale)
+        return self.proj(o.view(n, self.heads * HEAD_DIM).to(dtype))
 
 
 # ------------------------------------------------------------------ operator

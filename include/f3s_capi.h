@@ -257,6 +257,18 @@ f3s_status f3s_attention_fwd_planned(const f3s_plan* plan, const uint16_t* Q,
                                      int32_t n, int32_t d, int32_t H, float scale,
                                      void* stream);
 
+/* The masked pass of a compiled plan on one packed tensor QKV [n][3][H][64]
+ * (what a single projection of the node features writes: Q, K and V are its
+ * thirds) with O [n][H][64] in float32 or, with out_half, in binary16 (the
+ * float32 result rounded once, to nearest even).  No reference counterpart:
+ * a layer needs no copies of Q, K and V and no cast of O around the pass.
+ * Same results, bit for bit, as f3s_attention_fwd_planned on the copies.
+ * F3S_EINVAL unless the plan was compiled for this n; F3S_EUNSUPPORTED past
+ * n * H * 384 bytes = 4 GiB less 48 KiB. */
+f3s_status f3s_attention_fwd_packed(const f3s_plan* plan, const uint16_t* QKV, void* O,
+                                    int32_t out_half, int32_t n, int32_t d, int32_t H,
+                                    float scale, void* stream);
+
 /* Measurement only (no reference counterpart): the device's random-gather
  * ceiling for the fused pass's access pattern.  For each of `count` columns
  * (a multiple of 32) it loads the 128-byte row at byte offset

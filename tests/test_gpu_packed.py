@@ -1,0 +1,60 @@
+"""f3s_attention_fwd_packed: the compiled plan's pass on one [n][3][H][64]
+tensor gives the bits of the planned pass on copies of its thirds (float32),
+and those rounded once (binary16), for every launch shape of a masked plan:
+teams, one-wave workgroups, four-wave workgroups and split windows."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch  # noqa: F401  (torch's HIP runtime first)
+
+from conftest import random_csr, rng
+
+pytestmark = pytest.mark.gpu
+
+
+def star_csr(n: int, hubs: int, seed: int):
+    r = rng(seed)
+    rows = np.concatenate([np.repeat(np.arange(hubs), n // 2), np.arange(n)])
+    cols = np.concatenate([r.integers(0, n, hubs * (n // 2)), np.arange(n)])
+    keys = np.unique(rows.astype(np.int64) * n + cols)
+    rp = np.searchsorted(keys // n, np.arange(n + 1)).astype(np.int32)
+    return rp, (keys % n).astype(np.int32)
+
+
+@pytest.mark.parametrize("graph,n,H", [
+    ("random", 1, 1), ("random", 45, 3), ("random", 3000, 1),   # teams
+    ("random", 17_001, 1), ("random", 20_000, 5),               # one- and four-wave workgroups
+    ("star", 30_000, 2),                                        # split windows
+    ("random", 700, 64),                                        # the most heads
+])
+def test_packed_is_planned(gpu, graph, n, H):
+    from fused3s_amd import torch_ops
+    rp, ci = random_csr(n, 9, n + H) if graph == "random" else star_csr(n, 3, n)
+    g = torch_ops.TorchGraph(rp, ci, heads=H)
+    if graph == "star":
+        assert g.plan.num_split > 0
+    gen = torch.Generator().manual_seed(n)
+    qkv = torch.randn(n, 3 * H * 64, generator=gen).half().cuda()
+    q, k, v = (t.contiguous() for t in qkv.view(n, 3, H, 64).unbind(1))
+    want = g.attention(q, k, v, scale=0.125)
+    assert torch.equal(g.attention_packed(qkv, 0.125), want)
+    half = g.attention_packed(qkv, 0.125, torch.float16)
+    assert half.dtype == torch.float16 and torch.equal(half, want.half())
+
+
+def test_packed_rejects(gpu):
+    from fused3s_amd import torch_ops
+    rp, ci = random_csr(64, 3, 5)
+    g = torch_ops.TorchGraph(rp, ci, heads=1)
+    qkv = torch.zeros(64, 192, dtype=torch.float16, device="cuda")
+    for bad in (qkv[:, :128], qkv.float(), qkv.cpu(), qkv[:63]):
+        with pytest.raises(ValueError):
+            g.attention_packed(bad)
+    with pytest.raises(ValueError):
+        g.attention_packed(qkv, dtype=torch.bfloat16)
+    dense = torch_ops.TorchGraph(rp, ci, heads=1, masked=False)
+    assert not dense.takes_packed()
+    with pytest.raises(gpu.F3SError) as e:   # the plan holds no lists
+        dense.attention_packed(qkv)
+    assert e.value.name == "F3S_EINVAL"
