@@ -911,101 +911,177 @@ __host__ __device__ __forceinline__ void auto_segments(int64_t T, int32_t W, int
 
 // Work items per position of the plan's sequence (P positions; window
 // order[L], or L; invalid entries hold no window) for one or two item sets:
-// counts[3 k + 0] items, [3 k + 1] partial slots, [3 k + 2] split windows of
-// set k, each [P].  seg_fixed > 0 is the one set's segment size; 0 takes the
-// automatic sizes from T = offs[W] (thread 0 also reports T and the sizes in
-// info).
-__global__ void plan_count(const int32_t* __restrict__ offs, const int32_t* __restrict__ order,
-                           int32_t W, int32_t P, int32_t H, int32_t seg_fixed, int32_t nsets,
-                           int32_t team0, int32_t team1, int32_t* __restrict__ counts,
-                           int64_t* __restrict__ info)
+// [3 k + 0] items, [3 k + 1] partial slots, [3 k + 2] split windows of set k.
+// seg_fixed > 0 is the one set's segment size; 0 takes the automatic sizes
+// from T = offs[W].
+struct PlanSeq {
+    const int32_t* offs;
+    const int32_t* order;
+    int32_t W, P, H, seg_fixed, nsets, team[2];
+};
+constexpr int kPlanArrays = 6;
+
+__device__ __forceinline__ int32_t plan_segments(const PlanSeq& q, int64_t seg[2])
 {
-    const int32_t L = blockIdx.x * blockDim.x + threadIdx.x;
-    const int32_t T = W > 0 ? max(0, offs[W]) : 0;
-    int64_t seg[2];
-    if (seg_fixed > 0) {
-        seg[0] = seg[1] = seg_fixed;
-    } else {
-        auto_segments(T, W, H, seg);
+    const int32_t T = q.W > 0 ? max(0, q.offs[q.W]) : 0;
+    if (q.seg_fixed > 0)
+        seg[0] = seg[1] = q.seg_fixed;
+    else
+        auto_segments(T, q.W, q.H, seg);
+    return T;
+}
+
+__device__ __forceinline__ void plan_counts(const PlanSeq& q, int32_t T, const int64_t seg[2],
+                                            int64_t L, int32_t (&c)[kPlanArrays])
+{
+#pragma unroll
+    for (int j = 0; j < kPlanArrays; ++j) c[j] = 0;
+    if (L >= q.P) return;
+    const int32_t w = q.order ? q.order[L] : (int32_t)L;
+    int32_t nt = 0;
+    if (w >= 0 && w < q.W) {
+        const int32_t tb = max(0, min(q.offs[w], T)), te = max(tb, min(q.offs[w + 1], T));
+        nt = te - tb;
     }
-    if (L == 0) {
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        if (k >= q.nsets) break;
+        int32_t ns = 1;
+        if (q.team[k] > 1) {
+            ns = q.team[k];   // a team's items, merged in LDS: no partials
+        } else if (nt > seg[k]) {
+            ns = (int32_t)((nt + seg[k] - 1) / seg[k]);
+        }
+        const bool split = q.team[k] == 1 && ns > 1;
+        c[3 * k + 0] = ns;
+        c[3 * k + 1] = split ? ns : 0;
+        c[3 * k + 2] = split ? 1 : 0;
+    }
+}
+
+// The six counts and their scans in two launches (one for a single block of
+// positions), every array at once, counted where they are scanned: block
+// sums, then each block adds up the sums before its own and scans its
+// positions into bases[j][P + 1].  The last block reports to the host: info
+// [0] T, [1..2] segment sizes, [3 + j] total of array j.  (One count launch,
+// three per scanned array and one for the totals before: a plan of 1,251
+// windows took 104 us from call to completion with 24 launches, 44 us now.)
+constexpr int kPlanThreads = 256;
+constexpr int kPlanPer = 4;
+constexpr int kPlanTile = kPlanThreads * kPlanPer;
+
+__global__ void __launch_bounds__(kPlanThreads)
+plan_sums(const PlanSeq q, int64_t* __restrict__ sums)
+{
+    __shared__ int64_t lds[kPlanThreads / kWave];
+    int64_t seg[2];
+    const int32_t T = plan_segments(q, seg);
+    int64_t s[kPlanArrays] = {};
+    const int64_t base = (int64_t)blockIdx.x * kPlanTile + threadIdx.x;
+#pragma unroll
+    for (int i = 0; i < kPlanPer; ++i) {
+        int32_t c[kPlanArrays];
+        plan_counts(q, T, seg, base + i * kPlanThreads, c);
+#pragma unroll
+        for (int j = 0; j < kPlanArrays; ++j) s[j] += c[j];
+    }
+#pragma unroll
+    for (int j = 0; j < kPlanArrays; ++j) {
+        int64_t total;
+        (void)block_exclusive_scan<kPlanThreads>(s[j], lds, total);
+        if (threadIdx.x == 0) sums[(int64_t)j * gridDim.x + blockIdx.x] = total;
+    }
+}
+
+__global__ void __launch_bounds__(kPlanThreads)
+plan_bases(const PlanSeq q, const int64_t* __restrict__ sums, int64_t* __restrict__ bases,
+           int64_t* __restrict__ info)
+{
+    __shared__ int64_t lds[kPlanThreads / kWave];
+    int64_t seg[2];
+    const int32_t T = plan_segments(q, seg);
+    const int64_t base = (int64_t)blockIdx.x * kPlanTile + (int64_t)threadIdx.x * kPlanPer;
+    int32_t c[kPlanPer][kPlanArrays];
+#pragma unroll
+    for (int i = 0; i < kPlanPer; ++i) plan_counts(q, T, seg, base + i, c[i]);
+    const bool last = blockIdx.x == gridDim.x - 1;
+#pragma unroll
+    for (int j = 0; j < kPlanArrays; ++j) {
+        if (j >= 3 * q.nsets) break;
+        int64_t part = 0, before = 0, own = 0, total;
+        if (blockIdx.x > 0) {   // uniform
+            for (int64_t b = threadIdx.x; b < (int64_t)blockIdx.x; b += kPlanThreads)
+                part += sums[(int64_t)j * gridDim.x + b];
+            (void)block_exclusive_scan<kPlanThreads>(part, lds, before);
+        }
+#pragma unroll
+        for (int i = 0; i < kPlanPer; ++i) own += c[i][j];
+        int64_t ex = block_exclusive_scan<kPlanThreads>(own, lds, total) + before;
+        int64_t* out = bases + (int64_t)j * ((int64_t)q.P + 1);
+#pragma unroll
+        for (int i = 0; i < kPlanPer; ++i) {
+            if (base + i < q.P) out[base + i] = ex;
+            ex += c[i][j];
+        }
+        if (last && threadIdx.x == 0) {
+            out[q.P] = before + total;
+            info[3 + j] = before + total;
+        }
+    }
+    if (last && threadIdx.x == 0) {
         info[0] = T;
         info[1] = seg[0];
         info[2] = seg[1];
     }
-    if (L >= P) return;
-    const int32_t w = order ? order[L] : L;
-    int32_t nt = 0;
-    if (w >= 0 && w < W) {
-        const int32_t tb = max(0, min(offs[w], T)), te = max(tb, min(offs[w + 1], T));
-        nt = te - tb;
-    }
-    for (int k = 0; k < nsets; ++k) {
-        const int32_t team = k == 0 ? team0 : team1;
-        int32_t ns = 1;
-        if (team > 1) {
-            ns = team;   // a team's items, merged in LDS: no partials
-        } else if (nt > seg[k]) {
-            ns = (int32_t)((nt + seg[k] - 1) / seg[k]);
-        }
-        const bool split = team == 1 && ns > 1;
-        counts[(3 * k + 0) * (int64_t)P + L] = ns;
-        counts[(3 * k + 1) * (int64_t)P + L] = split ? ns : 0;
-        counts[(3 * k + 2) * (int64_t)P + L] = split ? 1 : 0;
-    }
 }
 
-// info[3 + j] = total of scanned count array j (bases[j][P]).
-__global__ void plan_totals(const int64_t* __restrict__ bases, int32_t P, int32_t arrays,
-                            int64_t* __restrict__ info)
-{
-    const int j = threadIdx.x;
-    if (j < arrays) info[3 + j] = bases[(int64_t)j * ((int64_t)P + 1) + P];
-}
+// One item set's lists (blockIdx.y: which); the first set's threads also
+// clear the arrival counts.
+struct PlanSetOut {
+    const int64_t* bases;   // items, slots, splits: [P + 1] each
+    Item* items;
+    SplitInfo* splits;
+    int32_t* slot_split;
+    int32_t seg, team;
+};
 
-__global__ void plan_fill(const int32_t* __restrict__ offs, const int32_t* __restrict__ order,
-                          int32_t W, int32_t P, int32_t seg, int32_t team,
-                          const int64_t* __restrict__ item_base,
-                          const int64_t* __restrict__ slot_base,
-                          const int64_t* __restrict__ split_base, Item* __restrict__ items,
-                          SplitInfo* __restrict__ splits, int32_t* __restrict__ slot_split)
+__global__ void plan_fill(const PlanSeq q, const PlanSetOut set0, const PlanSetOut set1,
+                          int32_t* __restrict__ counters, int64_t ncounters)
 {
     const int32_t L = blockIdx.x * blockDim.x + threadIdx.x;
-    if (L >= P) return;
-    const int32_t w = order ? order[L] : L;
-    const int64_t ib = item_base[L];
-    const int32_t ns = (int32_t)(item_base[L + 1] - ib);
-    if (w < 0 || w >= W) {
+    if (blockIdx.y == 0)
+        for (int64_t i = L; i < ncounters; i += (int64_t)gridDim.x * blockDim.x) counters[i] = 0;
+    if (L >= q.P) return;
+    const PlanSetOut& s = blockIdx.y == 0 ? set0 : set1;
+    const int32_t w = q.order ? q.order[L] : L;
+    const int64_t ib = s.bases[L];
+    const int32_t ns = (int32_t)(s.bases[L + 1] - ib);
+    if (w < 0 || w >= q.W) {
         for (int32_t k = 0; k < ns; ++k)
-            items[ib + k] = Item{-1, 0, 0, -1};   // no window: the pass skips these
+            s.items[ib + k] = Item{-1, 0, 0, -1};   // no window: the pass skips these
         return;
     }
-    const int32_t T = offs[W];
-    const int32_t tb = max(0, min(offs[w], T)), te = max(tb, min(offs[w + 1], T));
-    if (team > 1) {
-        for (int32_t k = 0; k < team; ++k)
-            items[ib + k] = Item{w, team_part(tb, te, k, team), team_part(tb, te, k + 1, team), -1};
+    const int32_t T = q.offs[q.W];
+    const int32_t tb = max(0, min(q.offs[w], T)), te = max(tb, min(q.offs[w + 1], T));
+    if (s.team > 1) {
+        for (int32_t k = 0; k < s.team; ++k)
+            s.items[ib + k] =
+                Item{w, team_part(tb, te, k, s.team), team_part(tb, te, k + 1, s.team), -1};
         return;
     }
     if (ns == 1) {
-        items[ib] = Item{w, tb, te, -1};
+        s.items[ib] = Item{w, tb, te, -1};
         return;
     }
-    const int32_t sb = (int32_t)slot_base[L];
-    const int64_t sid = split_base[L];
-    splits[sid] = SplitInfo{w, sb, ns, 0};
+    const int64_t stride = (int64_t)q.P + 1;
+    const int32_t sb = (int32_t)s.bases[stride + L];
+    const int64_t sid = s.bases[2 * stride + L];
+    s.splits[sid] = SplitInfo{w, sb, ns, 0};
     for (int32_t k = 0; k < ns; ++k) {
-        const int32_t a = tb + k * seg;
-        items[ib + k] = Item{w, a, min(te, a + seg), sb + k};
-        slot_split[sb + k] = (int32_t)sid;
+        const int32_t a = tb + k * s.seg;
+        s.items[ib + k] = Item{w, a, min(te, a + s.seg), sb + k};
+        s.slot_split[sb + k] = (int32_t)sid;
     }
-}
-
-__global__ void offsets_to_i32_plan(const int64_t* __restrict__ in, int32_t* __restrict__ out,
-                                    int64_t count)
-{
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < count) out[i] = (int32_t)in[i];
 }
 
 // Attended columns of each planned item (masked semantics): one wave per
@@ -1017,7 +1093,7 @@ __global__ void __launch_bounds__(256)
 plan_columns(const Item* __restrict__ items, int64_t num_items,
              const int32_t* __restrict__ block_col, const uint16_t* __restrict__ tile_mask,
              int32_t n, uint32_t ref_stride, uint32_t no_ref, int32_t* __restrict__ nchunks,
-             const int64_t* __restrict__ chunk_base, uint32_t* __restrict__ columns)
+             const int32_t* __restrict__ chunk_base, uint32_t* __restrict__ columns)
 {
     const int64_t it = (int64_t)blockIdx.x * 4 + threadIdx.x / kWave;
     const int lane = threadIdx.x % kWave;
@@ -1025,7 +1101,7 @@ plan_columns(const Item* __restrict__ items, int64_t num_items,
     const Item item = items[it];
     const int32_t nbc = (n + 15) >> 4;
     int64_t pos = 0;   // wave-uniform
-    uint32_t* rec0 = FILL ? columns + chunk_base[it] * 64 : nullptr;
+    uint32_t* rec0 = FILL ? columns + (int64_t)chunk_base[it] * 64 : nullptr;
     for (int32_t t0 = item.tb; t0 < item.te; t0 += kWave) {
         const int32_t t = t0 + lane;
         uint32_t u = 0;
@@ -1115,28 +1191,25 @@ static f3s_status build_plan_sets(f3s_plan* p, const int32_t* d_window_offsets,
         P = (int32_t)(kXcds * sched_xcd_slots(W));
     }
     p->xcd_contiguous = !scheduled && d_window_order == nullptr;
-    const size_t cnt_bytes = sizeof(int32_t) * (size_t)arrays * (size_t)P;
-    const size_t base_bytes = sizeof(int64_t) * (size_t)arrays * ((size_t)P + 1);
-    const size_t tmp_bytes = sizeof(int64_t) * (size_t)scan_tmp_elems(P);
-    auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
+    const int64_t nb = P > 0 ? ceil_div(P, kPlanTile) : 1;
+    const size_t base_bytes = round256(sizeof(int64_t) * (size_t)arrays * ((size_t)P + 1));
     StreamBuffer buf(st);
-    F3S_TRY(buf.reserve(256 + al(cnt_bytes) + al(base_bytes) + al(tmp_bytes)));
-    char* q = static_cast<char*>(buf.ptr);
-    int64_t* info = reinterpret_cast<int64_t*>(q);           // [0] T, [1..2] segs, [3..] totals
-    int32_t* counts = reinterpret_cast<int32_t*>(q + 256);
-    int64_t* bases = reinterpret_cast<int64_t*>(q + 256 + al(cnt_bytes));
-    int64_t* tmp = reinterpret_cast<int64_t*>(q + 256 + al(cnt_bytes) + al(base_bytes));
-    hipLaunchKernelGGL(plan_count, dim3((unsigned)ceil_div(P > 0 ? P : 1, 256)), dim3(256), 0, st,
-                       d_window_offsets, seq, W, P, H, seg_tiles, nsets, team_m, team_d, counts,
+    F3S_TRY(buf.reserve(256 + base_bytes + sizeof(int64_t) * kPlanArrays * (size_t)nb));
+    char* mem = static_cast<char*>(buf.ptr);
+    int64_t* bases = reinterpret_cast<int64_t*>(mem + 256);
+    int64_t* sums = reinterpret_cast<int64_t*>(mem + 256 + base_bytes);
+    bool pinned = false;
+    int64_t* h = host_staging(&pinned);
+    // [0] T, [1..2] segment sizes, [3..] totals
+    int64_t* info = pinned ? h : reinterpret_cast<int64_t*>(mem);
+    const PlanSeq q{d_window_offsets, seq, W, P, H, seg_tiles, nsets, {team_m, team_d}};
+    if (nb > 1)
+        hipLaunchKernelGGL(plan_sums, dim3((unsigned)nb), dim3(kPlanThreads), 0, st, q, sums);
+    hipLaunchKernelGGL(plan_bases, dim3((unsigned)nb), dim3(kPlanThreads), 0, st, q, sums, bases,
                        info);
     F3S_HIP(hipGetLastError());
-    for (int j = 0; j < arrays; ++j)
-        F3S_TRY(exclusive_scan_i32_to_i64(counts + (size_t)j * P, bases + (size_t)j * (P + 1), P,
-                                          tmp, st));
-    hipLaunchKernelGGL(plan_totals, dim3(1), dim3(64), 0, st, bases, P, arrays, info);
-    F3S_HIP(hipGetLastError());
-    int64_t* h = host_staging();
-    F3S_HIP(hipMemcpyAsync(h, info, sizeof(int64_t) * (3 + arrays), hipMemcpyDeviceToHost, st));
+    if (!pinned)
+        F3S_HIP(hipMemcpyAsync(h, info, sizeof(int64_t) * (3 + arrays), hipMemcpyDeviceToHost, st));
     F3S_HIP(hipStreamSynchronize(st));
     p->T = h[0];
     const int32_t seg_m = (int32_t)h[1], seg_d = (int32_t)h[2];
@@ -1160,20 +1233,20 @@ static f3s_status build_plan_sets(f3s_plan* p, const int32_t* d_window_offsets,
                                 st));
     // the in-launch merge's arrival counts start at zero (each pass leaves
     // them so); both sets share them, as they share the partials
-    const size_t cnt_b = sizeof(int32_t) * (size_t)H * (size_t)(max_split + 1);
-    F3S_TRY(p->counters.reserve(cnt_b, st));
-    F3S_HIP(hipMemsetAsync(p->counters.ptr, 0, cnt_b, st));
-    for (int k = 0; k < nsets && P > 0; ++k) {
-        if (k == 1 && !p->has_dense) break;
+    const int64_t ncounters = (int64_t)H * (max_split + 1);
+    F3S_TRY(p->counters.reserve(sizeof(int32_t) * (size_t)ncounters, st));
+    PlanSetOut out[2] = {};
+    for (int k = 0; k < nsets; ++k) {
         f3s_item_set& set = k == 0 ? p->masked : p->dense;
-        const int64_t* bk = bases + (size_t)3 * k * (P + 1);
-        hipLaunchKernelGGL(plan_fill, dim3((unsigned)ceil_div(P, 256)), dim3(256), 0, st,
-                           d_window_offsets, seq, W, P, set.seg, set.team, bk, bk + (P + 1),
-                           bk + 2 * (size_t)(P + 1), reinterpret_cast<Item*>(set.items.ptr),
-                           reinterpret_cast<SplitInfo*>(set.splits.ptr),
-                           reinterpret_cast<int32_t*>(set.slot_split.ptr));
-        F3S_HIP(hipGetLastError());
+        out[k] = PlanSetOut{bases + (size_t)3 * k * (P + 1), reinterpret_cast<Item*>(set.items.ptr),
+                            reinterpret_cast<SplitInfo*>(set.splits.ptr),
+                            reinterpret_cast<int32_t*>(set.slot_split.ptr), set.seg, set.team};
     }
+    hipLaunchKernelGGL(plan_fill,
+                       dim3((unsigned)ceil_div(P > 0 ? P : 1, 256), p->has_dense ? 2u : 1u),
+                       dim3(256), 0, st, q, out[0], out[1],
+                       reinterpret_cast<int32_t*>(p->counters.ptr), ncounters);
+    F3S_HIP(hipGetLastError());
     // the plan is complete (and its memory usable on any stream) on return
     F3S_HIP(hipStreamSynchronize(st));
     return F3S_OK;
@@ -1503,14 +1576,14 @@ f3s_status f3s_plan_compile(f3s_plan* plan, const int32_t* d_block_col,
     plan->compiled_block_col = nullptr;
     plan->compiled_n = -1;
     const int64_t ni = plan->masked.num_items;
-    auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
-    const size_t cnt_bytes = al(sizeof(int32_t) * (size_t)(ni + 1));
-    const size_t base_bytes = al(sizeof(int64_t) * (size_t)(ni + 1));
+    const size_t cnt_bytes = round256(sizeof(int32_t) * (size_t)(ni + 1));
     StreamBuffer buf(st);
-    F3S_TRY(buf.reserve(cnt_bytes + base_bytes + sizeof(int64_t) * (size_t)scan_tmp_elems(ni)));
-    auto* counts = reinterpret_cast<int32_t*>(buf.ptr);
-    auto* b64 = reinterpret_cast<int64_t*>(static_cast<char*>(buf.ptr) + cnt_bytes);
-    auto* tmp = reinterpret_cast<int64_t*>(static_cast<char*>(buf.ptr) + cnt_bytes + base_bytes);
+    F3S_TRY(buf.reserve(256 + cnt_bytes + sizeof(int64_t) * (size_t)offsets_sum_elems(ni)));
+    char* mem = static_cast<char*>(buf.ptr);
+    auto* counts = reinterpret_cast<int32_t*>(mem + 256);
+    auto* sums = reinterpret_cast<int64_t*>(mem + 256 + cnt_bytes);
+    F3S_TRY(plan->chunk_base.reserve(sizeof(int32_t) * (size_t)(ni + 1), st));
+    auto* chunk_base = reinterpret_cast<int32_t*>(plan->chunk_base.ptr);
     // the records hold row references: byte offsets, or node indices when the
     // feature tensors are too large for 32-bit offsets (wide launches)
     const bool wide = wide_features(n, plan->H);
@@ -1522,27 +1595,26 @@ f3s_status f3s_plan_compile(f3s_plan* plan, const int32_t* d_block_col,
         hipLaunchKernelGGL(plan_columns<false>, grid, dim3(256), 0, st, items, ni, d_block_col,
                            d_tile_mask, n, ref_stride, no_ref, counts, nullptr, nullptr);
     F3S_HIP(hipGetLastError());
-    F3S_TRY(exclusive_scan_i32_to_i64(counts, b64, ni, tmp, st));
-    int64_t* h = host_staging();
-    F3S_HIP(hipMemcpyAsync(h, b64 + ni, sizeof(int64_t), hipMemcpyDeviceToHost, st));
+    bool pinned = false;
+    int64_t* h = host_staging(&pinned);
+    int64_t* status = pinned ? h : reinterpret_cast<int64_t*>(mem);
+    F3S_TRY(counts_to_offsets(counts, chunk_base, ni, sums, nullptr, status, st));
+    if (!pinned)
+        F3S_HIP(hipMemcpyAsync(h, status, 2 * sizeof(int64_t), hipMemcpyDeviceToHost, st));
     F3S_HIP(hipStreamSynchronize(st));
-    const int64_t total = h[0];
+    const int64_t total = h[1];
     if (total >= INT32_MAX) {
         set_error("f3s_plan_compile: more than 2^31-1 chunks");
         return F3S_EUNSUPPORTED;
     }
     // four records of padding: the pass reads records in blocks of four
     F3S_TRY(plan->columns.reserve(sizeof(uint32_t) * 64 * (size_t)(total + 4), st));
-    F3S_TRY(plan->chunk_base.reserve(sizeof(int32_t) * (size_t)(ni + 1), st));
     if (ni > 0) {
         hipLaunchKernelGGL(plan_columns<true>, grid, dim3(256), 0, st, items, ni, d_block_col,
-                           d_tile_mask, n, ref_stride, no_ref, nullptr, b64,
+                           d_tile_mask, n, ref_stride, no_ref, nullptr, chunk_base,
                            reinterpret_cast<uint32_t*>(plan->columns.ptr));
         F3S_HIP(hipGetLastError());
     }
-    hipLaunchKernelGGL(offsets_to_i32_plan, dim3((unsigned)ceil_div(ni + 1, 256)), dim3(256), 0,
-                       st, b64, reinterpret_cast<int32_t*>(plan->chunk_base.ptr), ni + 1);
-    F3S_HIP(hipGetLastError());
     // the lists are complete (and usable on any stream) on return
     F3S_HIP(hipStreamSynchronize(st));
     plan->num_chunks = total;

@@ -16,6 +16,45 @@ __global__ void window_counts(const int32_t* __restrict__ offs, int32_t W,
     iota[w] = w;
 }
 
+// The order of up to kRankMax windows in one launch: every workgroup loads all
+// windows' keys (tile count descending, then index: unique) into LDS and
+// places 64 windows at their ranks, four lanes per window each counting the
+// smaller keys in a quarter of the list.  O(W^2), about 5 us at kRankMax; the
+// radix sort's five launches cost more host time than that up to there (1,251
+// windows, call to completion: 38 us sorted, 25 us ranked), and past it the
+// square overtakes.
+constexpr int32_t kRankMax = 4096;
+constexpr uint32_t kRankTiles = (1u << 20) - 1;   // a count above (no valid form has one) ties
+static_assert(kRankMax <= 1 << 12, "the index takes 12 bits of the key, the count 20");
+
+__global__ void __launch_bounds__(256)
+rank_windows(const int32_t* __restrict__ offs, int32_t W, int32_t* __restrict__ order)
+{
+    __shared__ __align__(16) uint32_t key[kRankMax];
+    const int tid = threadIdx.x;
+    const int32_t quarter = (W + 15) / 16 * 4;   // keys a lane looks at, a multiple of 4
+    for (int32_t i = tid; i < 4 * quarter; i += 256) {
+        uint32_t k = 0xffffffffu;   // past the list: above every key
+        if (i < W) {
+            const int32_t c = offs[i + 1] - offs[i];
+            k = (kRankTiles - min((uint32_t)max(c, 0), kRankTiles)) << 12 | (uint32_t)i;
+        }
+        key[i] = k;
+    }
+    __syncthreads();
+    const int32_t i = blockIdx.x * 64 + tid / 4;
+    const uint32_t ki = key[min(i, W - 1)];
+    const uint4* mine = reinterpret_cast<const uint4*>(&key[(tid & 3) * quarter]);
+    int32_t rank = 0;
+    for (int32_t j = 0; j < quarter / 4; ++j) {
+        const uint4 k = mine[j];
+        rank += (k.x < ki) + (k.y < ki) + (k.z < ki) + (k.w < ki);
+    }
+    rank += __shfl_xor(rank, 1, kWave);
+    rank += __shfl_xor(rank, 2, kWave);
+    if (i < W && (tid & 3) == 0) order[rank] = i;
+}
+
 __global__ void __launch_bounds__(256)
 bsf_stats_kernel(const int32_t* __restrict__ block_col, const uint16_t* __restrict__ tile_mask,
                  int64_t T, int32_t n, unsigned long long* __restrict__ out)
@@ -79,6 +118,13 @@ f3s_status f3s_window_order(const int32_t* d_window_offsets, int32_t W, int32_t*
     F3S_TRY(require_device());
     clear_error();
     hipStream_t st = as_stream(stream);
+    if (W <= kRankMax) {
+        hipLaunchKernelGGL(rank_windows, dim3((unsigned)ceil_div(W, 64)), dim3(256), 0, st,
+                           d_window_offsets, W, d_order);
+        F3S_HIP(hipGetLastError());
+        F3S_HIP(hipStreamSynchronize(st));
+        return F3S_OK;
+    }
     StreamBuffer keys_in(st), keys_out(st), vals_in(st), tmp(st);
     F3S_TRY(keys_in.reserve(sizeof(uint32_t) * (size_t)W));
     F3S_TRY(keys_out.reserve(sizeof(uint32_t) * (size_t)W));

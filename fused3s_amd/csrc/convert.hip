@@ -1075,17 +1075,15 @@ offsets_apply(const int32_t* __restrict__ counts, int64_t W, const int64_t* __re
     }
     if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
         offsets[W] = (int32_t)(before + total);
-        status[0] = *err;
+        status[0] = err ? *err : 0;
         status[1] = before + total;
     }
 }
 
-// `sums` holds offsets_sum_elems(W) elements.
-static int64_t offsets_sum_elems(int64_t W) { return W > 0 ? ceil_div(W, kOffsTile) : 1; }
+int64_t offsets_sum_elems(int64_t W) { return W > 0 ? ceil_div(W, kOffsTile) : 1; }
 
-static f3s_status counts_to_offsets(const int32_t* counts, int32_t* offsets, int64_t W,
-                                    int64_t* sums, const int32_t* err, int64_t* status,
-                                    hipStream_t stream)
+f3s_status counts_to_offsets(const int32_t* counts, int32_t* offsets, int64_t W, int64_t* sums,
+                             const int32_t* err, int64_t* status, hipStream_t stream)
 {
     const int64_t nb = offsets_sum_elems(W);
     if (nb > 1)

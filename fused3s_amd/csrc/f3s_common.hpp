@@ -25,12 +25,14 @@ inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s);
 
 constexpr int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
-// Device-wide exclusive scan of int32 counts into int64 (or int32) prefix
-// sums; out has count + 1 entries (out[count] = total).  tmp needs
-// scan_tmp_elems(count) int64 elements.
-int64_t scan_tmp_elems(int64_t count);
-f3s_status exclusive_scan_i32_to_i64(const int32_t* in, int64_t* out, int64_t count,
-                                     int64_t* tmp, hipStream_t stream);
+// int32 counts[W] -> their exclusive prefix sums offsets[W + 1], in two
+// launches (one for few counts).  The total goes to status[1] too, in 64 bits
+// (offsets are meaningless past INT32_MAX), and *err, or 0, to status[0];
+// `status` may be pinned host memory.  `sums` holds offsets_sum_elems(W)
+// elements.
+int64_t offsets_sum_elems(int64_t W);
+f3s_status counts_to_offsets(const int32_t* counts, int32_t* offsets, int64_t W, int64_t* sums,
+                             const int32_t* err, int64_t* status, hipStream_t stream);
 
 // Each translation unit's code object is loaded onto the device at its
 // first kernel launch; these launch one empty kernel per unit (f3s_init).

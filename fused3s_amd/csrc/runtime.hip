@@ -1,5 +1,4 @@
-// runtime.hip -- error reporting, device plumbing, fp32->fp16 cast and the
-// device-wide scan used by the converter and the planner.
+// runtime.hip -- error reporting, device memory and plumbing, fp32->fp16 cast.
 #include <stdio.h>
 #include <stdlib.h>
 
@@ -314,86 +313,6 @@ f3s_status StreamBuffer::reserve(size_t want)
     F3S_HIP(hipGetDevice(&device));
     F3S_TRY(dev_alloc(&ptr, alloc, stream));
     bytes = alloc;
-    return F3S_OK;
-}
-
-// ------------------------------------------------------------------ scan
-
-constexpr int kScanThreads = 256;
-constexpr int kScanPerThread = 8;
-constexpr int kScanTile = kScanThreads * kScanPerThread;
-
-int64_t scan_tmp_elems(int64_t count) { return ceil_div(count, kScanTile) + 1; }
-
-__global__ void __launch_bounds__(kScanThreads)
-scan_block_sums(const int32_t* __restrict__ in, int64_t count, int64_t* __restrict__ sums)
-{
-    __shared__ int64_t lds[kScanThreads / kWave];
-    const int64_t base = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * kScanPerThread;
-    int64_t s = 0;
-#pragma unroll
-    for (int i = 0; i < kScanPerThread; ++i)
-        if (base + i < count) s += in[base + i];
-    int64_t total;
-    (void)block_exclusive_scan<kScanThreads>(s, lds, total);
-    if (threadIdx.x == 0) sums[blockIdx.x] = total;
-}
-
-// One workgroup: exclusive scan of the block sums in place; writes the grand
-// total to *total_out.
-__global__ void __launch_bounds__(kScanThreads)
-scan_sums_single(int64_t* __restrict__ sums, int64_t nblocks, int64_t* __restrict__ total_out)
-{
-    __shared__ int64_t lds[kScanThreads / kWave];
-    int64_t carry = 0;
-    for (int64_t b0 = 0; b0 < nblocks; b0 += kScanThreads) {
-        int64_t i = b0 + threadIdx.x;
-        int64_t v = i < nblocks ? sums[i] : 0;
-        int64_t total;
-        int64_t ex = block_exclusive_scan<kScanThreads>(v, lds, total);
-        if (i < nblocks) sums[i] = carry + ex;
-        carry += total;
-    }
-    if (threadIdx.x == 0) *total_out = carry;
-}
-
-__global__ void __launch_bounds__(kScanThreads)
-scan_apply(const int32_t* __restrict__ in, int64_t count, const int64_t* __restrict__ sums,
-           int64_t* __restrict__ out)
-{
-    __shared__ int64_t lds[kScanThreads / kWave];
-    const int64_t base = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * kScanPerThread;
-    int64_t v[kScanPerThread];
-    int64_t s = 0;
-#pragma unroll
-    for (int i = 0; i < kScanPerThread; ++i) {
-        v[i] = (base + i < count) ? in[base + i] : 0;
-        s += v[i];
-    }
-    int64_t total;
-    int64_t ex = block_exclusive_scan<kScanThreads>(s, lds, total) + sums[blockIdx.x];
-#pragma unroll
-    for (int i = 0; i < kScanPerThread; ++i) {
-        if (base + i < count) out[base + i] = ex;
-        ex += v[i];
-    }
-}
-
-f3s_status exclusive_scan_i32_to_i64(const int32_t* in, int64_t* out, int64_t count,
-                                     int64_t* tmp, hipStream_t stream)
-{
-    if (count <= 0) {
-        F3S_HIP(hipMemsetAsync(out, 0, sizeof(int64_t), stream));
-        return F3S_OK;
-    }
-    const int64_t nb = ceil_div(count, kScanTile);
-    hipLaunchKernelGGL(scan_block_sums, dim3((unsigned)nb), dim3(kScanThreads), 0, stream,
-                       in, count, tmp);
-    hipLaunchKernelGGL(scan_sums_single, dim3(1), dim3(kScanThreads), 0, stream, tmp, nb,
-                       out + count);
-    hipLaunchKernelGGL(scan_apply, dim3((unsigned)nb), dim3(kScanThreads), 0, stream, in,
-                       count, tmp, out);
-    F3S_HIP(hipGetLastError());
     return F3S_OK;
 }
 
