@@ -69,17 +69,27 @@ def current_stream() -> Stream:
     return _TorchStream(torch.cuda.current_stream().cuda_stream)
 
 
-class _TensorView(DeviceArray):
-    """A torch tensor's device memory passed to the C-ABI (not owned)."""
+def _on_device(t, s: Stream) -> DeviceArray:
+    """An int32 copy of an index array in library memory: from host memory, or
+    device to device when it is a tensor on the current device already."""
+    if torch.is_tensor(t):
+        if t.is_cuda and t.device.index == torch.cuda.current_device():
+            t = t.to(torch.int32).contiguous()
+            a = DeviceArray(tuple(t.shape), np.int32)
+            if a.nbytes:
+                check(_lib.hip().f3s_memcpy_d2d(a.ptr, t.data_ptr(), a.nbytes, s.handle),
+                      "f3s_memcpy_d2d")
+            return a
+        t = t.cpu().numpy()
+    return DeviceArray.from_numpy(np.ascontiguousarray(t, np.int32), s)
 
-    def __init__(self, t: torch.Tensor):   # noqa: D107 -- nothing is allocated
-        self._ptr = t.data_ptr()
-        self.shape = tuple(t.shape)
-        self.nbytes = t.numel() * t.element_size()
-        self._tensor = t
 
-    def free(self) -> None:
-        self._ptr = None   # the memory is torch's
+def _device_csr(row_ptr, col_idx, s: Stream) -> DeviceCSR:
+    csr = DeviceCSR.__new__(DeviceCSR)
+    csr.row_ptr, csr.col_idx = _on_device(row_ptr, s), _on_device(col_idx, s)
+    csr.n = csr.row_ptr.shape[0] - 1
+    csr.nnz = csr.col_idx.shape[0]
+    return csr
 
 
 class TorchGraph:
@@ -90,16 +100,12 @@ class TorchGraph:
     def __init__(self, row_ptr, col_idx, heads: int = 1, masked: bool = True):
         if not torch.cuda.is_available():
             raise RuntimeError("TorchGraph needs a ROCm device (no CPU fallback)")
-        rp = np.ascontiguousarray(row_ptr.cpu().numpy() if torch.is_tensor(row_ptr) else row_ptr,
-                                  np.int32)
-        ci = np.ascontiguousarray(col_idx.cpu().numpy() if torch.is_tensor(col_idx) else col_idx,
-                                  np.int32)
-        self.n = len(rp) - 1
-        self.nnz = len(ci)
+        s = current_stream()
+        self.csr = _device_csr(row_ptr, col_idx, s)
+        self.n = self.csr.n
+        self.nnz = self.csr.nnz
         self.heads = heads
         self.masked = masked
-        s = current_stream()
-        self.csr = DeviceCSR(rp, ci, s)
         self.bsf: DeviceBSF = convert_device(self.csr, masks=True, stream=s)
         self.order = window_order_device(self.bsf, s)
         self.plan = Plan(self.bsf, self.order, H=heads, stream=s)
@@ -111,21 +117,27 @@ class TorchGraph:
         """softmax over each node's neighbours of scale * q.k, weights applied
         to v; [n, H, 64] fp16 contiguous CUDA tensors in, [n, H, 64] fp32 out.
         masked=False gives the reference's tile-dense semantics instead."""
-        shape = (self.n, self.heads, HEAD_DIM)
+        n, H = self.n, self.heads
+        shape = (n, H, HEAD_DIM)
         for name, t in (("q", q), ("k", k), ("v", v)):
             if t.requires_grad:
                 raise RuntimeError("the fused pass is forward-only (no autograd)")
-            if t.dtype != torch.float16 or not t.is_cuda or not t.is_contiguous():
+            if t.dtype is not torch.float16 or not t.is_cuda or not t.is_contiguous():
                 raise ValueError(f"{name} must be a contiguous float16 CUDA tensor")
-            if tuple(t.shape) != shape and tuple(t.shape) != (self.n, self.heads * HEAD_DIM):
+            if t.shape != shape and t.shape != (n, H * HEAD_DIM):   # (a Size is a tuple)
                 raise ValueError(f"{name} must have shape {shape}, got {tuple(t.shape)}")
         if out is None:
             out = torch.empty(shape, dtype=torch.float32, device=q.device)
         elif (out.dtype != torch.float32 or not out.is_contiguous()
-              or out.numel() != self.n * self.heads * HEAD_DIM):
+              or out.numel() != n * H * HEAD_DIM):
             raise ValueError("out must be a contiguous float32 tensor of n * H * 64 elements")
-        self.plan.forward(_TensorView(q), _TensorView(k), _TensorView(v), _TensorView(out),
-                          masked=self.masked, d=HEAD_DIM, scale=scale, stream=current_stream())
+        # Plan.forward without its wrappers: a small graph's pass is shorter
+        # than the Python around it
+        bsf = self.bsf
+        check(_lib.hip().f3s_attention_fwd_planned(
+            self.plan.handle, q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
+            bsf.block_col.ptr, bsf.tile_mask.ptr if self.masked else None, n, HEAD_DIM, H, scale,
+            torch.cuda.current_stream().cuda_stream), "f3s_attention_fwd_planned")
         return out
 
 

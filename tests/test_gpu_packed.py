@@ -58,3 +58,24 @@ def test_packed_rejects(gpu):
     with pytest.raises(gpu.F3SError) as e:   # the plan holds no lists
         dense.attention_packed(qkv)
     assert e.value.name == "F3S_EINVAL"
+
+
+@pytest.mark.parametrize("dtype", ["int32", "int64"])
+def test_graph_from_device_tensors(gpu, dtype):
+    """A graph prepared from CUDA index tensors (copied device to device, on
+    a side stream too) is the one prepared from host arrays, and keeps its own
+    copy of them."""
+    from fused3s_amd import torch_ops
+    rp, ci = random_csr(1500, 7, 8)
+    want = torch_ops.TorchGraph(rp, ci, heads=2)
+    drp, dci = (torch.as_tensor(a).to(getattr(torch, dtype)).cuda() for a in (rp, ci))
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        got = torch_ops.TorchGraph(drp, dci, heads=2)
+        drp.zero_(), dci.zero_()
+    s.synchronize()
+    assert np.array_equal(got.csr.row_ptr.numpy(), rp) and np.array_equal(got.csr.col_idx.numpy(), ci)
+    assert (got.n, got.nnz) == (want.n, want.nnz)
+    q, k, v = torch.randn(3, 1500, 2, 64).half().cuda().unbind(0)
+    assert torch.equal(got.attention(q, k, v), want.attention(q, k, v))
