@@ -66,6 +66,7 @@ HIP_API = {
                                           c_i32, c_i32, c_i32, c_f32, c_vp]),
     "f3s_attention_fwd_packed": (c_i32, [c_vp, c_vp, c_vp, c_i32, c_i32, c_i32, c_i32, c_f32,
                                          c_vp]),
+    "f3s_linear_f16": (c_i32, [c_vp, c_vp, c_vp, c_vp, c_i64, c_i32, c_i32, c_vp]),
     "f3s_probe_gather": (c_i32, [c_vp, c_vp, c_i64, c_i32, c_vp, c_i64, c_i32, c_vp, c_vp]),
 }
 

@@ -755,14 +755,6 @@ constexpr int kStageTiles = 160;                  // tiles staged at once (256: 
 constexpr uint32_t kFillWork = 6 * kLightEdges, kCountWork = 4 * kLightEdges;
 static_assert(kStageTiles * 36 <= (int)kFillWork, "the stage fits over the words");
 
-// Orders this wave's LDS accesses between its lanes.  The LDS unit runs a
-// wave's operations in their order, so only the compiler has to be held.
-__device__ __forceinline__ void wave_lds_order()
-{
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
-    __builtin_amdgcn_wave_barrier();
-}
-
 __host__ __device__ inline uint32_t wave_lds_bytes(int32_t sums, bool fill)
 {
     return align16(8u * (uint32_t)sums) + 4 * kWave + (fill ? 4 * 32 + 4 * 16 + kFillWork : kCountWork);

@@ -22,6 +22,14 @@ __device__ __forceinline__ void lds_barrier()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// Orders this wave's LDS accesses between its lanes.  The LDS unit runs a
+// wave's operations in their order, so only the compiler has to be held.
+__device__ __forceinline__ void wave_lds_order()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // Inclusive scan over the 64 lanes of a wave.
 template <typename T>
 __device__ __forceinline__ T wave_inclusive_scan(T v)

@@ -374,6 +374,7 @@ f3s_status f3s_init(void)
     F3S_HIP(warm_attention(nullptr));
     F3S_HIP(warm_bsf_util(nullptr));
     F3S_HIP(warm_naive(nullptr));
+    F3S_HIP(warm_linear(nullptr));
     F3S_HIP(hipDeviceSynchronize());
     F3S_TRY(noalloc_setup());
     return F3S_OK;

@@ -169,6 +169,46 @@ class TorchGraph:
         return out
 
 
+def _is_plain_linear(m: torch.nn.Module) -> bool:
+    """A torch.nn.Linear whose call is its product and nothing else."""
+    hooks = torch.nn.modules.module
+    return (type(m) is torch.nn.Linear and "forward" not in m.__dict__
+            and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
+                     or m._backward_pre_hooks or hooks._global_forward_hooks
+                     or hooks._global_forward_pre_hooks or hooks._global_backward_hooks
+                     or hooks._global_backward_pre_hooks))
+
+
+def _project(m: torch.nn.Module, x: torch.Tensor) -> torch.Tensor:
+    """m(x), by f3s_linear_f16 where that is the same thing: a plain fp16
+    Linear of a contiguous fp16 matrix on its own device, in sizes the kernel
+    takes, outside autocast and tracing.  (Called without autograd.)  Below
+    64 K rows of more than 128 inputs and outputs the library's tiles are the
+    better ones (20,011 x 256 -> 768: 17 against 28 us; -> 128: 8 against 9,
+    and half the call's host time)."""
+    if (type(x) is torch.Tensor and x.dim() == 2 and x.is_cuda and x.dtype is torch.float16
+            and x.is_contiguous() and x.shape[0] > 0 and _is_plain_linear(m)
+            and not torch.is_autocast_enabled() and not torch.compiler.is_compiling()
+            and not torch.jit.is_tracing()):
+        w, b = m.weight, m.bias
+        M, K = w.shape
+        if (K % 8 == 0 and K <= 256 and M % 32 == 0 and M <= 32768 and x.shape[1] == K
+                and (K <= 128 or M <= 128 or x.shape[0] >= 65536)
+                and w.dtype is torch.float16 and w.device == x.device and w.is_contiguous()
+                and type(w) is torch.nn.Parameter
+                and (b is None or (b.dtype is torch.float16 and b.device == x.device
+                                   and b.is_contiguous()))
+                and (x.data_ptr() | w.data_ptr()) % 16 == 0
+                and x.device.index == torch.cuda.current_device()):
+            y = torch.empty((x.shape[0], M), dtype=torch.float16, device=x.device)
+            check(_lib.hip().f3s_linear_f16(
+                x.data_ptr(), w.data_ptr(), b.data_ptr() if b is not None else None,
+                y.data_ptr(), x.shape[0], K, M, torch.cuda.current_stream().cuda_stream),
+                "f3s_linear_f16")
+            return y
+    return m(x)
+
+
 class GraphTransformerLayer(torch.nn.Module):
     """x -> [Q K V] = x W_qkv -> fused edge attention per head -> concat ->
     W_o, forward only.  Compute dtype of the projections is the module's
@@ -188,7 +228,7 @@ class GraphTransformerLayer(torch.nn.Module):
         if graph.heads != self.heads:
             raise ValueError("graph was planned for a different head count")
         n = x.shape[0]
-        qkv = self.qkv(x).to(torch.float16)
+        qkv = _project(self.qkv, x).to(torch.float16)
         dtype = self.proj.weight.dtype
         if graph.takes_packed() and qkv.dim() == 2 and qkv.is_contiguous():
             # the pass reads q, k and v where the projection wrote them, and
@@ -199,7 +239,7 @@ class GraphTransformerLayer(torch.nn.Module):
             qkv = qkv.view(n, 3, self.heads, HEAD_DIM)
             q, k, v = (qkv[:, i].contiguous() for i in range(3))
             o = graph.attention(q, k, v, scale=self.scale)
-        return self.proj(o.view(n, self.heads * HEAD_DIM).to(dtype))
+        return _project(self.proj, o.view(n, self.heads * HEAD_DIM).to(dtype))
 
 
 # ------------------------------------------------------------------ operator

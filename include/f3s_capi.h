@@ -269,6 +269,14 @@ f3s_status f3s_attention_fwd_packed(const f3s_plan* plan, const uint16_t* QKV, v
                                     int32_t out_half, int32_t n, int32_t d, int32_t H,
                                     float scale, void* stream);
 
+/* The projections around the fused pass (no reference counterpart): Y[n][M] =
+ * X[n][K] W[M][K]^T + bias[M] (NULL: none), all binary16, sums in float32,
+ * rounded once.  K a multiple of 8 up to 256, M a multiple of 32 up to 32768,
+ * X, W and Y 16-byte aligned; F3S_EUNSUPPORTED otherwise.  Asynchronous on
+ * `stream`. */
+f3s_status f3s_linear_f16(const uint16_t* X, const uint16_t* W, const uint16_t* bias, uint16_t* Y,
+                          int64_t n, int32_t K, int32_t M, void* stream);
+
 /* Measurement only (no reference counterpart): the device's random-gather
  * ceiling for the fused pass's access pattern.  For each of `count` columns
  * (a multiple of 32) it loads the 128-byte row at byte offset
