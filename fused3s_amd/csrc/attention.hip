@@ -1597,12 +1597,12 @@ f3s_status f3s_plan_compile(f3s_plan* plan, const int32_t* d_block_col,
     F3S_HIP(hipGetLastError());
     bool pinned = false;
     int64_t* h = host_staging(&pinned);
-    int64_t* status = pinned ? h : reinterpret_cast<int64_t*>(mem);
-    F3S_TRY(counts_to_offsets(counts, chunk_base, ni, sums, nullptr, status, st));
+    int64_t* chunks = pinned ? h : reinterpret_cast<int64_t*>(mem);
+    F3S_TRY(counts_to_offsets(counts, chunk_base, ni, sums, chunks, st));
     if (!pinned)
-        F3S_HIP(hipMemcpyAsync(h, status, 2 * sizeof(int64_t), hipMemcpyDeviceToHost, st));
+        F3S_HIP(hipMemcpyAsync(h, chunks, sizeof(int64_t), hipMemcpyDeviceToHost, st));
     F3S_HIP(hipStreamSynchronize(st));
-    const int64_t total = h[1];
+    const int64_t total = h[0];
     if (total >= INT32_MAX) {
         set_error("f3s_plan_compile: more than 2^31-1 chunks");
         return F3S_EUNSUPPORTED;

@@ -43,7 +43,11 @@ constexpr int kEPT = 8;                           // edges per thread kept in re
 constexpr int kHubBatch = 4;                      // edge loads in flight per thread, wide windows
 static_assert(kSumWords == kWave, "the summary is scanned by one wave");
 
-enum ConvErr : int32_t { kErrNone = 0, kErrRowPtr = 1, kErrCol = 2, kErrCount = 4 };
+// Error flags of a call, one word each: in pinned host memory, cleared by the
+// host before the launch, so that a kernel only ever stores to them (an atomic
+// OR there would cross PCIe) and no launch clears or copies them.
+enum ConvErr : int { kErrRowPtr = 0, kErrCol = 1, kErrCount = 2, kErrWords = 3 };
+__device__ __forceinline__ void raise_error(int32_t* err, ConvErr e) { err[e] = 1; }
 
 // The count pass needs only the bitmap; its LDS stays small for occupancy.
 // MT tile masks are staged at once (one per thread of the workgroup).
@@ -78,7 +82,7 @@ __device__ __forceinline__ WindowRows load_window_rows(const int32_t* __restrict
     __syncthreads();
     if ((int)threadIdx.x < wr.nrows) {
         int32_t a = rp[threadIdx.x], b = rp[threadIdx.x + 1];
-        if (a < 0 || b < a || b > nnz) atomicOr(err, kErrRowPtr);
+        if (a < 0 || b < a || b > nnz) raise_error(err, kErrRowPtr);
     }
     wr.e0 = rp[0];
     wr.E = (int64_t)rp[wr.nrows] - wr.e0;
@@ -120,7 +124,7 @@ convert_one_window(ConvLds<FILL, NT>& L, int32_t w, const int32_t* __restrict__ 
     WindowRows wr = load_window_rows(row_ptr, n, nnz, w, L.rp, err);
     __syncthreads();
     if (wr.E < 0 || wr.e0 < 0 || wr.e0 + wr.E > nnz) {
-        if (tid == 0) atomicOr(err, kErrRowPtr);
+        if (tid == 0) raise_error(err, kErrRowPtr);
         return;
     }
     int32_t out_base = 0, expect = 0;
@@ -132,7 +136,7 @@ convert_one_window(ConvLds<FILL, NT>& L, int32_t w, const int32_t* __restrict__ 
         out_base = window_offsets[w];
         expect = window_offsets[w + 1] - out_base;
         if (out_base < 0 || expect < 0 || out_base > total - expect) {
-            if (tid == 0) atomicOr(err, kErrCount);
+            if (tid == 0) raise_error(err, kErrCount);
             return;
         }
     }
@@ -372,9 +376,9 @@ convert_one_window(ConvLds<FILL, NT>& L, int32_t w, const int32_t* __restrict__ 
         __syncthreads();
     }
     if (tid == 0) {
-        if (L.bad) atomicOr(err, kErrCol);
+        if (L.bad) raise_error(err, kErrCol);
         if (FILL) {
-            if (running != expect) atomicOr(err, kErrCount);
+            if (running != expect) raise_error(err, kErrCount);
         } else {
             counts[w] = running;
         }
@@ -400,7 +404,8 @@ convert_wide(const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ co
 // either pass, lists them per block of kListBlock windows: the heavy ones
 // (more than kHeavyEdges edges) from the front of the block's part of
 // `hubs`, the others from its back, and both counts in seg[block] -- no
-// counter to clear first.  It also clears the pass's error bits.  The first
+// counter to clear first.  (Up to kFindW windows each hub workgroup looks
+// through the row pointers itself instead: a launch less.)  The first
 // workgroups of the main launch take one listed window each, heavy ones
 // first, so that the longest chains start first and the light windows fill
 // in behind them (hub workgroups dealt out between the light ones: 8 to 36 us
@@ -412,6 +417,8 @@ constexpr int kListBlock = 1024;
 constexpr int kHubLaunch = 2048;   // hub workgroups of a launch at most (they loop over the list)
 constexpr int kLightMaxW = 262144; // windows of the widest graph convert_waves takes
 static_assert(kLightMaxW / kListBlock <= kConvThreads, "one thread per block of the list");
+constexpr int kFindPer = 8;        // windows a thread looks at
+constexpr int kFindW = kConvThreads * kFindPer;
 
 // The window's edges as the main launch counts them too.
 __device__ __forceinline__ int32_t window_edges(int32_t first, int32_t end)
@@ -421,7 +428,7 @@ __device__ __forceinline__ int32_t window_edges(int32_t first, int32_t end)
 
 __global__ void __launch_bounds__(kListBlock)
 list_hubs(const int32_t* __restrict__ row_ptr, int32_t n, int32_t W, int2* __restrict__ seg,
-          int32_t* __restrict__ hubs, int32_t* __restrict__ err)
+          int32_t* __restrict__ hubs)
 {
     __shared__ int2 part[kListBlock / kWave];
     const int t = threadIdx.x, lane = t & (kWave - 1), wid = t / kWave;
@@ -443,35 +450,57 @@ list_hubs(const int32_t* __restrict__ row_ptr, int32_t n, int32_t W, int2* __res
     int32_t* dst = hubs + (int64_t)blockIdx.x * kListBlock;
     if (heavy) dst[before.x + __popcll(mh & below)] = w;
     if (other) dst[kListBlock - 1 - (before.y + __popcll(mo & below))] = w;
-    if (t == 0) {
-        seg[blockIdx.x] = all;
-        if (blockIdx.x == 0) *err = 0;
-    }
+    if (t == 0) seg[blockIdx.x] = all;
 }
 
-// Window of list entry i (heavy windows first), or -1 past the list's end.
-// Every thread of the workgroup calls it; `lds` needs kConvThreads / 64 + 1
-// int64.
-__device__ __forceinline__ int32_t hub_entry(int32_t i, int32_t W, const int2* __restrict__ seg,
+// Window of hub i (heavy windows first), or -1 past the last: from the list,
+// or (seg == NULL) from the row pointers.  Every thread of the workgroup calls
+// it; `lds` needs kConvThreads / 64 + 1 int64.
+__device__ __forceinline__ int32_t hub_entry(int32_t i, int32_t n, int32_t W,
+                                             const int32_t* __restrict__ row_ptr,
+                                             const int2* __restrict__ seg,
                                              const int32_t* __restrict__ hubs, int64_t* lds)
 {
-    const int32_t nb = (W + kListBlock - 1) / kListBlock;
     const int t = threadIdx.x;
     int32_t* found = reinterpret_cast<int32_t*>(lds + kConvThreads / kWave);
-    const int2 s = t < nb ? seg[t] : make_int2(0, 0);
+    int2 s = make_int2(0, 0);   // heavy and other hubs of this thread's part
+    uint32_t heavy = 0, other = 0;
+    if (seg) {
+        if (t < (W + kListBlock - 1) / kListBlock) s = seg[t];
+    } else {
+        int32_t e[kFindPer + 1];
+#pragma unroll
+        for (int k = 0; k <= kFindPer; ++k)
+            e[k] = row_ptr[min(16 * (int64_t)(t * kFindPer + k), (int64_t)n)];
+#pragma unroll
+        for (int k = 0; k < kFindPer; ++k) {
+            const int32_t E = window_edges(e[k], e[k + 1]);
+            if (t * kFindPer + k >= W || E <= kLightEdges) continue;
+            (E > kHeavyEdges ? heavy : other) |= 1u << k;
+        }
+        s = make_int2(__popc(heavy), __popc(other));
+    }
     if (t == 0) *found = -1;
     int64_t all;
     const int64_t ex = block_exclusive_scan<kConvThreads>(
         (int64_t)s.x | ((int64_t)s.y << 32), lds, all);   // barriers inside
-    const int32_t h = i - (int32_t)(ex & 0xffffffff);
-    const int32_t o = i - (int32_t)(all & 0xffffffff) - (int32_t)(ex >> 32);
-    if (h >= 0 && h < s.x) *found = t * kListBlock + h;
-    if (i >= (int32_t)(all & 0xffffffff) && o >= 0 && o < s.y)
-        *found = t * kListBlock + kListBlock - 1 - o;
+    int32_t h = i - (int32_t)(ex & 0xffffffff);
+    int32_t o = i - (int32_t)(all & 0xffffffff) - (int32_t)(ex >> 32);
+    if (h >= s.x) h = -1;
+    if (i < (int32_t)(all & 0xffffffff) || o >= s.y) o = -1;
+    if (h >= 0 || o >= 0) {   // one thread at most
+        if (seg) {
+            *found = hubs[t * kListBlock + (h >= 0 ? h : kListBlock - 1 - o)];
+        } else {
+            uint32_t m = h >= 0 ? heavy : other;
+            for (int32_t k = max(h, o); k > 0; --k) m &= m - 1u;
+            *found = t * kFindPer + __builtin_ctz(m);
+        }
+    }
     __syncthreads();
-    const int32_t at = *found;
+    const int32_t w = *found;
     __syncthreads();
-    return at < 0 ? -1 : hubs[at];
+    return w;
 }
 
 extern __shared__ __align__(16) unsigned char conv_lds[];
@@ -550,7 +579,7 @@ hub_window(int32_t w, const int32_t* __restrict__ row_ptr, const int32_t* __rest
     const WindowRows wr = load_window_rows(row_ptr, n, nnz, w, head.rp, err);   // a barrier inside
     if (wr.E < 0 || wr.e0 < 0 || wr.e0 + wr.E > nnz) {   // uniform
         if (tid == 0) {
-            atomicOr(err, kErrRowPtr);
+            raise_error(err, kErrRowPtr);
             if (!FILL) counts[w] = 0;
         }
         return;
@@ -584,7 +613,7 @@ hub_window(int32_t w, const int32_t* __restrict__ row_ptr, const int32_t* __rest
             }
         }
     }
-    if (__any(bad) && (tid & (kWave - 1)) == 0) atomicOr(err, kErrCol);
+    if (__any(bad) && (tid & (kWave - 1)) == 0) raise_error(err, kErrCol);
     if constexpr (!FILL) {
         int64_t T;
         (void)block_exclusive_scan<NT>((int64_t)fresh, head.scan, T);   // barriers inside
@@ -611,7 +640,7 @@ hub_window(int32_t w, const int32_t* __restrict__ row_ptr, const int32_t* __rest
         // [0, window_offsets[W]], the size of block_col / tile_mask
         const bool fits = out_base >= 0 && expect >= 0 &&
                           out_base <= window_offsets[W] - expect && total <= expect;
-        if ((!fits || total != expect) && tid == 0) atomicOr(err, kErrCount);
+        if ((!fits || total != expect) && tid == 0) raise_error(err, kErrCount);
         if (!fits) return;   // uniform
         auto rank = [&](int32_t c) __attribute__((always_inline)) -> uint32_t {
             const int32_t wi = c >> 9;
@@ -803,12 +832,13 @@ convert_waves(const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ c
               const int32_t* __restrict__ window_offsets, int32_t* __restrict__ block_col,
               uint16_t* __restrict__ tile_mask, bool stream, int32_t hub_wgs,
               const int2* __restrict__ seg,
-              const int32_t* __restrict__ hubs, int32_t* __restrict__ err)
+              const int32_t* __restrict__ hubs, int32_t* __restrict__ err,
+              int64_t* __restrict__ tiles_out)
 {
     if ((int32_t)blockIdx.x < hub_wgs) {
         HubHead& head = *reinterpret_cast<HubHead*>(conv_lds);
         for (int32_t i = blockIdx.x;; i += hub_wgs) {
-            const int32_t w = hub_entry(i, W, seg, hubs, head.scan);
+            const int32_t w = hub_entry(i, n, W, row_ptr, seg, hubs, head.scan);
             if (w < 0 || w >= W) return;   // uniform: past the list's end
             hub_window<FILL>(w, row_ptr, col_idx, n, nnz, W, counts, window_offsets, block_col,
                              tile_mask, stream, head, conv_lds + kHubHead,
@@ -832,6 +862,7 @@ convert_waves(const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ c
         if (FILL && lane == 19) p = window_offsets + W;
         if (p) v = *p;
     }
+    if (FILL && w == 0 && lane == 19) *tiles_out = v;   // for the host
     const int32_t sums = (W + 1023) / 1024;
     unsigned char* lds = conv_lds + wave * wave_lds_bytes(sums, FILL);
     uint2* sp = reinterpret_cast<uint2*>(lds);   // .x words that hold an edge, .y words before
@@ -867,9 +898,9 @@ convert_waves(const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ c
         if (lane == 0) {
             if (!FILL) counts[w] = 0;
             if (!rows_ok)
-                atomicOr(err, kErrRowPtr);
+                raise_error(err, kErrRowPtr);
             else if (FILL && (!out_ok || expect != 0))
-                atomicOr(err, kErrCount);
+                raise_error(err, kErrCount);
         }
         return;
     }
@@ -900,7 +931,7 @@ convert_waves(const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ c
         if (!ok) p = &dummy[lane];
         atomicOr(p, 1u << (wi & 31));
     });
-    if (__any(bad) && lane == 0) atomicOr(err, kErrCol);
+    if (__any(bad) && lane == 0) raise_error(err, kErrCol);
     wave_lds_order();
     int32_t nw = 0;
     for (int s0 = 0; s0 < sums; s0 += kWave) {
@@ -941,7 +972,7 @@ convert_waves(const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ c
         }
         wave_lds_order();
         if (total != expect) {
-            if (lane == 0) atomicOr(err, kErrCount);
+            if (lane == 0) raise_error(err, kErrCount);
             if (total > expect) return;
         }
         // an edge's row: the first edges of the non-empty rows up to its own
@@ -999,7 +1030,7 @@ convert_waves(const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ c
 // needs none), scans its block
 // straight into the int32 offsets -- T <= nnz <= INT32_MAX, since a tile
 // holds at least one edge -- and its last workgroup writes offsets[W] and the
-// host's status words (error bits, T).
+// total in 64 bits.
 // ---------------------------------------------------------------------------
 constexpr int kOffsThreads = 256;
 constexpr int kOffsPerThread = 8;
@@ -1038,8 +1069,7 @@ offsets_scan_sums(int64_t* __restrict__ sums, int64_t nblocks)
 
 __global__ void __launch_bounds__(kOffsThreads)
 offsets_apply(const int32_t* __restrict__ counts, int64_t W, const int64_t* __restrict__ sums,
-              bool scanned, int32_t* __restrict__ offsets, const int32_t* __restrict__ err,
-              int64_t* __restrict__ status)
+              bool scanned, int32_t* __restrict__ offsets, int64_t* __restrict__ total_out)
 {
     __shared__ int64_t lds[kOffsThreads / kWave];
     int64_t before;
@@ -1067,15 +1097,14 @@ offsets_apply(const int32_t* __restrict__ counts, int64_t W, const int64_t* __re
     }
     if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
         offsets[W] = (int32_t)(before + total);
-        status[0] = err ? *err : 0;
-        status[1] = before + total;
+        *total_out = before + total;
     }
 }
 
 int64_t offsets_sum_elems(int64_t W) { return W > 0 ? ceil_div(W, kOffsTile) : 1; }
 
 f3s_status counts_to_offsets(const int32_t* counts, int32_t* offsets, int64_t W, int64_t* sums,
-                             const int32_t* err, int64_t* status, hipStream_t stream)
+                             int64_t* total_out, hipStream_t stream)
 {
     const int64_t nb = offsets_sum_elems(W);
     if (nb > 1)
@@ -1085,27 +1114,30 @@ f3s_status counts_to_offsets(const int32_t* counts, int32_t* offsets, int64_t W,
     if (scanned)
         hipLaunchKernelGGL(offsets_scan_sums, dim3(1), dim3(kOffsThreads), 0, stream, sums, nb);
     hipLaunchKernelGGL(offsets_apply, dim3((unsigned)nb), dim3(kOffsThreads), 0, stream, counts,
-                       W, sums, scanned, offsets, err, status);
+                       W, sums, scanned, offsets, total_out);
     F3S_HIP(hipGetLastError());
     return F3S_OK;
 }
 
-// The fill pass's error bits and the tile count it was given (status[0..1]).
-__global__ void fill_status(const int32_t* __restrict__ window_offsets, int32_t W,
-                            const int32_t* __restrict__ err, int64_t* __restrict__ status)
+// The tile count a fill was given, for the host (convert_waves does it itself).
+__global__ void report_tiles(const int32_t* __restrict__ window_offsets, int32_t W,
+                             int64_t* __restrict__ tiles_out)
 {
-    if (threadIdx.x == 0) {
-        status[0] = *err;
-        status[1] = window_offsets[W];
-    }
+    if (threadIdx.x == 0) *tiles_out = window_offsets[W];
 }
 
-// Per-call workspace of the converter, one allocation: the error bits, the
-// two status words where the host cannot be written to, the hub list and, for
-// the count pass, the counts and their scan's block sums.
+// What a call reports to the host: the tile count and the error flags.
+struct ConvertStatus {
+    int64_t tiles;
+    int32_t err[kErrWords + 1];
+};
+static_assert(sizeof(ConvertStatus) <= 16 * sizeof(int64_t), "fits the staging words");
+
+// Per-call workspace of the converter, one allocation: the status where no
+// pinned memory was to be had, the hub list and, for the count pass, the
+// counts and their scan's block sums.
 struct ConvertScratch {
-    int32_t* err;
-    int64_t* status;
+    ConvertStatus* status;
     int2* seg;
     int32_t* hubs;
     int32_t* counts;
@@ -1114,18 +1146,16 @@ struct ConvertScratch {
 
 static f3s_status convert_scratch(StreamBuffer& buf, int32_t W, bool count, ConvertScratch& s)
 {
-    const size_t blocks = W <= kLightMaxW ? (size_t)ceil_div(W, kListBlock) : 0;
-    const size_t head = 32;   // err, pad, status[2]
+    const size_t blocks = W > kFindW && W <= kLightMaxW ? (size_t)ceil_div(W, kListBlock) : 0;
     const size_t seg = sizeof(int2) * blocks;
     const size_t hubs = sizeof(int32_t) * blocks * kListBlock;
     const size_t counts = count ? sizeof(int32_t) * (size_t)W : 0;
     const size_t tmp = count ? sizeof(int64_t) * (size_t)offsets_sum_elems(W) : 0;
     auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
-    F3S_TRY(buf.reserve(al(head) + al(seg) + al(hubs) + al(counts) + al(tmp)));
+    F3S_TRY(buf.reserve(al(sizeof(ConvertStatus)) + al(seg) + al(hubs) + al(counts) + al(tmp)));
     char* p = static_cast<char*>(buf.ptr);
-    s.err = reinterpret_cast<int32_t*>(p);
-    s.status = reinterpret_cast<int64_t*>(p + 16);
-    p += al(head);
+    s.status = reinterpret_cast<ConvertStatus*>(p);
+    p += al(sizeof(ConvertStatus));
     s.seg = reinterpret_cast<int2*>(p);
     p += al(seg);
     s.hubs = reinterpret_cast<int32_t*>(p);
@@ -1136,43 +1166,47 @@ static f3s_status convert_scratch(StreamBuffer& buf, int32_t W, bool count, Conv
     return F3S_OK;
 }
 
-// One pass (count or fill) over all windows: the hub list, then one launch of
-// a workgroup per hub window and a wave per other window.  A valid CSR of nnz
-// edges has at most nnz / (kLightEdges + 1) hub windows; how many it has is
-// known on the device only, so that many hub workgroups (at most kHubLaunch)
-// look for their entry and leave if there is none.  Graphs too wide for a
-// wave's bitmap run every window through the per-window kernel.
+// One pass (count or fill) over all windows: one launch of a workgroup per hub
+// window and a wave per other window, on larger graphs after the hub list's. A
+// valid CSR of nnz edges has at most nnz / (kLightEdges + 1) hub windows; how
+// many it has is known on the device only, so that many hub workgroups (at
+// most kHubLaunch) look for theirs and leave if there is none.  Graphs too
+// wide for a wave's bitmap run every window through the per-window kernel.
 template <bool FILL>
 static f3s_status launch_pass(const int32_t* row_ptr, const int32_t* col_idx, int32_t n,
                               int64_t nnz, int32_t W, const int32_t* window_offsets,
                               int32_t* block_col, uint16_t* tile_mask, const ConvertScratch& s,
-                              hipStream_t stream)
+                              ConvertStatus* status, hipStream_t stream)
 {
     if (W <= 0 || W > kLightMaxW) {
-        F3S_HIP(hipMemsetAsync(s.err, 0, sizeof(int32_t), stream));
         if (W > 0)
             hipLaunchKernelGGL(convert_wide<FILL>, dim3((unsigned)W), dim3(kConvThreads), 0,
                                stream, row_ptr, col_idx, n, nnz, W, s.counts, window_offsets,
-                               block_col, tile_mask, s.err);
+                               block_col, tile_mask, status->err);
+        if (FILL)
+            hipLaunchKernelGGL(report_tiles, dim3(1), dim3(64), 0, stream, window_offsets, W,
+                               &status->tiles);
         F3S_HIP(hipGetLastError());
         return F3S_OK;
     }
-    hipLaunchKernelGGL(list_hubs, dim3((unsigned)ceil_div(W, kListBlock)), dim3(kListBlock), 0,
-                       stream, row_ptr, n, W, s.seg, s.hubs, s.err);
     const int64_t most = std::min<int64_t>(nnz / (kLightEdges + 1), W);
     const int32_t hub_wgs = (int32_t)std::min<int64_t>(most, kHubLaunch);
+    const bool listed = hub_wgs > 0 && W > kFindW;
+    if (listed)
+        hipLaunchKernelGGL(list_hubs, dim3((unsigned)ceil_div(W, kListBlock)), dim3(kListBlock), 0,
+                           stream, row_ptr, n, W, s.seg, s.hubs);
     hipLaunchKernelGGL(convert_waves<FILL>, dim3((unsigned)(hub_wgs + ceil_div(W, kWavesPerWg))),
                        dim3(kConvThreads), convert_lds_bytes(W, FILL), stream, row_ptr, col_idx,
-                       n, nnz, W, s.counts, window_offsets, block_col, tile_mask, nnz > kStreamTiles,
-                       hub_wgs, s.seg, s.hubs, s.err);
+                       n, nnz, W, s.counts, window_offsets, block_col, tile_mask,
+                       nnz > kStreamTiles, hub_wgs, listed ? s.seg : nullptr, s.hubs, status->err,
+                       &status->tiles);
     F3S_HIP(hipGetLastError());
     return F3S_OK;
 }
 
-// Count call: tile counts, their scan into the caller's offsets, and one
-// host round trip for the error bits and T.  Fill call: the lists, and one
-// round trip for the error bits.  The last kernel of either writes the two
-// words to pinned host memory itself (a copy is one more launch).
+// Count call: tile counts and their scan into the caller's offsets.  Fill
+// call: the lists.  One host round trip each, for T and the error flags, which
+// the kernels write to pinned host memory themselves.
 static f3s_status convert_impl(const int32_t* row_ptr, const int32_t* col_idx, int32_t n,
                                int64_t nnz, int32_t* window_offsets, int32_t* block_col,
                                uint16_t* tile_mask, int64_t* T_out, hipStream_t stream)
@@ -1183,31 +1217,31 @@ static f3s_status convert_impl(const int32_t* row_ptr, const int32_t* col_idx, i
     ConvertScratch s;
     F3S_TRY(convert_scratch(buf, W, count, s));
     bool pinned = false;
-    int64_t* h = host_staging(&pinned);
-    int64_t* status = pinned ? h : s.status;
+    ConvertStatus* h = reinterpret_cast<ConvertStatus*>(host_staging(&pinned));
+    *h = ConvertStatus{};
+    ConvertStatus* status = pinned ? h : s.status;
+    if (!pinned) F3S_HIP(hipMemsetAsync(status, 0, sizeof(ConvertStatus), stream));
     if (count) {
         F3S_TRY(launch_pass<false>(row_ptr, col_idx, n, nnz, W, nullptr, nullptr, nullptr, s,
-                                   stream));
-        F3S_TRY(counts_to_offsets(s.counts, window_offsets, W, s.tmp, s.err, status, stream));
+                                   status, stream));
+        F3S_TRY(counts_to_offsets(s.counts, window_offsets, W, s.tmp, &status->tiles, stream));
     } else {
         F3S_TRY(launch_pass<true>(row_ptr, col_idx, n, nnz, W, window_offsets, block_col,
-                                  tile_mask, s, stream));
-        hipLaunchKernelGGL(fill_status, dim3(1), dim3(64), 0, stream, window_offsets, W, s.err,
-                           status);
+                                  tile_mask, s, status, stream));
     }
     F3S_HIP(hipGetLastError());
     if (!pinned)
-        F3S_HIP(hipMemcpyAsync(h, s.status, 2 * sizeof(int64_t), hipMemcpyDeviceToHost, stream));
+        F3S_HIP(hipMemcpyAsync(h, status, sizeof(ConvertStatus), hipMemcpyDeviceToHost, stream));
     F3S_HIP(hipStreamSynchronize(stream));
-    const int32_t h_err = (int32_t)h[0];
-    const int64_t total = h[1];
+    const int32_t* err = h->err;
+    const int64_t total = h->tiles;
     if (count) {
         // (on an error the offsets written are meaningless, as documented)
-        if (h_err & kErrRowPtr) {
+        if (err[kErrRowPtr]) {
             set_error("f3s_convert_csr_to_bsf: row_ptr is not monotone within [0, nnz]");
             return F3S_EDATA;
         }
-        if (h_err & kErrCol) {
+        if (err[kErrCol]) {
             set_error("f3s_convert_csr_to_bsf: a column index is outside [0, n)");
             return F3S_EDATA;
         }
@@ -1218,11 +1252,11 @@ static f3s_status convert_impl(const int32_t* row_ptr, const int32_t* col_idx, i
         *T_out = total;
         return F3S_OK;
     }
-    if (h_err & (kErrRowPtr | kErrCol)) {
+    if (err[kErrRowPtr] || err[kErrCol]) {
         set_error("f3s_convert_csr_to_bsf: CSR violates the format (row_ptr or column range)");
         return F3S_EDATA;
     }
-    if (h_err & kErrCount) {
+    if (err[kErrCount]) {
         set_error("f3s_convert_csr_to_bsf: window_offsets do not match this CSR "
                   "(call once with d_block_col = NULL first)");
         return F3S_EINVAL;

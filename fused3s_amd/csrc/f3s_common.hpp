@@ -26,13 +26,12 @@ inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s);
 constexpr int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // int32 counts[W] -> their exclusive prefix sums offsets[W + 1], in two
-// launches (one for few counts).  The total goes to status[1] too, in 64 bits
-// (offsets are meaningless past INT32_MAX), and *err, or 0, to status[0];
-// `status` may be pinned host memory.  `sums` holds offsets_sum_elems(W)
-// elements.
+// launches (one for few counts).  The total goes to *total_out too, in 64 bits
+// (offsets are meaningless past INT32_MAX); it may be pinned host memory.
+// `sums` holds offsets_sum_elems(W) elements.
 int64_t offsets_sum_elems(int64_t W);
 f3s_status counts_to_offsets(const int32_t* counts, int32_t* offsets, int64_t W, int64_t* sums,
-                             const int32_t* err, int64_t* status, hipStream_t stream);
+                             int64_t* total_out, hipStream_t stream);
 
 // Each translation unit's code object is loaded onto the device at its
 // first kernel launch; these launch one empty kernel per unit (f3s_init).
