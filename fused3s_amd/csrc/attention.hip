@@ -699,6 +699,48 @@ sched_count(const int32_t* __restrict__ window_offsets, const int32_t* __restric
     if (t < kSchedClasses) counts[(int64_t)t * nb + blockIdx.x] = hist[t];
 }
 
+// The tables of one wave, lane = class, from the class's windows: the heavy
+// classes come first, and the team list takes their first team_cap windows.
+// Returns the class's other windows.
+__device__ __forceinline__ int32_t sched_team_tables(int32_t tot, int lane, int32_t team_cap,
+                                                     SchedTables* tab)
+{
+    const int32_t heavy = lane < kSchedClasses / 2 ? tot : 0;
+    const int32_t before = wave_inclusive_scan(heavy) - heavy;
+    const int32_t take = max(0, min(heavy, team_cap - before));
+    const int32_t team_all = min(team_cap, __shfl(before + heavy, kWave - 1));
+    tab->team_base[lane] = lane < kSchedClasses / 2 ? min(before, team_cap) : team_all;
+    tab->taken[lane] = take;
+    tab->size[lane] = tot - take;
+    if (lane == 0) tab->team_items = team_all;
+    return tot - take;
+}
+
+// Wave x, lane = class of `sc` windows: XCD x's share of each class, scanned
+// over the classes.
+__device__ __forceinline__ void sched_xcd_tables(int64_t sc, int lane, int64_t x, SchedTables* tab)
+{
+    const int32_t share = (int32_t)(sc * (x + 1) / kXcds - sc * x / kXcds);
+    const int32_t incl = wave_inclusive_scan(share);
+    tab->xcd_base[x][lane] = incl - share;
+    if (lane == kWave - 1) tab->xcd_items[x] = incl;
+}
+
+// Window w, the r-th of class q, into its slot.
+__device__ __forceinline__ void sched_place(int32_t w, int q, int32_t r, const SchedTables* tab,
+                                            int32_t* __restrict__ team,
+                                            int32_t* __restrict__ sched)
+{
+    const int32_t take = tab->taken[q];
+    if (r < take) {
+        team[tab->team_base[q] + r] = w;
+        return;
+    }
+    const int64_t sz = tab->size[q], r2 = r - take;
+    const int64_t x = (kXcds * r2 + kXcds - 1) / sz;   // its share: [sz x / 8, sz (x + 1) / 8)
+    sched[(tab->xcd_base[x][q] + (r2 - sz * x / kXcds)) * kXcds + x] = w;
+}
+
 // One workgroup of 1,024 threads: counts[q][b] becomes the class-q windows in
 // blocks before b; then the tables.  The counts were written by other XCDs a
 // kernel earlier, so every load goes below L2: each class's row is cut into
@@ -762,28 +804,9 @@ sched_scan(int32_t* __restrict__ counts, int32_t nb, int32_t team_cap, SchedTabl
         }
     }
     __syncthreads();
-    if (wid == 0) {
-        // lane = class: the heavy classes come first, and the team list takes
-        // their first team_cap windows
-        const int32_t tot = total[lane];
-        const int32_t heavy = lane < kSchedClasses / 2 ? tot : 0;
-        const int32_t before = wave_inclusive_scan(heavy) - heavy;
-        const int32_t take = max(0, min(heavy, team_cap - before));
-        const int32_t team_all = min(team_cap, __shfl(before + heavy, kWave - 1));
-        tab->team_base[lane] = lane < kSchedClasses / 2 ? min(before, team_cap) : team_all;
-        tab->taken[lane] = take;
-        tab->size[lane] = size[lane] = tot - take;
-        if (lane == 0) tab->team_items = team_all;
-    }
+    if (wid == 0) size[lane] = sched_team_tables(total[lane], lane, team_cap, tab);
     __syncthreads();
-    if (wid < kXcds) {
-        // wave x: XCD x's share of each class, scanned over the classes
-        const int64_t x = wid, sc = size[lane];
-        const int32_t share = (int32_t)(sc * (x + 1) / kXcds - sc * x / kXcds);
-        const int32_t incl = wave_inclusive_scan(share);
-        tab->xcd_base[x][lane] = incl - share;
-        if (lane == kWave - 1) tab->xcd_items[x] = incl;
-    }
+    if (wid < kXcds) sched_xcd_tables(size[lane], lane, wid, tab);
 }
 
 // Slots: the team list (kHeavyMaxWindows entries) and 8 L one-wave slots, slot
@@ -819,15 +842,92 @@ sched_fill(const int32_t* __restrict__ window_offsets, const int32_t* __restrict
     __syncthreads();
     if (q < 0) return;
     for (int v = 0; v < wid; ++v) rank += wc[v][q];
-    const int32_t r = counts[(int64_t)q * nb + blockIdx.x] + rank;   // rank in its class
-    const int32_t take = tab->taken[q];
-    if (r < take) {
-        team[tab->team_base[q] + r] = w;
-        return;
+    sched_place(w, q, counts[(int64_t)q * nb + blockIdx.x] + rank, tab, team, sched);
+}
+
+// The whole schedule of up to kSmallSched windows in one workgroup and one
+// launch instead of three (3,126 windows: 9 us instead of 14): the same classes,
+// ranks and tables.  A thread has the windows t, t + 1024, ...; the windows of
+// a (block, wave) pair are in index order, so a class's ranks are a scan over
+// the pairs plus the rank in the wave.  Past kSmallSched the one workgroup's
+// loop takes longer than the launches it saves.
+constexpr int kSmallBlocks = 4;
+constexpr int32_t kSmallSched = kSmallBlocks * kSchedBlock;
+constexpr int kSchedWaves = kSchedBlock / kWave;
+__global__ void __launch_bounds__(kSchedBlock)
+sched_small(const int32_t* __restrict__ window_offsets, const int32_t* __restrict__ order,
+            const int32_t* __restrict__ inv, int32_t W, int32_t team_cap, int32_t L,
+            int32_t* __restrict__ team, int32_t* __restrict__ sched)
+{
+    // counts per (block, wave) and class, then the class's windows before
+    __shared__ int32_t wc[kSmallBlocks * kSchedWaves][kSchedClasses];
+    __shared__ SchedTables tab;
+    __shared__ int32_t total[kSchedClasses];
+    const int t = threadIdx.x, lane = t & (kWave - 1), wid = t / kWave;
+    const int32_t heavy = heavy_tiles(window_offsets[W], W, kHeavyMinTiles, kHeavyMeanFactor);
+    const uint64_t below = (1ull << lane) - 1ull;
+    int q[kSmallBlocks], rank[kSmallBlocks];
+#pragma unroll
+    for (int b = 0; b < kSmallBlocks; ++b)   // (all their loads in flight at once)
+        q[b] = sched_pos(window_offsets, order, inv, W, b * kSchedBlock + t, heavy);
+#pragma unroll
+    for (int b = 0; b < kSmallBlocks; ++b) {
+        if (b * kSchedBlock >= W) {   // uniform
+            wc[b * kSchedWaves + wid][lane] = 0;
+            continue;
+        }
+        int32_t* mine = wc[b * kSchedWaves + wid];
+        mine[lane] = 0;   // (one lane per class)
+        rank[b] = 0;
+        wave_lds_order();
+        uint64_t rem = __ballot(q[b] >= 0);
+        while (rem) {   // one round per class present in the wave
+            const int lead = __ffsll((unsigned long long)rem) - 1;
+            const int cq = __shfl(q[b], lead);
+            const uint64_t m = __ballot(q[b] == cq);
+            if (q[b] == cq) rank[b] = __popcll(m & below);
+            if (lane == lead) mine[cq] = __popcll(m);
+            rem &= ~m;
+        }
     }
-    const int64_t sz = tab->size[q], r2 = r - take;
-    const int64_t x = (kXcds * r2 + kXcds - 1) / sz;   // its share: [sz x / 8, sz (x + 1) / 8)
-    sched[(tab->xcd_base[x][q] + (r2 - sz * x / kXcds)) * kXcds + x] = w;
+    __syncthreads();
+    {
+        // class c = t / 16; each of its 16 lanes scans four (block, wave) pairs
+        constexpr int kPer = kSmallBlocks * kSchedWaves / kScanSegs;
+        const int c = t / kScanSegs, k = t % kScanSegs;
+        int32_t v[kPer], sum = 0;
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            v[i] = wc[k * kPer + i][c];
+            sum += v[i];
+        }
+        int32_t inc = sum;
+#pragma unroll
+        for (int off = 1; off < kScanSegs; off <<= 1) {
+            const int32_t y = __shfl_up(inc, off, kScanSegs);
+            if (k >= off) inc += y;
+        }
+        int32_t run = inc - sum;
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            wc[k * kPer + i][c] = run;
+            run += v[i];
+        }
+        if (k == kScanSegs - 1) total[c] = inc;
+    }
+    __syncthreads();
+    if (wid == 0) sched_team_tables(total[lane], lane, team_cap, &tab);
+    __syncthreads();
+    if (wid < kXcds) sched_xcd_tables(tab.size[lane], lane, wid, &tab);
+    __syncthreads();
+    for (int32_t g = t; g < kXcds * L; g += kSchedBlock)
+        if (g / kXcds >= tab.xcd_items[g % kXcds]) sched[g] = -1;
+    if (t < kHeavyMaxWindows && t >= tab.team_items) team[t] = -1;
+#pragma unroll
+    for (int b = 0; b < kSmallBlocks; ++b)
+        if (q[b] >= 0)
+            sched_place(b * kSchedBlock + t, q[b], wc[b * kSchedWaves + wid][q[b]] + rank[b], &tab,
+                        team, sched);
 }
 
 // Scratch of the scheduled launch for W windows, in 256-byte sections: the
@@ -873,12 +973,17 @@ static f3s_status launch_schedule(const int32_t* d_window_offsets, const int32_t
     if (ordered)
         hipLaunchKernelGGL(sched_inverse, dim3((unsigned)nb), dim3(kSchedBlock), 0, st,
                            d_window_order, W, inv);
-    hipLaunchKernelGGL(sched_count, dim3((unsigned)nb), dim3(kSchedBlock), 0, st,
-                       d_window_offsets, d_window_order, inv, W, nb, counts);
-    hipLaunchKernelGGL(sched_scan, dim3(1), dim3(1024), 0, st, counts, nb, team_cap, tab);
-    hipLaunchKernelGGL(sched_fill, dim3((unsigned)fill_blocks), dim3(kSchedBlock), 0, st,
-                       d_window_offsets, d_window_order, inv, W, nb, counts, tab, (int32_t)L,
-                       team, sched);
+    if (W <= kSmallSched) {
+        hipLaunchKernelGGL(sched_small, dim3(1), dim3(kSchedBlock), 0, st, d_window_offsets,
+                           d_window_order, inv, W, team_cap, (int32_t)L, team, sched);
+    } else {
+        hipLaunchKernelGGL(sched_count, dim3((unsigned)nb), dim3(kSchedBlock), 0, st,
+                           d_window_offsets, d_window_order, inv, W, nb, counts);
+        hipLaunchKernelGGL(sched_scan, dim3(1), dim3(1024), 0, st, counts, nb, team_cap, tab);
+        hipLaunchKernelGGL(sched_fill, dim3((unsigned)fill_blocks), dim3(kSchedBlock), 0, st,
+                           d_window_offsets, d_window_order, inv, W, nb, counts, tab, (int32_t)L,
+                           team, sched);
+    }
     const hipError_t le = hipGetLastError();
     if (le != hipSuccess) return hip_fail(le, "window schedule", __FILE__, __LINE__);
     *team_out = team;

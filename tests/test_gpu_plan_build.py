@@ -66,3 +66,35 @@ def test_plan_positions(gpu, W, seg):
         plan.forward(dq, dk, dv, out, masked=False, scale=0.125)
         gpu.synchronize()
         assert np.abs(out.numpy() - dense).max() <= 2e-3
+
+
+@pytest.mark.parametrize("W", [513, 1024, 1025, 2049, 4095, 4096, 4097])
+@pytest.mark.parametrize("masked", [True, False])
+def test_natural_order_schedule(gpu, W, masked):
+    # the drop-in launch without an order, whose schedule is built by one
+    # workgroup up to 4,096 windows: hub windows of every block column (heavy
+    # past 1,024), windows without edges, a short last window
+    n, r = 16 * W - 7, rng(W)
+    keys = [np.arange(0, n, 3, dtype=np.int64) * (n + 1)]
+    for w in (0, 7, 1000, W - 1):
+        if w < W:
+            u = 16 * w + int(r.integers(0, 9))
+            keys.append(u * np.int64(n) + np.arange(0, n, 16))
+    u = r.integers(0, n, 6 * n)
+    u = u[u // 16 % 50 != 13]
+    keys.append(u * np.int64(n) + r.integers(0, n, len(u)))
+    keys = np.unique(np.concatenate(keys))
+    rp = np.searchsorted(keys // n, np.arange(n + 1)).astype(np.int32)
+    ci = (keys % n).astype(np.int32)
+    bsf = gpu.convert_device(gpu.DeviceCSR(rp, ci))
+    q, k, v = (r.standard_normal((n, 1, 64)).astype(np.float16) for _ in range(3))
+    dev = [gpu.DeviceArray.from_numpy(x.view(np.uint16)) for x in (q, k, v)]
+    out = gpu.DeviceArray((n, 1, 64), np.float32)
+    out.fill_bytes(0xff)   # NaN: a row no window writes fails
+    gpu.attention_fwd(*dev, out, bsf, masked=masked, scale=0.125)
+    gpu.synchronize()
+    f = [x.astype(np.float32) for x in (q, k, v)]
+    want = (orc.masked_attention(n, 64, 1, *f, rp, ci, 0.125) if masked else
+            orc.tile_dense_attention(n, 64, 1, *f, bsf.window_offsets.numpy(),
+                                     bsf.block_col.numpy(), 0.125))
+    assert np.abs(out.numpy() - want).max() <= 2e-3
