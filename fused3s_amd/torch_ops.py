@@ -3,10 +3,10 @@
 The reference has no framework binding; its natural caller is a graph
 attention layer: a QKV projection GEMM, the fused sparse attention over the
 graph's edges, and an output projection.  Here torch supplies the device
-memory, the GEMMs (hipBLASLt through torch.nn.Linear) and the stream; the
-attention itself is the HIP library's planned pass
+memory and the stream; the attention is the HIP library's planned pass
 (f3s_attention_fwd_planned), called on torch's current stream with the
-tensors' device pointers.  There is no CPU fallback and no autograd: the
+tensors' device pointers, and the layer's projections are its f3s_linear_f16
+(torch.nn.Linear's own product where that kernel is not the better one).  There is no CPU fallback and no autograd: the
 fused pass is forward-only, so calling it on tensors that require grad
 raises.
 
@@ -140,7 +140,6 @@ class TorchGraph:
             torch.cuda.current_stream().cuda_stream), "f3s_attention_fwd_planned")
         return out
 
-
     def takes_packed(self) -> bool:
         """Whether attention_packed takes this graph: masked semantics, and
         the packed tensor within the 32-bit offsets of its launch."""
@@ -182,14 +181,14 @@ def _is_plain_linear(m: torch.nn.Module) -> bool:
 def _project(m: torch.nn.Module, x: torch.Tensor) -> torch.Tensor:
     """m(x), by f3s_linear_f16 where that is the same thing: a plain fp16
     Linear of a contiguous fp16 matrix on its own device, in sizes the kernel
-    takes, outside autocast and tracing.  (Called without autograd.)  Below
+    takes, outside autocast, tracing and dispatch modes.  (Called without autograd.)  Below
     64 K rows of more than 128 inputs and outputs the library's tiles are the
     better ones (20,011 x 256 -> 768: 17 against 28 us; -> 128: 8 against 9,
     and half the call's host time)."""
     if (type(x) is torch.Tensor and x.dim() == 2 and x.is_cuda and x.dtype is torch.float16
             and x.is_contiguous() and x.shape[0] > 0 and _is_plain_linear(m)
             and not torch.is_autocast_enabled() and not torch.compiler.is_compiling()
-            and not torch.jit.is_tracing()):
+            and not torch.jit.is_tracing() and torch._C._len_torch_dispatch_stack() == 0):
         w, b = m.weight, m.bias
         M, K = w.shape
         if (K % 8 == 0 and K <= 256 and M % 32 == 0 and M <= 32768 and x.shape[1] == K
@@ -207,6 +206,13 @@ def _project(m: torch.nn.Module, x: torch.Tensor) -> torch.Tensor:
                 "f3s_linear_f16")
             return y
     return m(x)
+
+
+def _is_plain_graph(graph) -> bool:
+    """Whether attention_packed stands for graph.attention: not where a
+    program brings an attention of its own."""
+    return (isinstance(graph, TorchGraph) and type(graph).attention is TorchGraph.attention
+            and "attention" not in graph.__dict__)
 
 
 class GraphTransformerLayer(torch.nn.Module):
@@ -230,7 +236,8 @@ class GraphTransformerLayer(torch.nn.Module):
         n = x.shape[0]
         qkv = _project(self.qkv, x).to(torch.float16)
         dtype = self.proj.weight.dtype
-        if graph.takes_packed() and qkv.dim() == 2 and qkv.is_contiguous():
+        if _is_plain_graph(graph) and graph.takes_packed() and qkv.dim() == 2 \
+                and qkv.is_contiguous():
             # the pass reads q, k and v where the projection wrote them, and
             # writes O in the dtype the output projection takes
             o = graph.attention_packed(qkv, self.scale,

@@ -68,3 +68,28 @@ def test_layer_projections(gpu):
     assert odd(torch.randn(700, 100, device="cuda").half(), graph).shape == (700, 40)
     wide = torch_ops.GraphTransformerLayer(96, heads=2).cuda()                      # float32 module
     assert wide(x.float(), graph).dtype == torch.float32
+
+
+def test_layer_yields_to_overrides(gpu):
+    """A dispatch mode sees the layer's products, and a graph that brings its
+    own attention has it called."""
+    from torch.utils.flop_counter import FlopCounterMode
+
+    from fused3s_amd import torch_ops
+    rp, ci = random_csr(100, 4, 3)
+    graph = torch_ops.TorchGraph(rp, ci, heads=1)
+    layer = torch_ops.GraphTransformerLayer(64, heads=1).cuda().half()
+    x = torch.randn(100, 64, dtype=torch.float16, device="cuda")
+    with FlopCounterMode(display=False) as counter:
+        layer(x, graph)
+    assert counter.get_total_flops() == 2 * 100 * 64 * (192 + 64)
+
+    calls = []
+
+    class Own(torch_ops.TorchGraph):
+        def attention(self, *args, **kwargs):
+            calls.append(1)
+            return super().attention(*args, **kwargs)
+
+    layer(x, Own(rp, ci, heads=1))
+    assert calls
