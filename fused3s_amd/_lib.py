@@ -46,6 +46,7 @@ HIP_API = {
     "f3s_event_elapsed_ms": (c_i32, [c_vp, c_vp, P_f32]),
     "f3s_cast_f32_to_f16": (c_i32, [c_vp, c_vp, c_i64, c_vp]),
     "f3s_convert_csr_to_bsf": (c_i32, [c_vp, c_vp, c_i32, c_i64, c_vp, c_vp, c_vp, P_i64, c_vp]),
+    "f3s_convert_csr_to_bsf_once": (c_i32, [c_vp, c_vp, c_i32, c_i64, c_vp, c_vp, c_vp, P_i64, c_vp]),
     "f3s_window_order": (c_i32, [c_vp, c_i32, c_vp, c_vp]),
     "f3s_bsf_stats": (c_i32, [c_vp, c_vp, c_i64, c_i32, P_i64, P_i64, c_vp]),
     "f3s_attention_fwd": (c_i32, [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp,

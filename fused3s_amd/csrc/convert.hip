@@ -565,8 +565,8 @@ __device__ __forceinline__ void
 hub_window(int32_t w, const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ col_idx,
            int32_t n, int64_t nnz, int32_t W, int32_t* __restrict__ counts,
            const int32_t* __restrict__ window_offsets, int32_t* __restrict__ block_col,
-           uint16_t* __restrict__ tile_mask, bool stream, HubHead& head, unsigned char* work,
-           uint32_t work_bytes, int32_t* __restrict__ err)
+           uint16_t* __restrict__ tile_mask, int32_t cap, bool stream, HubHead& head,
+           unsigned char* work, uint32_t work_bytes, int32_t* __restrict__ err)
 {
     constexpr int NT = kConvThreads;
     int tid = threadIdx.x;
@@ -637,9 +637,9 @@ hub_window(int32_t w, const int32_t* __restrict__ row_ptr, const int32_t* __rest
         __syncthreads();
         const int32_t total = (int32_t)all;
         // the caller's offsets have to describe this CSR, and stay inside
-        // [0, window_offsets[W]], the size of block_col / tile_mask
+        // [0, window_offsets[W]], the size of block_col / tile_mask (or cap)
         const bool fits = out_base >= 0 && expect >= 0 &&
-                          out_base <= window_offsets[W] - expect && total <= expect;
+                          out_base <= min(window_offsets[W], cap) - expect && total <= expect;
         if ((!fits || total != expect) && tid == 0) raise_error(err, kErrCount);
         if (!fits) return;   // uniform
         auto rank = [&](int32_t c) __attribute__((always_inline)) -> uint32_t {
@@ -830,7 +830,7 @@ __global__ void __launch_bounds__(kConvThreads) __attribute__((amdgpu_waves_per_
 convert_waves(const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ col_idx,
               int32_t n, int64_t nnz, int32_t W, int32_t* __restrict__ counts,
               const int32_t* __restrict__ window_offsets, int32_t* __restrict__ block_col,
-              uint16_t* __restrict__ tile_mask, bool stream, int32_t hub_wgs,
+              uint16_t* __restrict__ tile_mask, int32_t cap, bool stream, int32_t hub_wgs,
               const int2* __restrict__ seg,
               const int32_t* __restrict__ hubs, int32_t* __restrict__ err,
               int64_t* __restrict__ tiles_out)
@@ -841,7 +841,7 @@ convert_waves(const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ c
             const int32_t w = hub_entry(i, n, W, row_ptr, seg, hubs, head.scan);
             if (w < 0 || w >= W) return;   // uniform: past the list's end
             hub_window<FILL>(w, row_ptr, col_idx, n, nnz, W, counts, window_offsets, block_col,
-                             tile_mask, stream, head, conv_lds + kHubHead,
+                             tile_mask, cap, stream, head, conv_lds + kHubHead,
                              convert_lds_bytes(W, FILL) - kHubHead, err);
         }
     }
@@ -891,7 +891,7 @@ convert_waves(const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ c
         const int32_t oe = __builtin_amdgcn_readlane(v, 18);
         out_base = __builtin_amdgcn_readlane(v, 17);
         expect = oe - out_base;
-        out_ok = out_base >= 0 && oe >= out_base && oe <= __builtin_amdgcn_readlane(v, 19);
+        out_ok = out_base >= 0 && oe >= out_base && oe <= min(__builtin_amdgcn_readlane(v, 19), cap);
     }
     if (rows_ok && E > kLightEdges) return;   // a hub window: list_hubs has it
     if (!rows_ok || !out_ok || E == 0) {
@@ -1175,8 +1175,8 @@ static f3s_status convert_scratch(StreamBuffer& buf, int32_t W, bool count, Conv
 template <bool FILL>
 static f3s_status launch_pass(const int32_t* row_ptr, const int32_t* col_idx, int32_t n,
                               int64_t nnz, int32_t W, const int32_t* window_offsets,
-                              int32_t* block_col, uint16_t* tile_mask, const ConvertScratch& s,
-                              ConvertStatus* status, hipStream_t stream)
+                              int32_t* block_col, uint16_t* tile_mask, int32_t cap,
+                              const ConvertScratch& s, ConvertStatus* status, hipStream_t stream)
 {
     if (W <= 0 || W > kLightMaxW) {
         if (W > 0)
@@ -1197,7 +1197,7 @@ static f3s_status launch_pass(const int32_t* row_ptr, const int32_t* col_idx, in
                            stream, row_ptr, n, W, s.seg, s.hubs);
     hipLaunchKernelGGL(convert_waves<FILL>, dim3((unsigned)(hub_wgs + ceil_div(W, kWavesPerWg))),
                        dim3(kConvThreads), convert_lds_bytes(W, FILL), stream, row_ptr, col_idx,
-                       n, nnz, W, s.counts, window_offsets, block_col, tile_mask,
+                       n, nnz, W, s.counts, window_offsets, block_col, tile_mask, cap,
                        nnz > kStreamTiles, hub_wgs, listed ? s.seg : nullptr, s.hubs, status->err,
                        &status->tiles);
     F3S_HIP(hipGetLastError());
@@ -1206,13 +1206,15 @@ static f3s_status launch_pass(const int32_t* row_ptr, const int32_t* col_idx, in
 
 // Count call: tile counts and their scan into the caller's offsets.  Fill
 // call: the lists.  One host round trip each, for T and the error flags, which
-// the kernels write to pinned host memory themselves.
+// the kernels write to pinned host memory themselves.  `once`: both at once,
+// into lists of nnz entries, with one round trip -- the offsets of a CSR that
+// turns out to be invalid may pass the lists' end, so the fill is given it.
 static f3s_status convert_impl(const int32_t* row_ptr, const int32_t* col_idx, int32_t n,
                                int64_t nnz, int32_t* window_offsets, int32_t* block_col,
-                               uint16_t* tile_mask, int64_t* T_out, hipStream_t stream)
+                               uint16_t* tile_mask, bool once, int64_t* T_out, hipStream_t stream)
 {
     const int32_t W = (int32_t)ceil_div(n, 16);
-    const bool count = block_col == nullptr;
+    const bool count = once || block_col == nullptr;
     StreamBuffer buf(stream);
     ConvertScratch s;
     F3S_TRY(convert_scratch(buf, W, count, s));
@@ -1222,13 +1224,13 @@ static f3s_status convert_impl(const int32_t* row_ptr, const int32_t* col_idx, i
     ConvertStatus* status = pinned ? h : s.status;
     if (!pinned) F3S_HIP(hipMemsetAsync(status, 0, sizeof(ConvertStatus), stream));
     if (count) {
-        F3S_TRY(launch_pass<false>(row_ptr, col_idx, n, nnz, W, nullptr, nullptr, nullptr, s,
+        F3S_TRY(launch_pass<false>(row_ptr, col_idx, n, nnz, W, nullptr, nullptr, nullptr, 0, s,
                                    status, stream));
         F3S_TRY(counts_to_offsets(s.counts, window_offsets, W, s.tmp, &status->tiles, stream));
-    } else {
-        F3S_TRY(launch_pass<true>(row_ptr, col_idx, n, nnz, W, window_offsets, block_col,
-                                  tile_mask, s, status, stream));
     }
+    if (block_col)
+        F3S_TRY(launch_pass<true>(row_ptr, col_idx, n, nnz, W, window_offsets, block_col,
+                                  tile_mask, once ? (int32_t)nnz : INT32_MAX, s, status, stream));
     F3S_HIP(hipGetLastError());
     if (!pinned)
         F3S_HIP(hipMemcpyAsync(h, status, sizeof(ConvertStatus), hipMemcpyDeviceToHost, stream));
@@ -1249,8 +1251,10 @@ static f3s_status convert_impl(const int32_t* row_ptr, const int32_t* col_idx, i
             set_error("f3s_convert_csr_to_bsf: more than 2^31-1 active tiles");
             return F3S_EUNSUPPORTED;
         }
-        *T_out = total;
-        return F3S_OK;
+        if (!once) {
+            *T_out = total;
+            return F3S_OK;
+        }
     }
     if (err[kErrRowPtr] || err[kErrCol]) {
         set_error("f3s_convert_csr_to_bsf: CSR violates the format (row_ptr or column range)");
@@ -1290,5 +1294,27 @@ extern "C" f3s_status f3s_convert_csr_to_bsf(const int32_t* d_row_ptr, const int
     F3S_TRY(require_device());
     clear_error();
     return convert_impl(d_row_ptr, d_col_idx, n, nnz, d_window_offsets, d_block_col,
-                        d_tile_mask, T_out, as_stream(stream));
+                        d_tile_mask, false, T_out, as_stream(stream));
+}
+
+extern "C" f3s_status f3s_convert_csr_to_bsf_once(const int32_t* d_row_ptr,
+                                                  const int32_t* d_col_idx, int32_t n, int64_t nnz,
+                                                  int32_t* d_window_offsets, int32_t* d_block_col,
+                                                  uint16_t* d_tile_mask, int64_t* T_out,
+                                                  void* stream)
+{
+    using namespace f3s;
+    F3S_REQUIRE(n >= 0 && nnz >= 0, "f3s_convert_csr_to_bsf_once: negative size");
+    F3S_REQUIRE(nnz <= INT32_MAX, "f3s_convert_csr_to_bsf_once: nnz exceeds int32 CSR range");
+    F3S_REQUIRE(d_row_ptr && d_window_offsets && d_block_col && T_out,
+                "f3s_convert_csr_to_bsf_once: NULL pointer");
+    F3S_REQUIRE(nnz == 0 || d_col_idx, "f3s_convert_csr_to_bsf_once: NULL col_idx");
+    if (ceil_div(n, 16) > kLightMaxW) {
+        set_error("f3s_convert_csr_to_bsf_once: n exceeds 4,194,304");
+        return F3S_EUNSUPPORTED;
+    }
+    F3S_TRY(require_device());
+    clear_error();
+    return convert_impl(d_row_ptr, d_col_idx, n, nnz, d_window_offsets, d_block_col,
+                        d_tile_mask, true, T_out, as_stream(stream));
 }

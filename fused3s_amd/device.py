@@ -102,6 +102,11 @@ class DeviceArray:
             check(_lib.hip().f3s_memset(self._ptr, int(value), self.nbytes,
                                         stream.handle if stream else None), "f3s_memset")
 
+    def truncate(self, count: int) -> None:
+        """A 1-d array's first `count` elements from now on (the allocation stays)."""
+        self.shape = (min(int(count), self.shape[0]),)
+        self.nbytes = self.shape[0] * self.dtype.itemsize
+
     def free(self) -> None:
         if getattr(self, "_ptr", None):
             _lib.hip().f3s_free(self._ptr)

@@ -50,7 +50,8 @@ import ctypes as C
 from . import _lib
 from .attention import Plan
 from .device import DeviceArray, Stream, check
-from .graph import DeviceBSF, DeviceCSR, convert_device, window_order_device
+from .graph import (DeviceBSF, DeviceCSR, convert_device, converts_once,
+                    window_order_device)
 
 HEAD_DIM = 64
 
@@ -271,7 +272,8 @@ def to_block_sparse(row_ptr, col_idx, masks: bool = True):
     torch tensors: (window_offsets int32 [W + 1], block_col_indices int32
     [T], tile_mask int16 [T, 16] -- bit c of row r of a tile set iff that
     edge exists -- or None).  Two calls of f3s_convert_csr_to_bsf on torch's
-    current stream: the count (one host round trip for T), then the fill."""
+    current stream, the count (one host round trip for T), then the fill; or,
+    on small graphs, one call for both."""
     rp = _cuda_i32(row_ptr, "row_ptr")
     ci = _cuda_i32(col_idx, "col_idx")
     n = rp.numel() - 1
@@ -283,6 +285,15 @@ def to_block_sparse(row_ptr, col_idx, masks: bool = True):
     offs = torch.empty(W + 1, dtype=torch.int32, device=rp.device)
     T = C.c_int64(0)
     cptr = ci.data_ptr() if ci.numel() else None
+    if converts_once(n, ci.numel()):
+        bcol = torch.empty(ci.numel(), dtype=torch.int32, device=rp.device)
+        mask = (torch.empty((ci.numel(), 16), dtype=torch.int16, device=rp.device) if masks
+                else None)
+        check(lib.f3s_convert_csr_to_bsf_once(
+            rp.data_ptr(), cptr, n, ci.numel(), offs.data_ptr(), bcol.data_ptr(),
+            mask.data_ptr() if masks else None, C.byref(T), s), "f3s_convert_csr_to_bsf_once")
+        t = int(T.value)
+        return offs, bcol[:t], (mask[:t] if masks else None)
     check(lib.f3s_convert_csr_to_bsf(rp.data_ptr(), cptr, n, ci.numel(), offs.data_ptr(), None,
                                      None, C.byref(T), s), "f3s_convert_csr_to_bsf(count)")
     t = int(T.value)
