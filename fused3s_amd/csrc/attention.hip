@@ -158,11 +158,19 @@ __device__ __forceinline__ void merge_split(const AttnParams& p, const SplitInfo
 // the three copies and the cast around a layer's pass away: 500,000 nodes, 2
 // heads, layer 984 -> 742 us (copies 166 us, cast 57 us; the pass itself 491
 // -> 475 us, half the bytes of O).
-template <int MODE, int WPG, bool WIDE, int TEAM, bool PACKED>
+// MIXED: the drop-in launch of a graph that may have heavy windows.  The first
+// p.team_blocks workgroups are teams of WPG waves for those, the others run a
+// window per wave.  (Teams of 16 waves in a launch of their own had the chip to
+// themselves for 98 us on 1 M nodes, 512 heavy windows: 618 -> 581 us per
+// call; with none listed the launch alone cost 3 us, 50,001 nodes 96 -> 93.)
+template <int MODE, int WPG, bool WIDE, int TEAM, bool PACKED, bool MIXED = false>
 __global__ void __launch_bounds__(kWave * WPG) __attribute__((amdgpu_waves_per_eu(4)))
 fused_attention_kernel(const AttnParams p)
 {
     static_assert(TEAM == 1 || TEAM == WPG, "a team fills its workgroup");
+    static_assert(!MIXED || (TEAM == 1 && WPG == kTeamSmall && MODE != kModeList && !WIDE && !PACKED),
+                  "mixed launches: one-wave workgroups of four, unplanned, narrow");
+    constexpr int kTeam = MIXED ? WPG : TEAM;   // a team's waves
     static_assert(!PACKED || (MODE == kModeList && !WIDE), "packed tensors: compiled lists");
     const int H = p.H;
     __shared__ WaveLds lds_all[WPG];
@@ -179,7 +187,15 @@ fused_attention_kernel(const AttnParams p)
     // (num_items is a multiple of TEAM).
     int64_t item_idx;
     int h;
-    if constexpr (TEAM == 1) {
+    const bool in_team = TEAM > 1 || (MIXED && (int32_t)blockIdx.x < p.team_blocks);   // uniform
+    if (MIXED && in_team) {
+        item_idx = blockIdx.x / (uint32_t)H;
+        h = (int)(blockIdx.x % (uint32_t)H);
+    } else if constexpr (MIXED) {
+        const uint32_t gw = (blockIdx.x - (uint32_t)p.team_blocks) * WPG + wave;
+        item_idx = (int64_t)(gw / (uint32_t)H);
+        h = (int)(gw % (uint32_t)H);
+    } else if constexpr (TEAM == 1) {
         const uint32_t gw = (uint32_t)(logical_block(p.xcd_contiguous) * WPG + wave);
         item_idx = (int64_t)(gw / (uint32_t)H);
         h = (int)(gw % (uint32_t)H);
@@ -193,7 +209,7 @@ fused_attention_kernel(const AttnParams p)
     // ---- item decode (wave-uniform) ----
     int32_t w, tb, te, slot;
     int32_t team_n = 1;   // teams: non-empty parts of the window (uniform over the team)
-    if (p.items) {
+    if (!MIXED && p.items) {
         const Item it = p.items[item_idx];
         w = it.w;
         tb = it.tb;
@@ -208,30 +224,39 @@ fused_attention_kernel(const AttnParams p)
         }
     } else {
         const int64_t wi = item_idx / TEAM;
-        w = p.window_order ? p.window_order[wi] : (int32_t)wi;
+        const bool listed = MIXED && in_team && p.team_list;
+        w = listed ? p.team_list[wi] : p.window_order ? p.window_order[wi] : (int32_t)wi;
         if (w < 0 || w >= p.W) return;   // an empty slot or an invalid order entry
         const int32_t T = p.window_offsets[p.W];
         tb = max(0, min(p.window_offsets[w], T));
         te = max(tb, min(p.window_offsets[w + 1], T));
-        if (p.heavy_mode) {
-            // in an order's sequence, the heavy windows among its first
-            // kHeavyMaxWindows entries belong to the team launch (mode 2), all
-            // others to the one-wave launch (mode 1); uniform over a team
-            const bool heavy =
-                wi < kHeavyMaxWindows &&
-                te - tb > heavy_tiles(T, p.W, kHeavyMinTiles, kHeavyMeanFactor);
-            if (heavy != (p.heavy_mode == 2)) return;
+        if (MIXED || (TEAM > 1 && p.huge_only)) {
+            // A window of an order's sequence or of the team list belongs to
+            // one of the huge windows' launch, a team here and a wave here
+            // (uniform over a team; the schedule's one-wave slots hold none
+            // of the team list's).
+            const int32_t heavy = heavy_tiles(T, p.W, kHeavyMinTiles, kHeavyMeanFactor);
+            const bool is_heavy = wi < kHeavyMaxWindows && te - tb > heavy;
+            const bool huge = is_heavy && wi < kHugeMaxWindows && te - tb > kHugeTiles &&
+                              p.W > kHugeTiles;   // (as the launch's condition)
+            if constexpr (!MIXED) {
+                if (!huge) return;
+            } else if (in_team) {
+                if (huge || !is_heavy) return;
+            } else if (!p.team_list && is_heavy) {
+                return;
+            }
         }
-        if constexpr (TEAM > 1) {
-            team_n = team_parts(tb, te, TEAM);
-            const int32_t a = team_part(tb, te, wave, TEAM), b = team_part(tb, te, wave + 1, TEAM);
+        if (in_team) {
+            team_n = team_parts(tb, te, kTeam);
+            const int32_t a = team_part(tb, te, wave, kTeam), b = team_part(tb, te, wave + 1, kTeam);
             tb = a;
             te = b;
         }
         slot = -1;
     }
     // a window of at most one part is wave 0's alone: no merge, no barrier
-    if (TEAM > 1 && team_n <= 1 && wave != 0) return;
+    if (in_team && team_n <= 1 && wave != 0) return;
     const int32_t nbc = (n + 15) >> 4;   // valid block columns
     const int32_t* __restrict__ block_col = p.block_col;
     const __amdgpu_buffer_rsrc_t qres = make_rsrc(p.Q, p.feat_bytes);
@@ -461,7 +486,7 @@ fused_attention_kernel(const AttnParams p)
         }
     }
 
-    if (TEAM > 1 && team_n > 1) {   // uniform over the team
+    if (kTeam > 1 && team_n > 1) {   // uniform over the team (1 outside teams)
         // ---- team merge: waves 1 .. team_n-1 publish (m, l, O^T) lane by
         // lane in their own LDS area, wave 0 folds them in, in wave order
         // (deterministic) ----
@@ -477,7 +502,7 @@ fused_attention_kernel(const AttnParams p)
         if (wave != 0) return;
         float M = st.m;
 #pragma unroll
-        for (int k = 1; k < TEAM; ++k)
+        for (int k = 1; k < kTeam; ++k)
             if (k < team_n) M = __builtin_fmaxf(M, __uint_as_float(lds_all[k].off[lane]));
         if (M != -INFINITY) {   // else no part of the team attended row r: all zero
             const float c0 = fast_exp2(st.m - M);   // 0 when this part is empty
@@ -485,7 +510,7 @@ fused_attention_kernel(const AttnParams p)
 #pragma unroll
             for (int t = 0; t < 4; ++t) st.acc[t] *= c0;
 #pragma unroll
-            for (int k = 1; k < TEAM; ++k) {
+            for (int k = 1; k < kTeam; ++k) {
                 if (k >= team_n) break;
                 const float mk = __uint_as_float(lds_all[k].off[lane]);
                 const float f = fast_exp2(mk - M);   // mk = -inf: 0
@@ -602,7 +627,7 @@ hipError_t warm_attention(hipStream_t s)
 // untouched); the schedule is the library's own, whatever the order:
 //   * heavy windows -- more than max(kHeavyMinTiles, kHeavyMeanFactor x mean)
 //     tiles -- heaviest first; the first kHeavyMaxWindows of them run as
-//     16-wave teams in a launch of their own;
+//     teams;
 //   * every other window on one wave, by class of tile count (the octave;
 //     heavy windows past the team list form the first classes), heaviest
 //     class first, each class in index order and cut into eight contiguous
@@ -1395,6 +1420,14 @@ static void launch_mw(const AttnParams& p, int64_t waves, hipStream_t st)
             return;
         }
     }
+    if constexpr (!WIDE && MODE != kModeList) {
+        if (p.team_blocks > 0) {   // (counted in `waves`)
+            hipLaunchKernelGGL((fused_attention_kernel<MODE, kTeamSmall, false, 1, false, true>),
+                               dim3((unsigned)ceil_div(waves, kTeamSmall)),
+                               dim3(kTeamSmall * kWave), 0, st, p);
+            return;
+        }
+    }
     // Small launches use one-wave workgroups so they spread over all CUs.
     if (waves < 4 * 256 * 2) {
         hipLaunchKernelGGL((fused_attention_kernel<MODE, 1, WIDE, 1, PACKED>),
@@ -1417,7 +1450,7 @@ static void launch_m(const AttnParams& p, int64_t waves, hipStream_t st)
 static f3s_status launch(AttnParams p, int32_t H, float scale, hipStream_t st)
 {
     if (p.num_items <= 0) return F3S_OK;
-    const int64_t waves = p.num_items * H;
+    const int64_t waves = p.num_items * H + (int64_t)p.team_blocks * kTeamSmall;
     F3S_REQUIRE(waves < ((int64_t)1 << 31), "attention: too many work items");
     p.scale_log2 = scale * 1.4426950408889634f;
     p.H = H;
@@ -1505,10 +1538,11 @@ static f3s_status attention_fwd_impl(const uint16_t* Q, const uint16_t* K, const
     // then no team launch (the schedule gets an empty team list, so any
     // window still runs on one wave).
     const bool heavy_possible = W > kHeavyMinTiles;
+    bool mixed = false;   // heavy windows' teams in the launch's first workgroups
     if (p.team == 1 && !wide_features(n, H) && W > kHeavyMaxWindows &&
         (!ordered || (int64_t)W * H >= kSchedOrderedMin)) {
-        // the library's schedule (see sched_fill): heavy windows on teams of
-        // 16 waves, the others on one wave each, by class, XCD by XCD
+        // the library's schedule (see sched_fill): heavy windows on teams, the
+        // others on one wave each, by class, XCD by XCD
         char* sp = static_cast<char*>(fixed_scratch);
         if (!sp) {
             F3S_TRY(scratch.reserve(sched_scratch(W, ordered).bytes));
@@ -1517,29 +1551,30 @@ static f3s_status attention_fwd_impl(const uint16_t* Q, const uint16_t* K, const
         int32_t *team = nullptr, *sched = nullptr;
         F3S_TRY(launch_schedule(d_window_offsets, d_window_order, W,
                                 heavy_possible ? kHeavyMaxWindows : 0, sp, st, &team, &sched));
-        const int64_t L = sched_xcd_slots(W);
-        if (heavy_possible) {
-            AttnParams ph = p;
-            ph.window_order = team;
-            ph.xcd_contiguous = 0;
-            ph.team = kTeamLarge;
-            ph.num_items = (int64_t)kHeavyMaxWindows * kTeamLarge;
-            F3S_TRY(launch(ph, H, scale, st));
-        }
+        p.team_list = heavy_possible ? team : nullptr;
         p.window_order = sched;
         p.xcd_contiguous = 0;
-        p.num_items = kXcds * L;
+        p.num_items = kXcds * sched_xcd_slots(W);
+        mixed = heavy_possible;
     } else if (p.team == 1 && ordered && !wide_features(n, H) && heavy_possible) {
-        // The order's sequence: teams of 16 waves for the heavy windows among
-        // its first kHeavyMaxWindows entries (the reference's descending order
-        // puts the hubs there), then one wave per entry for all others; each
-        // entry belongs to exactly one of the two launches.
-        AttnParams ph = p;
-        ph.team = kTeamLarge;
-        ph.num_items = (int64_t)std::min<int32_t>(W, kHeavyMaxWindows) * kTeamLarge;
-        ph.heavy_mode = 2;
-        F3S_TRY(launch(ph, H, scale, st));
-        p.heavy_mode = 1;
+        // The order's sequence: teams for the heavy windows among its first
+        // kHeavyMaxWindows entries (the reference's descending order puts the
+        // hubs there), one wave per entry for all others.
+        mixed = true;
+    }
+    if (mixed) {
+        p.xcd_contiguous = 0;
+        p.team_blocks = kHeavyMaxWindows * H;
+        if (W > kHugeTiles) {   // else no window has that many
+            AttnParams ph = p;
+            ph.window_order = p.team_list ? p.team_list : p.window_order;
+            ph.team_list = nullptr;
+            ph.team_blocks = 0;
+            ph.team = kTeamLarge;
+            ph.num_items = (int64_t)kHugeMaxWindows * kTeamLarge;
+            ph.huge_only = 1;
+            F3S_TRY(launch(ph, H, scale, st));
+        }
     }
     return launch(p, H, scale, st);
 }

@@ -82,9 +82,10 @@ struct AttnParams {
     const int32_t* chunk_base;       // compiled plan: item i owns chunks [cb[i], cb[i+1])
     const uint32_t* columns;         // compiled plan: per chunk 32 row offsets, 32 row masks
     int32_t team;                    // waves per window (1, or kTeamSmall / kTeamLarge)
-    int32_t heavy_mode;              // order-sequence launches: 0 every entry; 1 all but the
-                                     // heavy windows among the first kHeavyMaxWindows
-                                     // entries; 2 only those (teams)
+    int32_t huge_only;               // (teams of kTeamLarge) only the huge windows of the order
+    int32_t team_blocks;             // mixed launch: its first workgroups, teams of kTeamSmall
+    const int32_t* team_list;        // (mixed) their windows; NULL: the heavy ones among the
+                                     // order's first kHeavyMaxWindows entries
     const int32_t* slot_split;       // planned launch: the split window of each partial slot
     int32_t* counters;               // planned launch: segments arrived per (split window,
                                      // head); zero between passes
@@ -96,10 +97,16 @@ struct AttnParams {
 // both kHeavyMinTiles and kHeavyMeanFactor x the mean window; on the
 // library's schedule the first kHeavyMaxWindows of them (heaviest first),
 // in an order's sequence those among its first kHeavyMaxWindows entries, run
-// as 16-wave teams.
+// as teams: of 4 waves, in the first workgroups of the one-wave windows'
+// launch, or, the huge ones among the first kHugeMaxWindows entries (more than
+// kHugeTiles tiles too), of 16 waves in a launch before it.
 constexpr int32_t kHeavyMinTiles = 1024;
 constexpr int32_t kHeavyMeanFactor = 8;
 constexpr int32_t kHeavyMaxWindows = 512;
+// A quarter of kHugeTiles takes a wave about as long as the plan's longest
+// segments (5,161 tiles on the largest random graphs: no tail).
+constexpr int32_t kHugeTiles = 16384;
+constexpr int32_t kHugeMaxWindows = 64;
 __host__ __device__ __forceinline__ int32_t heavy_tiles(int32_t T, int32_t W, int32_t min_tiles,
                                                         int32_t factor)
 {
