@@ -162,9 +162,13 @@ __device__ __forceinline__ void merge_split(const AttnParams& p, const SplitInfo
 // p.team_blocks workgroups are teams of WPG waves for those, the others run a
 // window per wave.  (Teams of 16 waves in a launch of their own had the chip to
 // themselves for 98 us on 1 M nodes, 512 heavy windows: 618 -> 581 us per
-// call; with none listed the launch alone cost 3 us, 50,001 nodes 96 -> 93.)
+// call.  heavy_apart says when they have that launch all the same.)
+// The masked unplanned kernels are held to 4 waves per SIMD: given the choice
+// the compiler takes 5 for some of them, with fewer loads in flight (100 k
+// to 800 k nodes: 2 to 5 % slower).
 template <int MODE, int WPG, bool WIDE, int TEAM, bool PACKED, bool MIXED = false>
-__global__ void __launch_bounds__(kWave * WPG) __attribute__((amdgpu_waves_per_eu(4)))
+__global__ void __launch_bounds__(kWave * WPG)
+__attribute__((amdgpu_waves_per_eu(4, MODE == kModeRing ? 4 : 8)))
 fused_attention_kernel(const AttnParams p)
 {
     static_assert(TEAM == 1 || TEAM == WPG, "a team fills its workgroup");
@@ -230,21 +234,21 @@ fused_attention_kernel(const AttnParams p)
         const int32_t T = p.window_offsets[p.W];
         tb = max(0, min(p.window_offsets[w], T));
         te = max(tb, min(p.window_offsets[w + 1], T));
-        if (MIXED || (TEAM > 1 && p.huge_only)) {
-            // A window of an order's sequence or of the team list belongs to
-            // one of the huge windows' launch, a team here and a wave here
-            // (uniform over a team; the schedule's one-wave slots hold none
-            // of the team list's).
+        if (MIXED || (TEAM > 1 && p.apart_windows > 0)) {
+            // A heavy window of an order's sequence or of the team list is a
+            // team's, here or in the launch apart (uniform over a team); the
+            // schedule's one-wave slots hold none of the team list's.
             const int32_t heavy = heavy_tiles(T, p.W, kHeavyMinTiles, kHeavyMeanFactor);
             const bool is_heavy = wi < kHeavyMaxWindows && te - tb > heavy;
-            const bool huge = is_heavy && wi < kHugeMaxWindows && te - tb > kHugeTiles &&
-                              p.W > kHugeTiles;   // (as the launch's condition)
-            if constexpr (!MIXED) {
-                if (!huge) return;
-            } else if (in_team) {
-                if (huge || !is_heavy) return;
-            } else if (!p.team_list && is_heavy) {
-                return;
+            if (MIXED && !in_team) {
+                if (!p.team_list && is_heavy) return;
+            } else {
+                if (!is_heavy) return;
+                const bool apart =
+                    wi < p.apart_windows &&
+                    heavy_apart<MODE != kModeDense>(p, listed ? p.team_list : p.window_order, T,
+                                                    heavy, lane);
+                if (apart == MIXED) return;
             }
         }
         if (in_team) {
@@ -1550,7 +1554,7 @@ static f3s_status attention_fwd_impl(const uint16_t* Q, const uint16_t* K, const
         }
         int32_t *team = nullptr, *sched = nullptr;
         F3S_TRY(launch_schedule(d_window_offsets, d_window_order, W,
-                                heavy_possible ? kHeavyMaxWindows : 0, sp, st, &team, &sched));
+                                heavy_possible ? team_entries(W, H) : 0, sp, st, &team, &sched));
         p.team_list = heavy_possible ? team : nullptr;
         p.window_order = sched;
         p.xcd_contiguous = 0;
@@ -1564,17 +1568,16 @@ static f3s_status attention_fwd_impl(const uint16_t* Q, const uint16_t* K, const
     }
     if (mixed) {
         p.xcd_contiguous = 0;
-        p.team_blocks = kHeavyMaxWindows * H;
-        if (W > kHugeTiles) {   // else no window has that many
-            AttnParams ph = p;
-            ph.window_order = p.team_list ? p.team_list : p.window_order;
-            ph.team_list = nullptr;
-            ph.team_blocks = 0;
-            ph.team = kTeamLarge;
-            ph.num_items = (int64_t)kHugeMaxWindows * kTeamLarge;
-            ph.huge_only = 1;
-            F3S_TRY(launch(ph, H, scale, st));
-        }
+        p.team_blocks = (p.team_list ? team_entries(W, H) : kHeavyMaxWindows) * H;
+        p.apart_windows = apart_entries(W, H);
+        // (T is on the device only, so whether there is such a window too)
+        AttnParams ph = p;
+        ph.window_order = p.team_list ? p.team_list : p.window_order;
+        ph.team_list = nullptr;
+        ph.team_blocks = 0;
+        ph.team = kTeamLarge;
+        ph.num_items = (int64_t)p.apart_windows * kTeamLarge;
+        F3S_TRY(launch(ph, H, scale, st));
     }
     return launch(p, H, scale, st);
 }

@@ -82,7 +82,7 @@ struct AttnParams {
     const int32_t* chunk_base;       // compiled plan: item i owns chunks [cb[i], cb[i+1])
     const uint32_t* columns;         // compiled plan: per chunk 32 row offsets, 32 row masks
     int32_t team;                    // waves per window (1, or kTeamSmall / kTeamLarge)
-    int32_t huge_only;               // (teams of kTeamLarge) only the huge windows of the order
+    int32_t apart_windows;           // (mixed, and the launch before it) entries that may run apart
     int32_t team_blocks;             // mixed launch: its first workgroups, teams of kTeamSmall
     const int32_t* team_list;        // (mixed) their windows; NULL: the heavy ones among the
                                      // order's first kHeavyMaxWindows entries
@@ -95,18 +95,31 @@ struct AttnParams {
 
 // A window is heavy for the unplanned launch's teams when its tiles exceed
 // both kHeavyMinTiles and kHeavyMeanFactor x the mean window; on the
-// library's schedule the first kHeavyMaxWindows of them (heaviest first),
-// in an order's sequence those among its first kHeavyMaxWindows entries, run
-// as teams: of 4 waves, in the first workgroups of the one-wave windows'
-// launch, or, the huge ones among the first kHugeMaxWindows entries (more than
-// kHugeTiles tiles too), of 16 waves in a launch before it.
+// library's schedule the first of them (heaviest first, team_entries), in an
+// order's sequence those among its first kHeavyMaxWindows entries, run as
+// teams: of 4 waves, in the first workgroups of the one-wave windows' launch,
+// or, the first of them (apart_entries) where the heaviest is too long for
+// four waves (heavy_apart), of 16 waves in a launch before it.
 constexpr int32_t kHeavyMinTiles = 1024;
 constexpr int32_t kHeavyMeanFactor = 8;
 constexpr int32_t kHeavyMaxWindows = 512;
-// A quarter of kHugeTiles takes a wave about as long as the plan's longest
-// segments (5,161 tiles on the largest random graphs: no tail).
-constexpr int32_t kHugeTiles = 16384;
-constexpr int32_t kHugeMaxWindows = 64;
+// Entries of the schedule's team list: fewer than 1 of kHeavyMeanFactor
+// windows can be heavy, and a workgroup per entry and head that finds nothing
+// is not free: the others fill in unevenly behind it (1,311 windows without a
+// heavy one, three heads, tile-dense: 448 us behind 1,536 empty workgroups,
+// 391 behind 192).
+__host__ __forceinline__ int32_t team_entries(int32_t W, int32_t H)
+{
+    const int32_t e = W / kHeavyMeanFactor / H;
+    return e < 64 ? 64 : e < kHeavyMaxWindows ? e : kHeavyMaxWindows;
+}
+// Entries that may run apart: the launch is made without knowing that there
+// are any, and costs 2 to 4 us.
+__host__ __forceinline__ int32_t apart_entries(int32_t W, int32_t H)
+{
+    const int32_t e = (W < 4096 ? W : 4096) / 64 / H;
+    return e < 8 ? 8 : e;
+}
 __host__ __device__ __forceinline__ int32_t heavy_tiles(int32_t T, int32_t W, int32_t min_tiles,
                                                         int32_t factor)
 {
@@ -164,6 +177,51 @@ __device__ __forceinline__ int64_t logical_block(int32_t xcd_contiguous)
     const int64_t G = gridDim.x;
     const int64_t x = b % kXcds, q = G / kXcds, rem = G % kXcds;
     return x * q + min(x, rem) + b / kXcds;
+}
+
+// Whether the first heavy windows of a launch run apart, as teams of 16 waves
+// before the others, instead of as teams of 4 among them: where the heaviest of
+// the list's first 64 entries, `most` tiles, takes four waves longer than the
+// rest of the pass takes, by more than the time that 16 waves take for it
+// alone: (1/4 - 1/16) of its tiles against `rest`, in tiles of one wave's
+// chain.  The rest is the whole pass at the chip's rate, or the longest windows
+// that are not heavy (where there are enough tiles for such).  A masked chain
+// goes by the attended columns, sampled in 64 of the window's tiles: a
+// node joined to all others costs about 6 times the tiles of a hub of two
+// edges a tile.  (Rates from timings of 30 k to 1 M nodes, one to four heads:
+// the chip's rate is 1,900 to 2,400 waves' chains.  Microseconds with every
+// heavy window in a launch of 16-wave teams before the others / with all of
+// them on 4 waves among the others / by this rule, natural order:
+//   power law, 262 k nodes, top 8,190 tiles: masked 146 / 163 / 147,
+//     tile-dense 1,476 / 1,628 / 1,491; four heads: 394 / 382 / 381, 4.81 / 4.83 / 4.83 ms
+//   the same, 100 k nodes, top 3,291: 106 / 84 / 87, 834 / 747 / 757
+//   1 M nodes, top 15,705: 639 / 599 / 601, 8.65 / 8.60 / 8.56 ms
+//   one node joined to all, 30 k nodes: 162 / 291 / 155, 131 k: 592 / 1,215 / 581)
+template <bool MASKED>
+__device__ __forceinline__ bool heavy_apart(const AttnParams& p, const int32_t* __restrict__ list,
+                                            int32_t T, int32_t heavy, int lane)
+{
+    const int32_t w = list[lane];
+    int32_t tb = 0, n = 0;
+    if (w >= 0 && w < p.W) {
+        tb = max(0, min(p.window_offsets[w], T));
+        n = max(tb, min(p.window_offsets[w + 1], T)) - tb;
+    }
+    int32_t most = n;
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) most = max(most, __shfl_xor(most, off, kWave));
+    if (most <= heavy) return false;
+    tb = __shfl(tb, __ffsll((unsigned long long)__ballot(n == most)) - 1, kWave);
+    const int64_t all = (int64_t)T * p.H;
+    const int64_t rest = max(all / (MASKED ? 1900 : 2400), min((int64_t)heavy, all / 350));
+    if (!MASKED) return 3 * (int64_t)most > 16 * rest;
+    const uint4* m =
+        reinterpret_cast<const uint4*>(p.tile_mask + (tb + (int64_t)most * lane / kWave) * 16);
+    const uint4 a = m[0], b = m[1];
+    uint32_t u = a.x | a.y | a.z | a.w | b.x | b.y | b.z | b.w;
+    u = (u | (u >> 16)) & 0xffffu;
+    const int64_t columns = (int64_t)wave_sum(__popc(u)) * most / kWave;
+    return 3 * (most + columns) > 40 * rest;
 }
 
 __device__ __forceinline__ f4 mfma16x16x32(h8 a, h8 b, f4 c)

@@ -159,23 +159,25 @@ f3s_status f3s_bsf_stats(const int32_t* d_block_col, const uint16_t* d_tile_mask
  * graphs (W > 512), given d_window_order on a launch of fewer than 2^18
  * window-heads (W x H), windows run in the order's sequence: the heavy
  * windows (more than max(1024, 8 x mean) tiles) among its first 512 entries
- * as teams of 4 waves in the launch's first workgroups (past 16,384 tiles,
- * among the first 64, teams of 16 in a launch before it), every other entry
- * on one wave.  In natural order, and with an order from 2^18 window-heads on, the
- * order only names the windows -- each named window is computed once;
+ * as teams of 4 waves in the launch's first workgroups, every other entry on
+ * one wave.  In natural order, and with an order from 2^18 window-heads on,
+ * the order only names the windows -- each named window is computed once;
  * invalid entries are skipped -- and the library schedules them itself,
  * identically for every order: the heavy windows, heaviest first, the first
- * 512 of them as such teams; every other window on one wave, by octave of its tile count, heaviest first, each
- * octave in index order and cut into eight contiguous shares interleaved
- * slot by slot across the XCDs (longest windows first for the tail, each
- * share's contiguous windows on one or a few XCDs for the L2; on a
- * community-ordered graph the reference's descending order would scatter
- * each community over the whole run).  With W <= 1024 no window can be heavy
- * (one tile per block column at most) and no teams are launched.  Three
- * small kernels (four given an order; ~15-30 us; one for the three up to 4,096
- * windows) build the schedule in
- * scratch of about 9 bytes per window taken from the
- * library's cache and returned to it in stream order on `stream` (the call
+ * W / 8 / H of them (64 to 512) as such teams; every other window on one
+ * wave, by octave of its tile count, heaviest first, each octave in index
+ * order and cut into eight contiguous shares interleaved slot by slot across
+ * the XCDs (longest windows first for the tail, each share's contiguous
+ * windows on one or a few XCDs for the L2; on a community-ordered graph the
+ * reference's descending order would scatter each community over the whole
+ * run).  Either way, where the heaviest window would outlast the rest of the
+ * pass on four waves (by T x H and, masked, its attended columns), the first
+ * up to 64 heavy entries run as teams of 16 waves in a launch before it.
+ * With W <= 1024 no window can be heavy (one tile per block column at most)
+ * and no teams are launched.  Three small kernels (four given an order;
+ * ~15-30 us; one for the three up to 4,096 windows) build the schedule in
+ * scratch of about 9 bytes per window taken from the library's cache and
+ * returned to it in stream order on `stream` (the call
  * does not wait).  Tensors past ~4 GiB take the sequence of the order, as
  * small graphs do.  Every other path allocates nothing. */
 f3s_status f3s_attention_fwd(const uint16_t* Q, const uint16_t* K, const uint16_t* V,
