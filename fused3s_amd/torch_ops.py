@@ -25,6 +25,8 @@ from __future__ import annotations
 
 import numpy as np
 import torch
+from torch.autograd import forward_ad
+from torch.utils._device import DeviceContext
 
 # torch ships its own HIP runtime (torch/lib/libamdhip64.so, soname
 # libamdhip64.so.7).  libf3s_hip.so binds to whichever libamdhip64.so.7 the
@@ -169,10 +171,29 @@ class TorchGraph:
         return out
 
 
+_LINEAR_FORWARD, _LINEAR = torch.nn.Linear.forward, torch.nn.functional.linear
+
+
+def _watched() -> bool:
+    """Whether something sees, replaces or transforms torch's calls: compilation
+    and tracing, autocast, dispatch modes, function modes (torch.device's own
+    does neither), functorch's transforms, forward-mode differentiation (which
+    no_grad leaves on)."""
+    c = torch._C
+    return (torch.compiler.is_compiling() or torch.jit.is_tracing()
+            or torch.is_autocast_enabled() or c._len_torch_dispatch_stack() > 0
+            or any(type(c._get_function_stack_at(i)) is not DeviceContext
+                   for i in range(c._len_torch_function_stack()))
+            or c._functorch.peek_interpreter_stack() is not None
+            or forward_ad._current_level >= 0)
+
+
 def _is_plain_linear(m: torch.nn.Module) -> bool:
     """A torch.nn.Linear whose call is its product and nothing else."""
     hooks = torch.nn.modules.module
     return (type(m) is torch.nn.Linear and "forward" not in m.__dict__
+            and torch.nn.Linear.forward is _LINEAR_FORWARD
+            and torch.nn.functional.linear is _LINEAR
             and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
                      or m._backward_pre_hooks or hooks._global_forward_hooks
                      or hooks._global_forward_pre_hooks or hooks._global_backward_hooks
@@ -182,14 +203,13 @@ def _is_plain_linear(m: torch.nn.Module) -> bool:
 def _project(m: torch.nn.Module, x: torch.Tensor) -> torch.Tensor:
     """m(x), by f3s_linear_f16 where that is the same thing: a plain fp16
     Linear of a contiguous fp16 matrix on its own device, in sizes the kernel
-    takes, outside autocast, tracing and dispatch modes.  (Called without autograd.)  Below
+    takes, where nothing watches the call.  (Called without autograd.)  Below
     64 K rows of more than 128 inputs and outputs the library's tiles are the
     better ones (20,011 x 256 -> 768: 17 against 28 us; -> 128: 8 against 9,
     and half the call's host time)."""
-    if (type(x) is torch.Tensor and x.dim() == 2 and x.is_cuda and x.dtype is torch.float16
-            and x.is_contiguous() and x.shape[0] > 0 and _is_plain_linear(m)
-            and not torch.is_autocast_enabled() and not torch.compiler.is_compiling()
-            and not torch.jit.is_tracing() and torch._C._len_torch_dispatch_stack() == 0):
+    if (not _watched() and type(x) is torch.Tensor and x.dim() == 2 and x.is_cuda
+            and x.dtype is torch.float16 and x.is_contiguous() and x.shape[0] > 0
+            and _is_plain_linear(m)):
         w, b = m.weight, m.bias
         M, K = w.shape
         if (K % 8 == 0 and K <= 256 and M % 32 == 0 and M <= 32768 and x.shape[1] == K

@@ -93,3 +93,59 @@ def test_layer_yields_to_overrides(gpu):
 
     layer(x, Own(rp, ci, heads=1))
     assert calls
+
+
+class _OwnAttention:
+    """A program's own attention in the place of a TorchGraph: each node's v."""
+
+    heads = 1
+
+    def attention(self, q, k, v, scale=1.0):
+        return v.float()
+
+
+def test_layer_yields_to_watchers(gpu):
+    """The layer's products are torch's own where a function mode, a functorch
+    transform, forward-mode differentiation or a replaced torch.nn.functional.
+    linear is there to see them."""
+    import torch.autograd.forward_ad as forward_ad
+    from torch.overrides import TorchFunctionMode
+
+    from fused3s_amd import torch_ops
+    layer = torch_ops.GraphTransformerLayer(64, heads=1).cuda().half()
+    graph = _OwnAttention()
+    x = torch.randn(100, 64, dtype=torch.float16, device="cuda")
+    own = layer(x, graph)
+    seen = []
+
+    class Count(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return func(*args, **(kwargs or {}))
+
+    with Count():
+        y = layer(x, graph)
+    assert seen.count(torch.nn.functional.linear) == 2
+    bound = 2e-3 * own.abs().max()
+    assert (y - own).abs().max() <= bound
+
+    with torch.device("cuda"):   # a function mode too, but it sees no products
+        assert torch.equal(layer(x, graph), own)
+
+    z = torch.func.vmap(lambda t: layer(t, graph))(torch.stack([x, -x]))
+    assert (z[0] - own).abs().max() <= bound
+
+    with forward_ad.dual_level():
+        dual = layer(forward_ad.make_dual(x, x), graph)
+        tangent = forward_ad.unpack_dual(dual).tangent
+    assert tangent is not None   # the layer is affine here: J x = f(x) - f(0)
+    assert (tangent - (own - layer(torch.zeros_like(x), graph))).abs().max() <= 2 * bound
+
+    product = torch.nn.functional.linear
+    calls = []
+    torch.nn.functional.linear = lambda *a: calls.append(1) or product(*a)
+    try:
+        layer(x, graph)
+    finally:
+        torch.nn.functional.linear = product
+    assert len(calls) == 2

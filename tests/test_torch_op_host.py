@@ -56,3 +56,31 @@ def test_index_narrowing(torch_ops):
         torch_ops._cuda_i32(torch.tensor([0, 2**31], dtype=torch.int64), "col_idx")
     with pytest.raises(ValueError, match="int32 \\(or int64\\)"):
         torch_ops._cuda_i32(torch.tensor([0.0, 1.0]), "row_ptr")
+
+
+def test_watched_calls():
+    """What keeps the layer's products with torch: see _watched."""
+    import torch.autograd.forward_ad as forward_ad
+    from torch.overrides import BaseTorchFunctionMode
+    from torch.utils.flop_counter import FlopCounterMode
+
+    from fused3s_amd.torch_ops import _watched
+    seen = []
+    note = lambda x: seen.append(_watched()) or x
+    x = torch.zeros(2, 3)
+    with torch.no_grad():
+        note(x)
+    with torch.device("cpu"):
+        note(x)
+    assert seen == [False, False]
+    for context in (BaseTorchFunctionMode(), FlopCounterMode(display=False),
+                    forward_ad.dual_level()):
+        with context:
+            note(x)
+    with torch.device("cpu"), BaseTorchFunctionMode(), torch.device("cpu"):
+        note(x)
+    torch.func.vmap(note)(x)
+    torch.func.jvp(note, (x,), (x,))
+    torch.jit.trace(note, x, check_trace=False)
+    assert all(seen[2:]) and len(seen) >= 9
+    assert not _watched()
