@@ -229,10 +229,14 @@ def _project(m: torch.nn.Module, x: torch.Tensor) -> torch.Tensor:
     return m(x)
 
 
+_ATTENTION = TorchGraph.attention
+
+
 def _is_plain_graph(graph) -> bool:
     """Whether attention_packed stands for graph.attention: not where a
-    program brings an attention of its own."""
-    return (isinstance(graph, TorchGraph) and type(graph).attention is TorchGraph.attention
+    program brings an attention of its own, in a subclass, on the graph or in
+    the place of TorchGraph's."""
+    return (isinstance(graph, TorchGraph) and type(graph).attention is _ATTENTION
             and "attention" not in graph.__dict__)
 
 

@@ -95,6 +95,29 @@ def test_layer_yields_to_overrides(gpu):
     assert calls
 
 
+def test_layer_calls_a_replaced_attention(gpu, monkeypatch):
+    """One assigned on a graph, and one assigned on TorchGraph itself."""
+    from fused3s_amd import torch_ops
+    rp, ci = random_csr(100, 4, 3)
+    graph = torch_ops.TorchGraph(rp, ci, heads=1)
+    layer = torch_ops.GraphTransformerLayer(64, heads=1).cuda().half()
+    x = torch.randn(100, 64, dtype=torch.float16, device="cuda")
+    calls = []
+    attention = torch_ops.TorchGraph.attention
+
+    def own(self, *args, **kwargs):
+        calls.append(1)
+        return attention(self, *args, **kwargs)
+
+    graph.attention = own.__get__(graph)
+    layer(x, graph)
+    assert len(calls) == 1
+    del graph.attention
+    monkeypatch.setattr(torch_ops.TorchGraph, "attention", own)
+    layer(x, graph)
+    assert len(calls) == 2
+
+
 class _OwnAttention:
     """A program's own attention in the place of a TorchGraph: each node's v."""
 
