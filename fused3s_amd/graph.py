@@ -154,6 +154,14 @@ def converts_once(n: int, nnz: int) -> bool:
     return 0 < nnz <= 2**19 and 0 < n <= 2**19
 
 
+def lists_oversized(T: int, nnz: int) -> bool:
+    """Whether the T tiles found are copied out of lists of nnz entries (36
+    bytes each): where the lists are over twice as long and that is 1 MB at
+    least (clustered graphs of many edges per tile, whose lists a program may
+    keep by the hundred)."""
+    return 2 * T < nnz and 36 * (nnz - T) >= 2**20
+
+
 def convert_device(csr: DeviceCSR, masks: bool = True, stream: Stream | None = None) -> DeviceBSF:
     """f3s_convert_csr_to_bsf: counts, then tile lists (and masks), or both at
     once on small graphs."""
@@ -168,9 +176,9 @@ def convert_device(csr: DeviceCSR, masks: bool = True, stream: Stream | None = N
         check(lib.f3s_convert_csr_to_bsf_once(
             csr.row_ptr.ptr, csr.col_idx.ptr, csr.n, csr.nnz, offs.ptr, bcol.ptr,
             mask.ptr if mask else None, C.byref(T), s), "f3s_convert_csr_to_bsf_once")
-        bcol.truncate(T.value)
+        bcol = bcol.first(T.value, lists_oversized(T.value, csr.nnz), stream)
         if mask:
-            mask.truncate(T.value * 16)
+            mask = mask.first(T.value * 16, lists_oversized(T.value, csr.nnz), stream)
         return DeviceBSF(csr.n, W, int(T.value), offs, bcol, mask)
     check(lib.f3s_convert_csr_to_bsf(csr.row_ptr.ptr, csr.col_idx.ptr, csr.n, csr.nnz, offs.ptr,
                                      None, None, C.byref(T), s), "f3s_convert_csr_to_bsf(count)")

@@ -52,7 +52,7 @@ import ctypes as C
 from . import _lib
 from .attention import Plan
 from .device import DeviceArray, Stream, check
-from .graph import (DeviceBSF, DeviceCSR, convert_device, converts_once,
+from .graph import (DeviceBSF, DeviceCSR, convert_device, converts_once, lists_oversized,
                     window_order_device)
 
 HEAD_DIM = 64
@@ -297,7 +297,8 @@ def to_block_sparse(row_ptr, col_idx, masks: bool = True):
     [T], tile_mask int16 [T, 16] -- bit c of row r of a tile set iff that
     edge exists -- or None).  Two calls of f3s_convert_csr_to_bsf on torch's
     current stream, the count (one host round trip for T), then the fill; or,
-    on small graphs, one call for both."""
+    on small graphs, one call for both, whose lists are then views of storage
+    for at most twice their entries, or 1 MB more (lists_oversized)."""
     rp = _cuda_i32(row_ptr, "row_ptr")
     ci = _cuda_i32(col_idx, "col_idx")
     n = rp.numel() - 1
@@ -317,7 +318,10 @@ def to_block_sparse(row_ptr, col_idx, masks: bool = True):
             rp.data_ptr(), cptr, n, ci.numel(), offs.data_ptr(), bcol.data_ptr(),
             mask.data_ptr() if masks else None, C.byref(T), s), "f3s_convert_csr_to_bsf_once")
         t = int(T.value)
-        return offs, bcol[:t], (mask[:t] if masks else None)
+        bcol, mask = bcol[:t], (mask[:t] if masks else None)
+        if lists_oversized(t, ci.numel()):
+            bcol, mask = bcol.clone(), (mask.clone() if masks else None)
+        return offs, bcol, mask
     check(lib.f3s_convert_csr_to_bsf(rp.data_ptr(), cptr, n, ci.numel(), offs.data_ptr(), None,
                                      None, C.byref(T), s), "f3s_convert_csr_to_bsf(count)")
     t = int(T.value)

@@ -102,3 +102,29 @@ def test_once_invalid(gpu, hub):
     with pytest.raises(gpu.F3SError) as e:
         gpu.convert_device(gpu.DeviceCSR(rp, ci))
     assert e.value.name == "F3S_EDATA"
+
+
+@pytest.mark.parametrize("n,degree,copied", [(4000, 100, True), (4000, 2, False), (700, 30, False)])
+def test_lists_keep_no_more_than_twice_their_size(gpu, n, degree, copied):
+    """Clustered graphs, 100, 2 and 30 edges a node in groups of 160: a
+    conversion's lists are copies of their own size where the lists of nnz
+    entries they were found in are far longer; contents as the oracle's."""
+    torch = pytest.importorskip("torch")
+    from fused3s_amd import torch_ops
+    r = rng(n + degree)
+    rows = np.repeat(np.arange(n), degree)
+    key = np.unique(rows * n + np.minimum(rows // 160 * 160 + r.integers(0, 160, len(rows)), n - 1))
+    rp = np.searchsorted(key, np.arange(n + 1) * n).astype(np.int32)
+    ci = (key % n).astype(np.int32)
+    offs, bcol, mask = orc.convert(n, rp, ci)
+    T, nnz = len(bcol), len(ci)
+    o, b, m = torch_ops.to_block_sparse(rp, ci)
+    assert np.array_equal(o.cpu().numpy(), offs) and np.array_equal(b.cpu().numpy(), bcol)
+    assert np.array_equal(m.cpu().numpy().view(np.uint16), mask)
+    kept = T if copied else nnz
+    assert b.untyped_storage().nbytes() == 4 * kept and m.untyped_storage().nbytes() == 32 * kept
+    assert kept <= 2 * T or 36 * (kept - T) < 2**20
+    assert torch_ops.to_block_sparse(rp, ci, masks=False)[1].untyped_storage().nbytes() == 4 * kept
+    h = gpu.convert_device(gpu.DeviceCSR(rp, ci)).to_host()
+    assert np.array_equal(h.window_offsets, offs) and np.array_equal(h.block_col_indices, bcol)
+    assert np.array_equal(h.tile_masks, mask)
