@@ -1334,6 +1334,7 @@ static f3s_status build_plan_sets(f3s_plan* p, const int32_t* d_window_offsets,
     int64_t* sums = reinterpret_cast<int64_t*>(mem + 256 + base_bytes);
     bool pinned = false;
     int64_t* h = host_staging(&pinned);
+    StagingGuard staging(st);
     // [0] T, [1..2] segment sizes, [3..] totals
     int64_t* info = pinned ? h : reinterpret_cast<int64_t*>(mem);
     const PlanSeq q{d_window_offsets, seq, W, P, H, seg_tiles, nsets, {team_m, team_d}};
@@ -1344,7 +1345,7 @@ static f3s_status build_plan_sets(f3s_plan* p, const int32_t* d_window_offsets,
     F3S_HIP(hipGetLastError());
     if (!pinned)
         F3S_HIP(hipMemcpyAsync(h, info, sizeof(int64_t) * (3 + arrays), hipMemcpyDeviceToHost, st));
-    F3S_HIP(hipStreamSynchronize(st));
+    F3S_HIP(staging.wait());
     p->T = h[0];
     const int32_t seg_m = (int32_t)h[1], seg_d = (int32_t)h[2];
     p->has_dense = automatic && (team_d != team_m || (team_d == 1 && seg_d != seg_m));
@@ -1740,11 +1741,12 @@ f3s_status f3s_plan_compile(f3s_plan* plan, const int32_t* d_block_col,
     F3S_HIP(hipGetLastError());
     bool pinned = false;
     int64_t* h = host_staging(&pinned);
+    StagingGuard staging(st);
     int64_t* chunks = pinned ? h : reinterpret_cast<int64_t*>(mem);
     F3S_TRY(counts_to_offsets(counts, chunk_base, ni, sums, chunks, st));
     if (!pinned)
         F3S_HIP(hipMemcpyAsync(h, chunks, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-    F3S_HIP(hipStreamSynchronize(st));
+    F3S_HIP(staging.wait());
     const int64_t total = h[0];
     if (total >= INT32_MAX) {
         set_error("f3s_plan_compile: more than 2^31-1 chunks");

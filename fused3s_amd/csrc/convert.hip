@@ -1220,6 +1220,7 @@ static f3s_status convert_impl(const int32_t* row_ptr, const int32_t* col_idx, i
     F3S_TRY(convert_scratch(buf, W, count, s));
     bool pinned = false;
     ConvertStatus* h = reinterpret_cast<ConvertStatus*>(host_staging(&pinned));
+    StagingGuard staging(stream);
     *h = ConvertStatus{};
     ConvertStatus* status = pinned ? h : s.status;
     if (!pinned) F3S_HIP(hipMemsetAsync(status, 0, sizeof(ConvertStatus), stream));
@@ -1234,7 +1235,7 @@ static f3s_status convert_impl(const int32_t* row_ptr, const int32_t* col_idx, i
     F3S_HIP(hipGetLastError());
     if (!pinned)
         F3S_HIP(hipMemcpyAsync(h, status, sizeof(ConvertStatus), hipMemcpyDeviceToHost, stream));
-    F3S_HIP(hipStreamSynchronize(stream));
+    F3S_HIP(staging.wait());
     const int32_t* err = h->err;
     const int64_t total = h->tiles;
     if (count) {

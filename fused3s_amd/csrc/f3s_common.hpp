@@ -62,9 +62,32 @@ void dev_free_idle(void* ptr, int device);
 void dev_free_synced(void* ptr, int device);
 // Host-pinned staging words of the calling thread (16 x int64), for the small
 // device-to-host reads of counts and status that size outputs.
-// Kernels may write them too (then wait for the stream), unless *pinned comes
-// back false: no pinned memory was to be had.
-int64_t* host_staging(bool* pinned = nullptr);
+// Kernels may write them too (see StagingGuard), unless *pinned comes back
+// false: no pinned memory was to be had.
+int64_t* host_staging(bool* pinned);
+
+// Held while kernels that write the staging words may be queued: waits for
+// their stream on the way out, so that a call which fails half way leaves no
+// kernel to write them under the thread's next call.  wait() is the call's own.
+class StagingGuard {
+public:
+    explicit StagingGuard(hipStream_t s) : stream_(s) {}
+    StagingGuard(const StagingGuard&) = delete;
+    StagingGuard& operator=(const StagingGuard&) = delete;
+    hipError_t wait()
+    {
+        waited_ = true;
+        return hipStreamSynchronize(stream_);
+    }
+    ~StagingGuard()
+    {
+        if (!waited_) (void)hipStreamSynchronize(stream_);
+    }
+
+private:
+    hipStream_t stream_;
+    bool waited_ = false;
+};
 
 // Grow-only device buffer owned by a long-lived object (a plan): allocated on
 // the owner's stream, which the owner synchronises before handing the buffer

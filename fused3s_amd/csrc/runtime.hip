@@ -269,12 +269,12 @@ int64_t* host_staging(bool* pinned)
             hipSuccess) {
             (void)hipGetLastError();
             thread_local int64_t fallback[16];
-            if (pinned) *pinned = false;
+            *pinned = false;
             return fallback;   // pageable: correct, only slower to copy into
         }
         words = static_cast<int64_t*>(p);
     }
-    if (pinned) *pinned = true;
+    *pinned = true;
     return words;
 }
 

@@ -128,3 +128,41 @@ def test_lists_keep_no_more_than_twice_their_size(gpu, n, degree, copied):
     h = gpu.convert_device(gpu.DeviceCSR(rp, ci)).to_host()
     assert np.array_equal(h.window_offsets, offs) and np.array_equal(h.block_col_indices, bcol)
     assert np.array_equal(h.tile_masks, mask)
+
+
+def test_failed_call_leaves_the_next_its_status(gpu):
+    """A call that fails after its first launch (here on an error that another
+    library's HIP call left pending on the thread) waits for its kernels: one
+    that finds a bad column then does not write it into the next call's status
+    words, which are the thread's."""
+    torch = pytest.importorskip("torch")
+    from fused3s_amd import _lib
+    with open("/proc/self/maps") as f:
+        path = next(line.split()[-1] for line in f if "libamdhip64" in line)
+    hip = C.CDLL(path)
+    f = _lib.hip().f3s_convert_csr_to_bsf
+    n = 4_000_000
+    rp = torch.arange(n + 1, dtype=torch.int32, device="cuda") * 16
+    ci = torch.randint(n, (16 * n,), dtype=torch.int32, device="cuda")
+    offs = torch.empty(n // 16 + 1, dtype=torch.int32, device="cuda")
+    small_rp, small_ci = (torch.from_numpy(a).cuda() for a in random_csr(2000, 5, 6))
+    small_offs = torch.empty(126, dtype=torch.int32, device="cuda")
+    T = C.c_int64(-1)
+
+    def big():
+        return f(rp.data_ptr(), ci.data_ptr(), n, 16 * n, offs.data_ptr(), None, None, C.byref(T),
+                 None)
+
+    def small():
+        return f(small_rp.data_ptr(), small_ci.data_ptr(), 2000, small_ci.numel(),
+                 small_offs.data_ptr(), None, None, C.byref(T), None)
+
+    assert big() == 0 and small() == 0   # (the scratch of both is cached now)
+    ci[-1] = n                           # outside [0, n)
+    torch.cuda.synchronize()
+    assert hip.hipSetDevice(10_000) != 0
+    failed = big()
+    status = small()
+    assert failed == 4 and status == 0   # F3S_ENODEV (the pending error), F3S_OK
+    assert small_offs[125].item() == T.value
+    torch.cuda.synchronize()
