@@ -1207,8 +1207,9 @@ static f3s_status launch_pass(const int32_t* row_ptr, const int32_t* col_idx, in
 // Count call: tile counts and their scan into the caller's offsets.  Fill
 // call: the lists.  One host round trip each, for T and the error flags, which
 // the kernels write to pinned host memory themselves.  `once`: both at once,
-// into lists of nnz entries, with one round trip -- the offsets of a CSR that
-// turns out to be invalid may pass the lists' end, so the fill is given it.
+// into lists of min(nnz, W * W) entries, with one round trip -- the offsets of
+// a CSR that turns out to be invalid may pass the lists' end, so the fill is
+// given it.
 static f3s_status convert_impl(const int32_t* row_ptr, const int32_t* col_idx, int32_t n,
                                int64_t nnz, int32_t* window_offsets, int32_t* block_col,
                                uint16_t* tile_mask, bool once, int64_t* T_out, hipStream_t stream)
@@ -1231,7 +1232,9 @@ static f3s_status convert_impl(const int32_t* row_ptr, const int32_t* col_idx, i
     }
     if (block_col)
         F3S_TRY(launch_pass<true>(row_ptr, col_idx, n, nnz, W, window_offsets, block_col,
-                                  tile_mask, once ? (int32_t)nnz : INT32_MAX, s, status, stream));
+                                  tile_mask,
+                                  once ? (int32_t)std::min<int64_t>(nnz, (int64_t)W * W) : INT32_MAX,
+                                  s, status, stream));
     F3S_HIP(hipGetLastError());
     if (!pinned)
         F3S_HIP(hipMemcpyAsync(h, status, sizeof(ConvertStatus), hipMemcpyDeviceToHost, stream));

@@ -145,7 +145,7 @@ class DeviceBSF:
 
 
 def converts_once(n: int, nnz: int) -> bool:
-    """Whether a graph is converted by one call into lists of nnz entries
+    """Whether a graph is converted by one call into lists of most_tiles entries
     instead of a count call and a fill call: small graphs, whose conversion is
     mostly launches and host round trips, and whose lists hold 19 MB at most.
     (2,708 nodes: 47 -> 33 us; 20,011 nodes prepared and through a layer once:
@@ -154,12 +154,18 @@ def converts_once(n: int, nnz: int) -> bool:
     return 0 < nnz <= 2**19 and 0 < n <= 2**19
 
 
-def lists_oversized(T: int, nnz: int) -> bool:
-    """Whether the T tiles found are copied out of lists of nnz entries (36
+def most_tiles(n: int, nnz: int) -> int:
+    """The most tiles that nnz edges among n nodes can have: one for each edge,
+    or every pair of windows."""
+    return min(nnz, ((n + 15) // 16) ** 2)
+
+
+def lists_oversized(T: int, most: int) -> bool:
+    """Whether the T tiles found are copied out of lists of `most` entries (36
     bytes each): where the lists are over twice as long and that is 1 MB at
     least (clustered graphs of many edges per tile, whose lists a program may
-    keep by the hundred)."""
-    return 2 * T < nnz and 36 * (nnz - T) >= 2**20
+    keep by the hundred).  It takes 10 to 15 us."""
+    return 2 * T < most and 36 * (most - T) >= 2**20
 
 
 def convert_device(csr: DeviceCSR, masks: bool = True, stream: Stream | None = None) -> DeviceBSF:
@@ -171,14 +177,16 @@ def convert_device(csr: DeviceCSR, masks: bool = True, stream: Stream | None = N
     T = C.c_int64(0)
     s = stream.handle if stream else None
     if converts_once(csr.n, csr.nnz):
-        bcol = DeviceArray(csr.nnz, np.int32)
-        mask = DeviceArray(csr.nnz * 16, np.uint16) if masks else None
+        most = most_tiles(csr.n, csr.nnz)
+        bcol = DeviceArray(most, np.int32)
+        mask = DeviceArray(most * 16, np.uint16) if masks else None
         check(lib.f3s_convert_csr_to_bsf_once(
             csr.row_ptr.ptr, csr.col_idx.ptr, csr.n, csr.nnz, offs.ptr, bcol.ptr,
             mask.ptr if mask else None, C.byref(T), s), "f3s_convert_csr_to_bsf_once")
-        bcol = bcol.first(T.value, lists_oversized(T.value, csr.nnz), stream)
+        copy = lists_oversized(T.value, most)
+        bcol = bcol.first(T.value, copy, stream)
         if mask:
-            mask = mask.first(T.value * 16, lists_oversized(T.value, csr.nnz), stream)
+            mask = mask.first(T.value * 16, copy, stream)
         return DeviceBSF(csr.n, W, int(T.value), offs, bcol, mask)
     check(lib.f3s_convert_csr_to_bsf(csr.row_ptr.ptr, csr.col_idx.ptr, csr.n, csr.nnz, offs.ptr,
                                      None, None, C.byref(T), s), "f3s_convert_csr_to_bsf(count)")

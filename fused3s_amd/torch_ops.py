@@ -53,7 +53,7 @@ from . import _lib
 from .attention import Plan
 from .device import DeviceArray, Stream, check
 from .graph import (DeviceBSF, DeviceCSR, convert_device, converts_once, lists_oversized,
-                    window_order_device)
+                    most_tiles, window_order_device)
 
 HEAD_DIM = 64
 
@@ -311,15 +311,15 @@ def to_block_sparse(row_ptr, col_idx, masks: bool = True):
     T = C.c_int64(0)
     cptr = ci.data_ptr() if ci.numel() else None
     if converts_once(n, ci.numel()):
-        bcol = torch.empty(ci.numel(), dtype=torch.int32, device=rp.device)
-        mask = (torch.empty((ci.numel(), 16), dtype=torch.int16, device=rp.device) if masks
-                else None)
+        most = most_tiles(n, ci.numel())
+        bcol = torch.empty(most, dtype=torch.int32, device=rp.device)
+        mask = torch.empty((most, 16), dtype=torch.int16, device=rp.device) if masks else None
         check(lib.f3s_convert_csr_to_bsf_once(
             rp.data_ptr(), cptr, n, ci.numel(), offs.data_ptr(), bcol.data_ptr(),
             mask.data_ptr() if masks else None, C.byref(T), s), "f3s_convert_csr_to_bsf_once")
         t = int(T.value)
         bcol, mask = bcol[:t], (mask[:t] if masks else None)
-        if lists_oversized(t, ci.numel()):
+        if lists_oversized(t, most):
             bcol, mask = bcol.clone(), (mask.clone() if masks else None)
         return offs, bcol, mask
     check(lib.f3s_convert_csr_to_bsf(rp.data_ptr(), cptr, n, ci.numel(), offs.data_ptr(), None,

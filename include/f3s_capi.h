@@ -122,9 +122,9 @@ f3s_status f3s_convert_csr_to_bsf(const int32_t* d_row_ptr, const int32_t* d_col
                                   uint16_t* d_tile_mask, int64_t* T_out, void* stream);
 
 /* Count and fill in one call and one host round trip (no reference
- * counterpart): block_col and tile_mask (NULL: no masks) hold nnz entries,
- * which T never exceeds; the first T are written.  n up to 4,194,304.  Errors
- * as of the two calls. */
+ * counterpart): block_col and tile_mask (NULL: no masks) hold min(nnz, W * W)
+ * entries, W = ceil(n / 16), which T never exceeds; the first T are written.
+ * n up to 4,194,304.  Errors as of the two calls. */
 f3s_status f3s_convert_csr_to_bsf_once(const int32_t* d_row_ptr, const int32_t* d_col_idx,
                                        int32_t n, int64_t nnz, int32_t* d_window_offsets,
                                        int32_t* d_block_col, uint16_t* d_tile_mask,

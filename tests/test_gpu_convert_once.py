@@ -14,17 +14,21 @@ from conftest import random_csr, rng
 
 pytestmark = pytest.mark.gpu
 
-GUARD = 64   # tiles past the lists' nnz, filled with 0x5a
+GUARD = 64   # tiles past the lists' end, filled with 0x5a
+
+
+def most(n: int, nnz: int) -> int:
+    return min(nnz, ((n + 15) // 16) ** 2)
 
 
 def once(gpu, rp, ci, masks=True):
-    """(status, T, offsets, block_col, tile_mask): both lists nnz + GUARD long."""
+    """(status, T, offsets, block_col, tile_mask): both lists `most` + GUARD long."""
     from fused3s_amd import _lib
     n, nnz = len(rp) - 1, len(ci)
     csr = gpu.DeviceCSR(rp, ci)
     offs = gpu.DeviceArray((n + 15) // 16 + 1, np.int32)
-    bcol = gpu.DeviceArray(nnz + GUARD, np.int32)
-    mask = gpu.DeviceArray((nnz + GUARD) * 16, np.uint16)
+    bcol = gpu.DeviceArray(most(n, nnz) + GUARD, np.int32)
+    mask = gpu.DeviceArray((most(n, nnz) + GUARD) * 16, np.uint16)
     bcol.fill_bytes(0x5a)
     mask.fill_bytes(0x5a)
     T = C.c_int64(-1)
@@ -62,9 +66,13 @@ def hubs(n: int, seed: int):
 
 @pytest.mark.parametrize("graph,n", [("random", 1), ("random", 16), ("random", 17),
                                      ("random", 2708), ("random", 40_001),
+                                     ("full", 16), ("full", 200), ("full", 700),
                                      ("hubs", 20_000), ("hubs", 33_003)])
 def test_once_is_two_calls(gpu, graph, n):
-    rp, ci = random_csr(n, min(n, 7), n) if graph == "random" else hubs(n, n)
+    rp, ci = (random_csr(n, min(n, 7), n) if graph == "random" else hubs(n, n) if graph == "hubs"
+              else (np.arange(n + 1, dtype=np.int32) * n, np.tile(np.arange(n, dtype=np.int32), n)))
+    if graph == "full":   # every tile there is
+        assert len(orc.convert(n, rp, ci)[1]) == most(n, n * n) < n * n
     offs, bcol, mask = orc.convert(n, rp, ci)
     T = len(bcol)
     for want in ((offs, bcol, mask), two_calls(gpu, rp, ci)):
@@ -93,22 +101,23 @@ def test_once_invalid(gpu, hub):
     rp[n] = 0
     status, _, _, b, m = once(gpu, rp, ci)
     assert status != 0
-    assert (b[E:] == 0x5a5a5a5a).all() and (m[E:] == 0x5a5a).all()
+    assert (b[E:] == 0x5a5a5a5a).all() and (m[E:] == 0x5a5a).all()   # (E < W * W)
     rp, ci = random_csr(300, 5, 2)
     ci = ci.copy()
     ci[7] = 300
     status, _, _, b, m = once(gpu, rp, ci)
-    assert status != 0 and (b[len(ci):] == 0x5a5a5a5a).all() and (m[len(ci):] == 0x5a5a).all()
+    end = most(300, len(ci))
+    assert status != 0 and (b[end:] == 0x5a5a5a5a).all() and (m[end:] == 0x5a5a).all()
     with pytest.raises(gpu.F3SError) as e:
         gpu.convert_device(gpu.DeviceCSR(rp, ci))
     assert e.value.name == "F3S_EDATA"
 
 
-@pytest.mark.parametrize("n,degree,copied", [(4000, 100, True), (4000, 2, False), (700, 30, False)])
+@pytest.mark.parametrize("n,degree,copied", [(4000, 100, True), (4000, 2, False), (700, 90, False)])
 def test_lists_keep_no_more_than_twice_their_size(gpu, n, degree, copied):
-    """Clustered graphs, 100, 2 and 30 edges a node in groups of 160: a
-    conversion's lists are copies of their own size where the lists of nnz
-    entries they were found in are far longer; contents as the oracle's."""
+    """Clustered graphs, 100, 2 and 90 edges a node in groups of 160: a
+    conversion's lists are copies of their own size where the lists they were
+    found in are far longer; contents as the oracle's."""
     torch = pytest.importorskip("torch")
     from fused3s_amd import torch_ops
     r = rng(n + degree)
@@ -121,7 +130,7 @@ def test_lists_keep_no_more_than_twice_their_size(gpu, n, degree, copied):
     o, b, m = torch_ops.to_block_sparse(rp, ci)
     assert np.array_equal(o.cpu().numpy(), offs) and np.array_equal(b.cpu().numpy(), bcol)
     assert np.array_equal(m.cpu().numpy().view(np.uint16), mask)
-    kept = T if copied else nnz
+    kept = T if copied else most(n, nnz)
     assert b.untyped_storage().nbytes() == 4 * kept and m.untyped_storage().nbytes() == 32 * kept
     assert kept <= 2 * T or 36 * (kept - T) < 2**20
     assert torch_ops.to_block_sparse(rp, ci, masks=False)[1].untyped_storage().nbytes() == 4 * kept
