@@ -3,7 +3,7 @@
 // outputs per row.
 //
 // Such a product is bound by the rows it reads and writes, not by the matrix
-// cores (128 inputs, 384 outputs: 98 flops per byte), so W is laid out once
+// cores (128 inputs, 384 outputs: 96 flops per byte), so W is laid out once
 // per workgroup in LDS, in the order the MFMA operands are read, and each wave
 // streams blocks of 16 rows past it: a row block's operands are loaded straight
 // into registers, one block ahead of the products.  W is the A operand, its
@@ -116,11 +116,12 @@ linear_kernel(const LinearParams p)
     }
 }
 
-// Many rows: 16 waves share up to 96 KB of W and read X once per 96 KB of it.
+// Many rows: 16 waves share up to 96 KB of W and read X once per 96 KB of it
+// (64,000 x 128 -> 1,536: 43 us, 66 by fours, 63 in the library).
 // Fewer: 4 waves and 32 KB, more workgroups (50,000 x 128 -> 384: 19 us, 26 in
 // the library; 2,708 x 128 -> 192: 5.2 and 4.6, with half the host time).
 constexpr int kBigPieces = 6144, kSmallPieces = 2048;
-constexpr int64_t kBigRows = 64 * 1024;
+constexpr int64_t kBigRows = 48 * 1024;
 
 template <int KF>
 static f3s_status launch_linear(LinearParams p, int cus, hipStream_t st)

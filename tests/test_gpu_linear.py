@@ -16,7 +16,8 @@ pytestmark = pytest.mark.gpu
     (1, 8, 32, True), (15, 64, 96, False), (16, 72, 192, True), (17, 128, 416, True),
     (65, 136, 64, True), (1000, 256, 1536, False), (333, 120, 2048, True),
     (65535, 128, 192, True), (65536, 128, 384, True), (65553, 64, 800, False),
-    (70001, 256, 416, True),
+    (70001, 256, 416, True), (49151, 96, 224, True), (49152, 96, 224, False),   # 4 and 16 waves
+    (33, 64, 2080, True), (5, 8, 12_320, False), (17, 256, 32_768, True), (49_160, 40, 4128, True),
 ])
 def test_linear(gpu, n, K, M, bias):
     from fused3s_amd import _lib
