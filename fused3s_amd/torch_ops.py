@@ -74,9 +74,11 @@ def current_stream() -> Stream:
 
 def _on_device(t, s: Stream) -> DeviceArray:
     """An int32 copy of an index array in library memory: from host memory, or
-    device to device when it is a tensor on the current device already."""
+    device to device when it is a tensor of an index type on the current device
+    already."""
     if torch.is_tensor(t):
-        if t.is_cuda and t.device.index == torch.cuda.current_device():
+        if (t.is_cuda and t.device.index == torch.cuda.current_device()
+                and t.dtype in (torch.int32, torch.int64)):
             t = t.to(torch.int32).contiguous()
             a = DeviceArray(tuple(t.shape), np.int32)
             if a.nbytes:

@@ -79,3 +79,15 @@ def test_graph_from_device_tensors(gpu, dtype):
     assert (got.n, got.nnz) == (want.n, want.nnz)
     q, k, v = torch.randn(3, 1500, 2, 64).half().cuda().unbind(0)
     assert torch.equal(got.attention(q, k, v), want.attention(q, k, v))
+
+
+def test_graph_refuses_device_tensors_as_host_ones(gpu):
+    """Types that numpy does not take are no index types on the device either;
+    the other ones are converted as on the host."""
+    from fused3s_amd import torch_ops
+    rp, ci = (torch.from_numpy(a) for a in random_csr(60, 4, 9))
+    for device in ("cpu", "cuda"):
+        with pytest.raises(TypeError):
+            torch_ops.TorchGraph(rp.to(device), ci.bfloat16().to(device))
+        g = torch_ops.TorchGraph(rp.short().to(device), ci.double().to(device))
+        assert np.array_equal(g.csr.col_idx.numpy(), ci) and g.n == 60
