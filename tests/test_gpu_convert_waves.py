@@ -136,3 +136,27 @@ def test_masks_of_one_node_joined_to_all(gpu):
         return best
 
     assert us(True) < 1.7 * us(False)
+
+
+def test_more_hubs_than_workgroups(gpu):
+    """2,600 hub windows, 2,300 of them heavy: each of the launch's 2,048 hub
+    workgroups takes a second window after a staged, few-tile or many-tile one."""
+    W, n = 2600, 16 * 2600
+    r = rng(12)
+    windows = {}
+    for w in range(W):
+        kind = w % 4 if w % 26 < 23 else 4
+        if kind == 0:     # heavy, a tile for nearly every edge
+            c = r.integers(0, n, 4200)
+        elif kind == 1:   # heavy, 20 tiles
+            c = (r.integers(0, n - 320) + r.integers(0, 320, 4800)).astype(np.int64)
+        elif kind == 2:   # heavy, a row of consecutive columns of more tiles than are staged
+            c = np.arange(n) if w % 400 == 2 else np.arange(5000) + int(r.integers(0, n - 5000))
+        elif kind == 3:   # heavy by one edge
+            c = r.integers(0, n, 4097)
+        else:             # staged
+            c = r.integers(0, n, int(r.integers(1025, 4097)))
+        windows[w] = c
+    rp, ci = window_graph(windows, n, True, 13)
+    check(gpu, rp, ci)
+    check(gpu, rp, ci, masks=False)

@@ -91,3 +91,35 @@ def test_graph_refuses_device_tensors_as_host_ones(gpu):
             torch_ops.TorchGraph(rp.to(device), ci.bfloat16().to(device))
         g = torch_ops.TorchGraph(rp.short().to(device), ci.double().to(device))
         assert np.array_equal(g.csr.col_idx.numpy(), ci) and g.n == 60
+
+
+@pytest.mark.parametrize("n,H", [(11_184_682, 1), (174_760, 64)])
+def test_packed_at_its_limit(gpu, n, H):
+    """The largest packed tensors taken, within 384 bytes a head of 4 GiB less
+    48 KiB, give the planned pass's bits in every row; one node more is refused."""
+    from fused3s_amd import torch_ops
+    assert 3 * n * H * 128 <= 0xffff4000 < 3 * (n + 1) * H * 128
+
+    def graph(nodes):
+        i = torch.arange(nodes, device="cuda")
+        pair = torch.stack([i, torch.where(i % 3 == 0, nodes - 1 - i // 64, (i * 7919 + 13) % nodes)])
+        return torch_ops.TorchGraph((torch.arange(nodes + 1, device="cuda") * 2).int(),
+                                    pair.sort(0).values.t().flatten().int(), heads=H)
+
+    g = graph(n)
+    assert g.takes_packed()
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    qkv = torch.empty(n, 3 * H * 64, dtype=torch.float16, device="cuda")
+    qkv.normal_(generator=gen)
+    got = g.attention_packed(qkv, 0.125)
+    half = g.attention_packed(qkv, 0.125, torch.float16)
+    q, k, v = (t.contiguous() for t in qkv.view(n, 3, H, 64).unbind(1))
+    del qkv
+    want = g.attention(q, k, v, scale=0.125)
+    assert torch.equal(got, want) and torch.equal(half, want.half())
+    del q, k, v, want, got, half, g
+    more = graph(n + 1)
+    assert not more.takes_packed()
+    with pytest.raises(gpu.F3SError) as e:
+        more.attention_packed(torch.empty(n + 1, 3 * H * 64, dtype=torch.float16, device="cuda"))
+    assert e.value.name == "F3S_EUNSUPPORTED"
