@@ -102,17 +102,10 @@ class DeviceArray:
             check(_lib.hip().f3s_memset(self._ptr, int(value), self.nbytes,
                                         stream.handle if stream else None), "f3s_memset")
 
-    def first(self, count: int, copy: bool, stream: "Stream | None" = None) -> "DeviceArray":
-        """A 1-d array's first `count` elements: a copy in an allocation of
-        their size, or this array cut short (the allocation stays)."""
-        if copy:
-            a = DeviceArray(count, self.dtype)
-            check(_lib.hip().f3s_memcpy_d2d(a.ptr, self._ptr, a.nbytes,
-                                            stream.handle if stream else None), "f3s_memcpy_d2d")
-            return a
+    def truncate(self, count: int) -> None:
+        """A 1-d array's first `count` elements from now on (the allocation stays)."""
         self.shape = (min(int(count), self.shape[0]),)
         self.nbytes = self.shape[0] * self.dtype.itemsize
-        return self
 
     def free(self) -> None:
         if getattr(self, "_ptr", None):

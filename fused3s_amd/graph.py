@@ -161,16 +161,18 @@ def most_tiles(n: int, nnz: int) -> int:
 
 
 def lists_oversized(T: int, most: int) -> bool:
-    """Whether the T tiles found are copied out of lists of `most` entries (36
-    bytes each): where the lists are over twice as long and that is 1 MB at
-    least (clustered graphs of many edges per tile, whose lists a program may
-    keep by the hundred).  It takes 10 to 15 us."""
-    return 2 * T < most and 36 * (most - T) >= 2**20
+    """Whether a program's tensors of the T tiles found are copied out of lists
+    of `most` entries (36 bytes each): where the lists are over four times as
+    long and that is 4 MB at least (clustered graphs of many edges per tile).
+    The copy takes 15 us, a quarter of the conversion of 10,000 nodes, so lists
+    twice as long as they have to be are kept."""
+    return 4 * T < most and 36 * (most - T) >= 2**22
 
 
 def convert_device(csr: DeviceCSR, masks: bool = True, stream: Stream | None = None) -> DeviceBSF:
     """f3s_convert_csr_to_bsf: counts, then tile lists (and masks), or both at
-    once on small graphs."""
+    once on small graphs, whose lists keep the memory of most_tiles entries (19 MB
+    at most; cutting them to size took 45 us of a 307 us mini-batch step)."""
     lib = _lib.hip()
     W = (csr.n + 15) // 16
     offs = DeviceArray(W + 1, np.int32)
@@ -183,10 +185,9 @@ def convert_device(csr: DeviceCSR, masks: bool = True, stream: Stream | None = N
         check(lib.f3s_convert_csr_to_bsf_once(
             csr.row_ptr.ptr, csr.col_idx.ptr, csr.n, csr.nnz, offs.ptr, bcol.ptr,
             mask.ptr if mask else None, C.byref(T), s), "f3s_convert_csr_to_bsf_once")
-        copy = lists_oversized(T.value, most)
-        bcol = bcol.first(T.value, copy, stream)
+        bcol.truncate(T.value)
         if mask:
-            mask = mask.first(T.value * 16, copy, stream)
+            mask.truncate(T.value * 16)
         return DeviceBSF(csr.n, W, int(T.value), offs, bcol, mask)
     check(lib.f3s_convert_csr_to_bsf(csr.row_ptr.ptr, csr.col_idx.ptr, csr.n, csr.nnz, offs.ptr,
                                      None, None, C.byref(T), s), "f3s_convert_csr_to_bsf(count)")

@@ -100,7 +100,8 @@ def _device_csr(row_ptr, col_idx, s: Stream) -> DeviceCSR:
 class TorchGraph:
     """A graph prepared once for repeated fused passes: CSR on the device,
     block-sparse form with row masks (GPU converter), descending-workload
-    window order, and a compiled plan for `heads` heads of 64 dims."""
+    window order, and a compiled plan for `heads` heads of 64 dims.  A small
+    graph's block-sparse lists keep the memory of a tile per edge (19 MB at most)."""
 
     def __init__(self, row_ptr, col_idx, heads: int = 1, masked: bool = True):
         if not torch.cuda.is_available():
@@ -181,13 +182,15 @@ def _watched() -> bool:
     and tracing, autocast, dispatch modes, function modes (torch.device's own
     does neither), functorch's transforms, forward-mode differentiation (which
     no_grad leaves on)."""
+    if torch.compiler.is_compiling():
+        return True
     c = torch._C
-    return (torch.compiler.is_compiling() or torch.jit.is_tracing()
-            or torch.is_autocast_enabled() or c._len_torch_dispatch_stack() > 0
-            or any(type(c._get_function_stack_at(i)) is not DeviceContext
-                   for i in range(c._len_torch_function_stack()))
-            or c._functorch.peek_interpreter_stack() is not None
-            or forward_ad._current_level >= 0)
+    modes = c._len_torch_function_stack()
+    return (c._len_torch_dispatch_stack() > 0
+            or modes > 0 and any(type(c._get_function_stack_at(i)) is not DeviceContext
+                                 for i in range(modes))
+            or torch.is_autocast_enabled() or forward_ad._current_level >= 0
+            or c._functorch.peek_interpreter_stack() is not None or torch.jit.is_tracing())
 
 
 def _is_plain_linear(m: torch.nn.Module) -> bool:
@@ -202,14 +205,14 @@ def _is_plain_linear(m: torch.nn.Module) -> bool:
                      or hooks._global_backward_pre_hooks))
 
 
-def _project(m: torch.nn.Module, x: torch.Tensor) -> torch.Tensor:
+def _project(m: torch.nn.Module, x: torch.Tensor, watched: bool) -> torch.Tensor:
     """m(x), by f3s_linear_f16 where that is the same thing: a plain fp16
     Linear of a contiguous fp16 matrix on its own device, in sizes the kernel
-    takes, where nothing watches the call.  (Called without autograd.)  Below
+    takes, where nothing watches the call (_watched).  (Called without autograd.)  Below
     64 K rows of more than 128 inputs and outputs the library's tiles are the
     better ones (20,011 x 256 -> 768: 17 against 28 us; -> 128: 8 against 9,
     and half the call's host time)."""
-    if (not _watched() and type(x) is torch.Tensor and x.dim() == 2 and x.is_cuda
+    if (not watched and type(x) is torch.Tensor and x.dim() == 2 and x.is_cuda
             and x.dtype is torch.float16 and x.is_contiguous() and x.shape[0] > 0
             and _is_plain_linear(m)):
         w, b = m.weight, m.bias
@@ -261,7 +264,8 @@ class GraphTransformerLayer(torch.nn.Module):
         if graph.heads != self.heads:
             raise ValueError("graph was planned for a different head count")
         n = x.shape[0]
-        qkv = _project(self.qkv, x).to(torch.float16)
+        watched = _watched()
+        qkv = _project(self.qkv, x, watched).to(torch.float16)
         dtype = self.proj.weight.dtype
         if _is_plain_graph(graph) and graph.takes_packed() and qkv.dim() == 2 \
                 and qkv.is_contiguous():
@@ -273,7 +277,7 @@ class GraphTransformerLayer(torch.nn.Module):
             qkv = qkv.view(n, 3, self.heads, HEAD_DIM)
             q, k, v = (qkv[:, i].contiguous() for i in range(3))
             o = graph.attention(q, k, v, scale=self.scale)
-        return _project(self.proj, o.view(n, self.heads * HEAD_DIM).to(dtype))
+        return _project(self.proj, o.view(n, self.heads * HEAD_DIM).to(dtype), watched)
 
 
 # ------------------------------------------------------------------ operator
@@ -300,7 +304,7 @@ def to_block_sparse(row_ptr, col_idx, masks: bool = True):
     edge exists -- or None).  Two calls of f3s_convert_csr_to_bsf on torch's
     current stream, the count (one host round trip for T), then the fill; or,
     on small graphs, one call for both, whose lists are then views of storage
-    for at most twice their entries, or 1 MB more (lists_oversized)."""
+    for at most four times their entries, or 4 MB more (lists_oversized)."""
     rp = _cuda_i32(row_ptr, "row_ptr")
     ci = _cuda_i32(col_idx, "col_idx")
     n = rp.numel() - 1
