@@ -234,7 +234,7 @@ fused_attention_kernel(const AttnParams p)
         const int32_t T = p.window_offsets[p.W];
         tb = max(0, min(p.window_offsets[w], T));
         te = max(tb, min(p.window_offsets[w + 1], T));
-        if (MIXED || (TEAM > 1 && p.apart_windows > 0)) {
+        if (MIXED || (TEAM == kTeamLarge && p.apart_windows > 0)) {
             // A heavy window of an order's sequence or of the team list is a
             // team's, here or in the launch apart (uniform over a team); the
             // schedule's one-wave slots hold none of the team list's.

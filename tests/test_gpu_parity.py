@@ -228,16 +228,17 @@ def test_converter_hub_windows(gpu):
 
 
 def test_converter_edge_count_boundaries(gpu):
-    # Windows at each edge-count boundary of the converter: the persistent
-    # kernel takes up to 1,024 edges per window (256 threads x 4), the hub
-    # kernel keeps up to 8,192 in registers (1,024 threads x 8) and ORs the
-    # masks of heavier windows straight into the output; one window of each
-    # of 1,023 / 1,024 / 1,025 / 8,191 / 8,192 / 8,193 edges (row 0 of the
-    # window carries the excess, partly repeated columns), beside light ones.
-    n = 16 * 64
+    # Windows at each edge-count boundary of the converter: a wave takes up to
+    # 1,024 edges, a hub workgroup keeps up to 4,096 in registers (256 threads
+    # x 16, one chunk) and reads a heavier window chunk by chunk; one window
+    # of each of 1,023 / 1,024 / 1,025, 4,095 / 4,096 / 4,097 and 8,191 /
+    # 8,192 / 8,193 edges (two chunks; row 0 of the window carries the excess,
+    # partly repeated columns), beside light ones.
+    n = 16 * 72
+    sizes = [1023, 1024, 1025, 4095, 4096, 4097, 8191, 8192, 8193]
     r = rng(12)
     rows, cols = [np.arange(n)], [np.arange(n)]                 # self-loops
-    for k, E in enumerate((1023, 1024, 1025, 8191, 8192, 8193)):
+    for k, E in enumerate(sizes):
         u = 16 * (8 * k + 3)
         extra = E - 16                                           # the window's 16 self-loops
         rows.append(np.full(extra, u))
@@ -249,14 +250,14 @@ def test_converter_edge_count_boundaries(gpu):
     np.add.at(rp, rr + 1, 1)
     rp = np.cumsum(rp).astype(np.int32)
     edges = np.diff(rp[::16])
-    assert [int(edges[8 * k + 3]) for k in range(6)] == [1023, 1024, 1025, 8191, 8192, 8193]
+    assert [int(edges[8 * k + 3]) for k in range(len(sizes))] == sizes
     check_converter(gpu, rp, cc.astype(np.int32))
 
 
 def test_converter_column_slices(gpu):
-    # 137,500 block columns: one 4,297-word bitmap in the persistent kernel
-    # (more than the per-window kernel's 65,536-column slice), windows with
-    # edges at both ends of the column range
+    # 137,500 block columns: 4,297 bitmap words under a wave's two-level bitmap
+    # (more than convert_wide's 65,536-column slice), windows with edges at
+    # both ends of the column range
     n = 2_200_000
     r = rng(11)
     deg = r.integers(0, 4, n)
@@ -272,9 +273,9 @@ def test_converter_column_slices(gpu):
 @pytest.mark.parametrize("n", [4_194_304, 4_194_320])
 def test_converter_bitmap_limit(gpu, n):
     # 4,194,304 nodes = 262,144 block columns: the widest graph whose block
-    # columns fit the persistent kernel's LDS bitmap (8,192 words); one more
-    # window sends every window through the per-window kernel instead.
-    # Hub rows (> 1,024 edges per window) exercise the hub launch as well.
+    # columns fit the LDS bitmaps of convert_waves (8,192 words); one more
+    # window sends every window through convert_wide instead.  Hub rows
+    # (> 1,024 edges per window) exercise the hub workgroups as well.
     r = rng(12)
     deg = r.integers(0, 3, n)
     deg[:64] += 200                      # four hub windows
@@ -767,10 +768,10 @@ def test_schedule_scratch_outlives_its_launches(gpu):
 
 def test_unplanned_heavy_windows(gpu):
     # Without a plan, windows of more than max(1024, 8 x mean) tiles run as
-    # 16-wave teams in a launch of their own -- in natural order (the
-    # library's schedule) the first 512 such windows, heaviest first; given a
-    # window order on a launch this size (under 2^18 window-heads), those
-    # among its first 512 entries -- and every other window on one wave.
+    # teams, of 4 waves beside the others or of 16 before them -- in natural
+    # order (the library's schedule) the first such windows, heaviest first;
+    # given a window order on a launch this size (under 2^18 window-heads),
+    # those among its first 512 entries -- and every other window on one wave.
     # Hubs sit in windows 0, 1 and 562 (1,250 tiles each); the orders put
     # them first (sorted) or at positions 700, 5 and 100 (one past 512).
     rp, ci = star_graph(20000, hubs=(0, 3, 17, 9000))
@@ -1310,7 +1311,7 @@ def test_schedule_on_a_graph_of_550_count_blocks(gpu):
     one-bitmap limit): the schedule's class counts span 550 blocks, more
     than sched_scan keeps in registers, so it takes its two-pass segment
     loop.  Masked attention on every row for the drop-in launch in natural
-    order (three hub windows of ~20,000 tiles on 16-wave teams) and a
+    order (three hub windows of ~20,000 tiles on teams) and a
     compiled plan (on the same schedule); the drop-in launch in descending
     order (562,500 window-heads: the schedule too) and the allocation-free
     entry point give the natural-order bits, a plan given the order those of

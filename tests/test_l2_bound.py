@@ -4,7 +4,7 @@ computed on the CPU.
 The pass reads each attended K and V row (one 128-byte line each) where the
 plan puts its item, and the eight XCDs' L2s (4 MB each) do not share lines.
 From the planned pass's own items and their XCDs -- the plan restated from
-attention.hip (plan_count / plan_fill: windows in the descending order, heavy
+attention.hip (plan_counts / plan_fill: windows in the descending order, heavy
 windows cut into segments of `seg` tiles) and the launch's mapping (four items
 per workgroup, workgroups dealt to the XCDs round-robin: item i on XCD
 (i / 4) mod 8) -- this builds each XCD's read trace: Q rows at an item's start,
